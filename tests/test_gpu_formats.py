@@ -49,6 +49,61 @@ def test_quantize_affine_bit_exact(pkg, bits, group):
     assert np.array_equal(host_bits(qb), biases_ref)
 
 
+@pytest.mark.parametrize("bits,group", [(8, 64), (8, 32), (4, 64), (4, 32)])
+@pytest.mark.parametrize("N,K_groups", [(1, 1), (3, 5), (33, 67)])
+def test_quantize_affine_edges(pkg, bits, group, N, K_groups):
+    """One group, ragged tails of the flat sequence, quotients on exact half-integers, a zero
+    point far from its group (quotients past the code range), scales down to the denormals
+    (1 / scale overflows): bit-exact against the oracle. With infinities and NaN added, the
+    aligned kernel against the one for weights off 16-byte alignment, whose codes come from
+    the division itself: whole bytes, so equal."""
+    K = group * K_groups
+    say(f"quantize edges w{bits}g{group} {N}x{K}")
+    rng = np.random.default_rng(24)
+    qmax = (1 << bits) - 1
+    w = rng_normal(rng, (N * K_groups, group), 0.02)
+    kinds = rng.integers(0, 6, N * K_groups)
+    for i, kind in enumerate(kinds):
+        if kind == 1:     # lo 0, scale 1: k + 0.5 is a tie
+            w[i] = rng.integers(0, qmax, group) + 0.5
+            w[i, 0], w[i, 1] = 0.0, qmax
+        elif kind == 2:   # the rounded zero point is far off the values
+            w[i] = 1000.3 + rng_normal(rng, (group,), 1e-3)
+        elif kind == 3:
+            w[i] = rng_normal(rng, (group,), 1.0) * np.float32(2.0 ** -int(rng.integers(110, 135)))
+        elif kind == 4:
+            w[i] = rng_normal(rng, (group,), 1e30)
+    w = np.ascontiguousarray(w.reshape(N, K), dtype=np.float32)
+
+    def run(src):
+        flat = torch.zeros(N * K + 1, device="cuda")
+        outs = []
+        for off in (0, 1):   # 16-byte aligned, and one float past it
+            t = flat[off:off + N * K]
+            t.copy_(dev_f32(src).view(-1))
+            codes = torch.empty((N, K * bits // 8), dtype=torch.uint8, device="cuda")
+            sc = torch.empty((N, K // group), dtype=torch.bfloat16, device="cuda")
+            qb = torch.empty((N, K // group), dtype=torch.bfloat16, device="cuda")
+            pkg.quantize_affine(t, codes, sc, qb, N, K, bits, group)
+            torch.cuda.synchronize()
+            outs.append((codes.cpu().numpy(), host_bits(sc), host_bits(qb)))
+        return outs
+
+    codes_ref, scales_ref, biases_ref, _ = orc.quantize_affine(w, bits, group)
+    for codes, sc, qb in run(w):
+        assert np.array_equal(sc, scales_ref)
+        assert np.array_equal(qb, biases_ref)
+        assert np.array_equal(codes, codes_ref.view(np.uint8).reshape(N, -1))
+    special = w.reshape(-1).copy()
+    at = rng.integers(0, special.size, max(2, special.size // 50))
+    special[at] = rng.choice(np.array([np.inf, -np.inf, np.nan, 0.0, -0.0], np.float32), at.size)
+    a, b = run(special.reshape(N, K))
+    assert np.array_equal(a[0], b[0])
+    for i in (1, 2):
+        fa, fb = orc.bf16_to_f32(a[i]), orc.bf16_to_f32(b[i])
+        assert np.array_equal(fa, fb, equal_nan=True)
+
+
 def test_quantize_golden_fixtures(pkg):
     for name in ["quantize_w8g64.npz", "quantize_w4g32.npz"]:
         g = np.load(os.path.join(GOLDEN, name))

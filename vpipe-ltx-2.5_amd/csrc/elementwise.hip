@@ -187,13 +187,118 @@ dequant_kernel(const uint8_t* codes, const uint16_t* scales,
   }
 }
 
-// Group-affine quantize, one thread per (row, group). Step for step the
-// quantizer of tests/ltx25-qlinear-test.cc:108-139: fmin/fmax over the
-// group, scale and min rounded to bf16 first, codes by round-half-away of
-// (w - bias) / scale with IEEE division, clamped; LOW bits first.
+// Group-affine quantize. Step for step the quantizer of
+// tests/ltx25-qlinear-test.cc:108-139: fmin/fmax over the group, scale and
+// min rounded to bf16 first, codes by round-half-away of (w - bias) / scale
+// with IEEE division, clamped; LOW bits first.
+//
+// Bound by memory (4 B in, 1 B and 4 / group B out per element at w8). The
+// groups are one flat sequence (K is whole groups), so a lane takes four
+// consecutive floats and a group is 16 or 8 neighbouring lanes: every load is
+// 1 KB of contiguous memory per wave, kQuantItems of them in flight per lane,
+// the extrema are DPP reductions inside the group's lanes (no LDS) and the
+// codes leave as contiguous words. About 65 us for a 16384 x 4096 weight at
+// w8g64 (340 MB, 5.2 TB/s, the rate of a plain copy); one thread per group,
+// reading its 256-byte run float by float, twice, took 2119 us.
+constexpr int kQuantItems = 4;
+
+// The value of the lane that `CTRL` names, within a row of 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v)
+{
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// clamp(roundf(d / s), 0, qmax) of four values, roundf(d / s) with the
+// quotient correctly rounded; 0 for s <= 0 or NaN and for a NaN quotient.
+// rs = 1 / s rounded. t = d * rs is within 2^-21.9 |t| of d / s (rs down to
+// 2^-128 keeps 21 bits, and one rounding of the product), so for t in
+// [-1, 256] the two are within 2^-13.9 of each other and of the rounded
+// quotient, and round alike unless t lies within 2^-13 of a half-integer;
+// beyond that range both clamp to the same end. Values near a half-integer,
+// and every value when 1 / s overflows, take the division itself, tested once
+// for the four.
+__device__ __forceinline__ void quant4(const float* d, float s, float rs, float qmax, uint32_t* q)
+{
+  const bool pos = s > 0.0f;
+  float r[4];
+  int slow = (int)!(rs < __builtin_inff());
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float t = fminf(fmaxf(d[j] * rs, -1.0f), qmax + 1.0f);   // NaN gives -1, then 0
+    r[j] = rintf(t);
+    slow |= (int)(fabsf(t - r[j]) > 0.5f - 0x1p-13f);
+  }
+  if (slow && pos) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { r[j] = roundf(d[j] / s); }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    q[j] = pos ? (uint32_t)fminf(fmaxf(r[j], 0.0f), qmax) : 0u;
+  }
+}
+
+template <int BITS, int GROUP>
 __global__ void __launch_bounds__(kBlock)
-quantize_affine_kernel(const float* w, uint32_t* codes, uint16_t* scales,
-                       uint16_t* qbias, int N, int K, int bits, int group)
+quantize_affine_kernel(const float* w, uint32_t* codes, uint16_t* scales, uint16_t* qbias,
+                       size_t total)
+{
+  constexpr int kLanes = GROUP / 4;   // lanes per group
+  constexpr float qmax = (float)((1 << BITS) - 1);
+  const size_t base = (size_t)blockIdx.x * (kBlock * 4 * kQuantItems) + threadIdx.x * 4;
+  f32x4 v[kQuantItems];
+#pragma unroll
+  for (int i = 0; i < kQuantItems; ++i) {
+    const size_t e = base + (size_t)i * (kBlock * 4);
+    v[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (e < total) { v[i] = *(const f32x4*)(w + e); }
+  }
+#pragma unroll
+  for (int i = 0; i < kQuantItems; ++i) {
+    const size_t e = base + (size_t)i * (kBlock * 4);
+    if (e >= total) { return; }   // a whole group's lanes together
+    float lo = fminf(fminf(v[i][0], v[i][1]), fminf(v[i][2], v[i][3]));
+    float hi = fmaxf(fmaxf(v[i][0], v[i][1]), fmaxf(v[i][2], v[i][3]));
+    // quad_perm [1,0,3,2] and [2,3,0,1], then the mirrors of 8 and 16 lanes
+    lo = fminf(lo, dpp<0xb1>(lo));
+    hi = fmaxf(hi, dpp<0xb1>(hi));
+    lo = fminf(lo, dpp<0x4e>(lo));
+    hi = fmaxf(hi, dpp<0x4e>(hi));
+    lo = fminf(lo, dpp<0x141>(lo));
+    hi = fmaxf(hi, dpp<0x141>(hi));
+    if constexpr (kLanes == 16) {
+      lo = fminf(lo, dpp<0x140>(lo));
+      hi = fmaxf(hi, dpp<0x140>(hi));
+    }
+    const uint16_t sc_b = f32_to_bf16((hi - lo) / qmax);
+    const uint16_t lo_b = f32_to_bf16(lo);
+    if (threadIdx.x % kLanes == 0) {
+      scales[e / GROUP] = sc_b;
+      qbias[e / GROUP] = lo_b;
+    }
+    const float scr = bf16_to_f32(sc_b);
+    const float lor = bf16_to_f32(lo_b);
+    const float d[4] = {v[i][0] - lor, v[i][1] - lor, v[i][2] - lor, v[i][3] - lor};
+    uint32_t q[4];
+    quant4(d, scr, 1.0f / scr, qmax, q);
+    if constexpr (BITS == 8) {
+      codes[e / 4] = q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24);
+    } else {
+      // eight codes per word: the odd lane's half moves to the even lane
+      const uint32_t half = q[0] | (q[1] << 4) | (q[2] << 8) | (q[3] << 12);
+      const uint32_t next = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)half, 0xb1, 0xf, 0xf, true);
+      if ((threadIdx.x & 1) == 0) { codes[e / 8] = half | (next << 16); }
+    }
+  }
+}
+
+// The same with one thread per (row, group) and single-float loads, for a
+// weight that is not 16-byte aligned.
+__global__ void __launch_bounds__(kBlock)
+quantize_affine_unaligned_kernel(const float* w, uint32_t* codes, uint16_t* scales,
+                                 uint16_t* qbias, int N, int K, int bits, int group)
 {
   const int gcols = K / group;
   const size_t gid = (size_t)blockIdx.x * kBlock + threadIdx.x;
@@ -346,10 +451,22 @@ hipError_t launch_quantize_affine(const float* w, uint32_t* codes,
                                   int K, int bits, int group,
                                   hipStream_t stream)
 {
-  const size_t groups = (size_t)N * (K / group);
-  hipLaunchKernelGGL(quantize_affine_kernel, dim3(blocks_for(groups)),
-                     dim3(kBlock), 0, stream, w, codes, scales, qbias, N, K,
-                     bits, group);
+  const size_t total = (size_t)N * K;
+  if (((uintptr_t)w & 15u) != 0) {
+    hipLaunchKernelGGL(quantize_affine_unaligned_kernel, dim3(blocks_for(total / group)),
+                       dim3(kBlock), 0, stream, w, codes, scales, qbias, N, K, bits, group);
+    return hipGetLastError();
+  }
+  const size_t per_block = (size_t)kBlock * 4 * kQuantItems;
+  const dim3 grid((unsigned)((total + per_block - 1) / per_block));
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, w, codes, scales, qbias, total);
+  };
+  if (bits == 8) {
+    group == 64 ? go(quantize_affine_kernel<8, 64>) : go(quantize_affine_kernel<8, 32>);
+  } else {
+    group == 64 ? go(quantize_affine_kernel<4, 64>) : go(quantize_affine_kernel<4, 32>);
+  }
   return hipGetLastError();
 }
 
