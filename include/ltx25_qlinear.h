@@ -226,8 +226,8 @@ int ltx25_dequant_once_takes(int M, int K, int N);
  *   TALL    256 x 256 output tiles, all of K per workgroup (the video GEMMs)
  *   MID     128 x 128 tiles, K split across workgroups until they cover the
  *           CUs once, f32 partials summed in split order by a second launch
- *   SKINNY  at most 128 tokens: 32-column slices, K split between the 8
- *           waves (and across workgroups above K = 2048)
+ *   SKINNY  at most 128 tokens: 32-column slices of 128, 64 or 32 rows, K
+ *           split between the 8 waves (and across workgroups above K = 2048)
  * ltx25_set_tile forces one for every later linear and for the second GEMM
  * of the LoRA pair (AUTO restores the planner); a forced SKINNY falls back to the planner for shapes it cannot
  * take (M > 128). Results are deterministic for a given route; different
@@ -496,7 +496,7 @@ int ltx25_probe_mfma(void* stream, int iters, int random, int waves_per_simd, vo
  * one w8 linear y = x . dequant(w)^T (+ bias) with M <= 128, through the
  * same kernel as ltx25_linear_q's M <= 128 route, instantiated with stamps
  * (the instantiations linear runs carry none). k_chunk is the K per
- * workgroup: 0 for the planner's split, else a multiple of 64 up to 2048,
+ * workgroup (of 128 rows): 0 for the planner's split, else a multiple of 64 up to 2048,
  * which forces ceil(K / k_chunk) splits (their f32 partials in the
  * library's workspace, then the split-K reduction launch, as in linear).
  * Lane 0 of each wave writes ten u64 to `stamps` (device) at

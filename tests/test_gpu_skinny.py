@@ -89,6 +89,29 @@ def test_selection_gemm_is_bit_exact(pkg, dev, M, K, N, bits, group, bias):
     assert np.array_equal(host_bits(y), orc.bf16_rne(want.astype(np.float32)))
 
 
+# The rows of a workgroup (32, 64 or 128, by how many column slices there are): M at each
+# side of a row tile, N at each side of the 256-workgroup line, chunk counts that leave
+# waves with 0 to 4 chunks.
+ROWS = [  # M, K, N, bits, group, bias
+    (31, 64, 8224, 8, 64, "none"),        # 32 rows, more slices than CUs
+    (33, 576, 4096, 8, 64, "bf16"),       # 2 x 128 slices: 32 rows, ragged second tile
+    (33, 576, 4128, 8, 64, "f32"),        # 2 x 129: 64 rows
+    (64, 1600, 8200, 4, 32, "f32"),       # 64 rows, N not whole slices
+    (65, 448, 4096, 8, 32, "none"),       # 2 x 128: 64 rows, one row in the second tile
+    (97, 1600, 4128, 8, 64, "bf16"),      # 128 rows
+    (128, 2112, 4100, 16, 64, "f32"),     # dense, split 2: 128 rows, N % 8 != 0
+    (96, 2112, 2044, 4, 64, "f32"),       # split 2: 64 rows, f32 partials four at a time
+    (127, 2048, 2048, 16, 64, "none"),    # 4 x 64: 32 rows, every ring slot used
+]
+
+
+@pytest.mark.parametrize("M,K,N,bits,group,bias", ROWS,
+                         ids=[f"M{c[0]}-K{c[1]}-N{c[2]}-w{c[3]}g{c[4]}-{c[5]}" for c in ROWS])
+def test_row_tiles_are_bit_exact(pkg, dev, M, K, N, bits, group, bias):
+    assert pkg.linear_route(M, K, N, bits)["tile"] == pkg.TILE_SKINNY
+    test_selection_gemm_is_bit_exact(pkg, dev, M, K, N, bits, group, bias)
+
+
 RAGGED = [  # M, K, N, bits, group, bias, epilogue
     (126, 64, 96, 8, 64, "f32", 0),       # one chunk: waves 1..7 idle
     (126, 448, 200, 4, 64, "bf16", 1),    # 7 chunks

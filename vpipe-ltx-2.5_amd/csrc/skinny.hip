@@ -5,15 +5,16 @@
 //
 // At these shapes the activation slab X [M][K] is small (516 KB at
 // K = 2048) and every XCD's L2 holds it after the first touch; the time is
-// set by how fast each CU pulls X and its share of the weight. A 128-column
-// tile with split-K reads 1/s of X per workgroup but writes s f32 partial
-// outputs -- at 126 tokens as many bytes as the codes -- and needs a
-// reduction launch. Here each workgroup owns a 32-column slice of the
-// output and up to 2048 of K:
+// set by how fast each CU pulls X and its share of the weight, so the rows
+// are split between workgroups as well while that fills idle CUs (rows_for).
+// A 128-column tile with split-K reads 1/s of X per workgroup but writes s
+// f32 partial outputs -- at 126 tokens as many bytes as the codes -- and
+// needs a reduction launch. Here each workgroup owns a 32-column slice of the
+// output for 128, 64 or 32 rows and up to 2048 of K:
 //   - the 8 waves split the workgroup's K into contiguous runs of 64-wide
 //     chunks, so each X element and each weight code is read once per
 //     workgroup;
-//   - a chunk of X [128 rows][64] is loaded as 128-byte row segments
+//   - a chunk of X [up to 128 rows][64] is loaded as 128-byte row segments
 //     (8 lanes per row; a load instruction that touches 32 rows at 32 bytes
 //     each moves 1.6x less per unit time from L2 on this GPU), written to
 //     the wave's own LDS slot with an XOR swizzle and read back as MFMA
@@ -51,6 +52,7 @@ constexpr int kCols = 32;            // output columns per workgroup
 constexpr int kChunk = 64;           // K per chunk
 constexpr int kMaxChunks = 4;        // chunks per wave: 2048 of K per workgroup
 constexpr int kRows = 128;           // token rows (M <= 128)
+constexpr int kHalfSlot = 8192;      // bytes: X units below it load ahead of the codes
 constexpr int kMaxGroups = kWaves * kMaxChunks * kChunk / 32;   // groups per workgroup (g32)
 // Per-wave LDS slot: the X chunk (128 rows x 128 B), the wave's codes
 // (32 rows x 256 B at most) and, after the K loop, the wave's partial tile
@@ -58,7 +60,6 @@ constexpr int kMaxGroups = kWaves * kMaxChunks * kChunk / 32;   // groups per wo
 // reduction's reads are conflict-free.
 constexpr int kRedPitch = 68;
 constexpr int kSlotBytes = 16 * kRedPitch * 16;   // 17408 >= 16384
-constexpr int kUnitBytes = 64 * 128;              // X unit: 64 rows x 128 B
 constexpr uint32_t kOob = 0x80000000u;            // past every buffer's range
 
 typedef uint32_t __attribute__((address_space(3))) lds_u32;
@@ -130,12 +131,21 @@ __device__ __forceinline__ bf16x8 dequant8(uint32_t lo, uint32_t hi, float s, fl
   return __builtin_bit_cast(bf16x8, make_uint4(o[0], o[1], o[2], o[3]));
 }
 
-template <int BITS, bool SPLIT, bool STAMPS = false>
+// ROWS: token rows per workgroup (128, 64 or 32; rows_for). The K order of
+// a row's sums does not depend on it, so neither do the output bits.
+template <int BITS, bool SPLIT, int ROWS, bool STAMPS = false>
 __global__ void __launch_bounds__(kThreads)
 skinny_kernel(SParams p)
 {
   constexpr bool QUANT = BITS != 16;
-  static_assert(2 * kUnitBytes <= kSlotBytes, "slot too small");
+  constexpr int kMb = ROWS / 32;                    // 32-row blocks
+  constexpr int kURows = ROWS < 64 ? ROWS : 64;     // rows of an X unit
+  constexpr int kUpc = ROWS / kURows;               // X units per chunk
+  constexpr int kULoads = kURows / 8;               // 1 KB loads per unit
+  constexpr int kUnitBytes = kURows * 128;
+  constexpr int kRing = 2 * kHalfSlot / kUnitBytes; // X units in the slot: 2, or 4 at 32 rows
+  constexpr int kUj = kURows / 32;                  // 32-row blocks of a unit
+  static_assert(kRing * kUnitBytes <= kSlotBytes, "slot too small");
 
   __shared__ __attribute__((aligned(16))) uint8_t lds[kWaves * kSlotBytes];
   __shared__ float lds_bias[kCols];
@@ -163,6 +173,7 @@ skinny_kernel(SParams p)
   uint8_t* const slot = lds + wave * kSlotBytes;
 
   const int n0 = blockIdx.x * kCols;
+  const int m0 = blockIdx.z * ROWS;
   const int split = SPLIT ? (int)blockIdx.y : 0;
   const int kbeg = split * p.k_chunk;
   const int nch = (min(p.K, kbeg + p.k_chunk) - kbeg) / kChunk;
@@ -219,21 +230,22 @@ skinny_kernel(SParams p)
     }
   }
 
-  // ---- X: units of 64 rows x 64 K (8 KB: rows 64 hf.. of chunk t, u = 2t + hf),
-  // loaded straight into LDS (buffer_load ... lds) through a 2-unit ring in
-  // the wave's slot. One 1 KB load covers rows 8 i..8 i+7 of the unit; lane l
-  // lands at byte 16 l of it (row 8 i + l / 8, position l % 8) and fetches the
-  // row's 16-byte segment (l % 8) ^ ((row / 2) % 8), the swizzle that keeps
-  // the fragment reads conflict-free. Rows past M read as zeros.
-  const int nunits = 2 * cnt;
+  // ---- X: units of kURows rows x 64 K (chunk t's rows kURows hf.., u = kUpc t
+  // + hf), loaded straight into LDS (buffer_load ... lds) through a ring of
+  // kRing units in the wave's slot. One 1 KB load covers rows 8 i..8 i+7 of
+  // the unit; lane l lands at byte 16 l of it (row 8 i + l / 8, position l % 8)
+  // and fetches the row's 16-byte segment (l % 8) ^ ((row / 2) % 8), the
+  // swizzle that keeps the fragment reads conflict-free. Rows past M read as
+  // zeros.
+  const int nunits = kUpc * cnt;
   auto load_unit = [&](int u) {
-    const int t = u >> 1;
-    const int hf = u & 1;
-    lds_u32* dst = (lds_u32*)(slot + (u & 1) * kUnitBytes);
+    const int t = u / kUpc;
+    const int hf = u % kUpc;
+    lds_u32* dst = (lds_u32*)(slot + (u % kRing) * kUnitBytes);
     const uint32_t soff = (uint32_t)(kw0 + t * kChunk) * 2;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r0 = 64 * hf + 8 * i;              // first row of this load
+    for (int i = 0; i < kULoads; ++i) {
+      const int r0 = m0 + kURows * hf + 8 * i;     // first row of this load
       // row r0 + l/8: swizzle (r/2) % 8 = (4 i + l/16) % 8 (r0 is a multiple of 8)
       const int sw = ((4 * i) + (lane >> 4)) & 7;
       const uint32_t vo = (uint32_t)((size_t)(r0 + (lane >> 3)) * p.K * 2 +
@@ -241,10 +253,13 @@ skinny_kernel(SParams p)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst + i * 256, 16, (int)vo, (int)soff, 0, 0);
     }
   };
+  // the units of the slot's first half go ahead of the weight, those of its
+  // second half after the codes have passed through it
+  constexpr int kAhead = kHalfSlot / kUnitBytes;
 
-  f32x16 acc[4];
+  f32x16 acc[kMb];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
+  for (int mb = 0; mb < kMb; ++mb) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) { acc[mb][r] = 0.0f; }
   }
@@ -254,18 +269,21 @@ skinny_kernel(SParams p)
   // loads into registers outstanding. (The compiler's wait counting does not
   // see direct-to-LDS loads: a register load still in flight inside the loop
   // would make it wait for the X units issued after it as well.)
-  if (nunits > 0) { load_unit(0); }
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    if (u < nunits) { load_unit(u); }
+  }
   if constexpr (QUANT) {
     // The codes [32 rows][cnt * WB bytes] as WLPR 16-byte runs per row
     // (256 B per row for w8, 128 B for w4: a load instruction covers whole
-    // rows), then through unit 1's LDS region, XOR-swizzled by row so that
+    // rows), then through the slot's second half, XOR-swizzled by row so that
     // both the writes and the fragment reads are conflict-free.
     constexpr int WB = kChunk * BITS / 8;
     constexpr int WROW = kMaxChunks * WB;
     constexpr int WLPR = WROW / 16;
     constexpr int WRPI = 64 / WLPR;
     constexpr int WNI = 32 / WRPI;
-    static_assert(32 * WROW <= kUnitBytes, "the codes must fit one X unit region");
+    static_assert(32 * WROW <= kHalfSlot, "the codes must fit the slot's second half");
     const int c16 = lane % WLPR;
     uint4 wl[WNI];
 #pragma unroll
@@ -276,7 +294,7 @@ skinny_kernel(SParams p)
                                : kOob;
       wl[i] = ld16(wr, off, (uint32_t)((size_t)kw0 * BITS / 8));
     }
-    uint8_t* const wst = slot + kUnitBytes;
+    uint8_t* const wst = slot + kHalfSlot;
 #pragma unroll
     for (int i = 0; i < WNI; ++i) {
       const int r = i * WRPI + lane / WLPR;
@@ -292,7 +310,7 @@ skinny_kernel(SParams p)
         wv[t][j] = *(const uint4*)(wst + l32 * WROW + ((s16 ^ sw) * 16));
       }
     }
-    // the region is unit 1's: its reads have returned before unit 1 lands
+    // the reads have returned before the region's X units land
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     LTX25_STAMP(st[1])
   } else {
@@ -310,7 +328,10 @@ skinny_kernel(SParams p)
       }
     }
   }
-  if (nunits > 1) { load_unit(1); }
+#pragma unroll
+  for (int u = kAhead; u < kRing; ++u) {
+    if (u < nunits) { load_unit(u); }
+  }
   if constexpr (QUANT) {
 #pragma unroll
     for (int i = 0; i < kSqLoads; ++i) {
@@ -322,34 +343,51 @@ skinny_kernel(SParams p)
   __syncthreads();   // the scale block is in LDS
   LTX25_STAMP(st[2])
 
-  // fragment reads: unit row 32 j + l32 (block mb = 2 hf + j), 16-byte
+  // fragment reads: unit row 32 j + l32 (block mb = kUj hf + j), 16-byte
   // segment 4 h + s, stored at (4 h + s) ^ ((l32 / 2) % 8)
   const int fsw = (l32 >> 1) & 7;
   bf16x8 wf[4];   // the current chunk's weight fragments
 #pragma unroll
-  for (int u = 0; u < 2 * kMaxChunks; ++u) {
+  for (int u = 0; u < kUpc * kMaxChunks; ++u) {
     if (u < nunits) {
-      const int t = u >> 1;
-      const int hf = u & 1;
-      // Unit u has landed once at most unit u+1's 8 loads are outstanding
-      // (loads complete in issue order).
-      if (u + 1 < nunits) {
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      const int t = u / kUpc;
+      const int hf = u % kUpc;
+      // Unit u has landed once at most the loads of the units issued after it
+      // are outstanding (loads complete in issue order): up to kRing - 1.
+      const int later = nunits - 1 - u;
+      if constexpr (kRing == 2) {
+        if (later > 0) {
+          asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
       } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        static_assert(kRing == 2 || (kRing == 4 && kULoads == 4 && kUpc * kMaxChunks == 4),
+                      "the waits below count 4 loads per unit, every unit in the ring");
+        if (later >= 3) {
+          asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        } else if (later == 2) {
+          asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        } else if (later == 1) {
+          asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
       }
-      const uint8_t* src = slot + (u & 1) * kUnitBytes;
-      bf16x8 xf[2][4];
+      const uint8_t* src = slot + (u % kRing) * kUnitBytes;
+      bf16x8 xf[kUj][4];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < kUj; ++j) {
 #pragma unroll
         for (int sp = 0; sp < 4; ++sp) {
           xf[j][sp] = *(const bf16x8*)(src + (32 * j + l32) * 128 + (((4 * h + sp) ^ fsw) * 16));
         }
       }
-      // the slot is free once the reads have returned; refill it with unit u+2
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (u + 2 < nunits) { load_unit(u + 2); }
+      if constexpr (kRing < kUpc * kMaxChunks) {
+        // the slot is free once the reads have returned; refill it
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (u + kRing < nunits) { load_unit(u + kRing); }
+      }
       if (hf == 0) {
         // dequantize chunk t (group of K value k0 + 32 h, relative to the
         // workgroup's first group); VALU work under the X stream
@@ -373,9 +411,9 @@ skinny_kernel(SParams p)
 #pragma unroll
       for (int sp = 0; sp < 4; ++sp) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          acc[2 * hf + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[sp], xf[j][sp],
-                                                                    acc[2 * hf + j], 0, 0, 0);
+        for (int j = 0; j < kUj; ++j) {
+          acc[kUj * hf + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[sp], xf[j][sp],
+                                                                      acc[kUj * hf + j], 0, 0, 0);
         }
       }
     }
@@ -388,7 +426,7 @@ skinny_kernel(SParams p)
   // registers 4g..4g+3 of lane l: row 32 mb + l % 32, columns
   // 8 g + 4 (l / 32) + 0..3 of the slice.
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
+  for (int mb = 0; mb < kMb; ++mb) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const f32x4 v = {acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]};
@@ -398,66 +436,80 @@ skinny_kernel(SParams p)
   __syncthreads();
   LTX25_STAMP(st[4])
 
-  // thread -> row m (0..127), 8 columns 8 nq .. 8 nq + 7
-  const int m = tid >> 2;
-  const int nq = tid & 3;
-  float v[8];
+  // thread -> row r of the workgroup's, kCpt consecutive columns from c: the
+  // f32x4 runs that hold them are run c / 8 of block r / 32, halves (c / 4) % 2
+  constexpr int kCpt = ROWS * kCols / kThreads;   // 8, 4 or 2
+  typedef float fv __attribute__((ext_vector_type(kCpt < 4 ? kCpt : 4)));
+  constexpr int kFv = kCpt < 4 ? kCpt : 4;
+  const int r = tid / (kCols / kCpt);
+  const int c = (tid % (kCols / kCpt)) * kCpt;
+  const int m = m0 + r;
+  float v[kCpt];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) { v[j] = 0.0f; }
+  for (int j = 0; j < kCpt; ++j) { v[j] = 0.0f; }
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) {
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const f32x4 a = *(const f32x4*)(lds + w * kSlotBytes +
-                                      (((m >> 5) * 4 + nq) * kRedPitch + (m & 31) + 32 * hh) * 16);
+    for (int q = 0; q < kCpt; q += kFv) {
+      const int hh = ((c + q) >> 2) & 1;
+      const fv a = *(const fv*)(lds + w * kSlotBytes +
+                                (((r >> 5) * 4 + (c >> 3)) * kRedPitch + (r & 31) + 32 * hh) * 16 +
+                                (c & 3) * 4);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) { v[4 * hh + j] += a[j]; }
+      for (int j = 0; j < kFv; ++j) { v[q + j] += a[j]; }
     }
   }
   if (m < p.M) {
-    const int n = n0 + 8 * nq;
+    const int n = n0 + c;
     if constexpr (SPLIT) {
       float* prow = p.partial + ((size_t)split * p.M + m) * p.N;
-      if ((p.N & 3) == 0 && n + 8 <= p.N) {
-        *(f32x4*)(prow + n) = f32x4{v[0], v[1], v[2], v[3]};
-        *(f32x4*)(prow + n + 4) = f32x4{v[4], v[5], v[6], v[7]};
+      if ((p.N & 3) == 0 && n + kCpt <= p.N) {
+#pragma unroll
+        for (int q = 0; q < kCpt; q += kFv) {
+          fv o;
+#pragma unroll
+          for (int j = 0; j < kFv; ++j) { o[j] = v[q + j]; }
+          *(fv*)(prow + n + q) = o;
+        }
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < kCpt; ++j) {
           if (n + j < p.N) { prow[n + j] = v[j]; }
         }
       }
     } else {
       const uint16_t* yin = p.y_in != nullptr ? p.y_in + (size_t)m * p.N : nullptr;
       uint16_t* yrow = p.y + (size_t)m * p.N;
-      const bool vec = (p.N & 7) == 0 && n + 8 <= p.N;
+      const bool vec = (p.N & 7) == 0 && n + kCpt <= p.N;
       if (yin != nullptr) {
         if (vec) {
-          const uint4 o = *(const uint4*)(yin + n);
-          const uint32_t e[4] = {o.x, o.y, o.z, o.w};
+          uint32_t e[kCpt / 2];
+          __builtin_memcpy(e, __builtin_assume_aligned(yin + n, 2 * kCpt), 2 * kCpt);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < kCpt / 2; ++j) {
             v[2 * j] += __uint_as_float(e[j] << 16);
             v[2 * j + 1] += __uint_as_float(e[j] & 0xffff0000u);
           }
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
+          for (int j = 0; j < kCpt; ++j) {
             if (n + j < p.N) { v[j] += bf16_to_f32(yin[n + j]); }
           }
         }
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        v[j] += lds_bias[8 * nq + j];
+      for (int j = 0; j < kCpt; ++j) {
+        v[j] += lds_bias[c + j];
         if (p.epilogue == kEpiGelu) { v[j] = gelu_tanh(v[j]); }
       }
       if (vec) {
-        *(uint4*)(yrow + n) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
-                                         pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+        uint32_t o[kCpt / 2];
+#pragma unroll
+        for (int j = 0; j < kCpt / 2; ++j) { o[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]); }
+        __builtin_memcpy(__builtin_assume_aligned(yrow + n, 2 * kCpt), o, 2 * kCpt);
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < kCpt; ++j) {
           if (n + j < p.N) { yrow[n + j] = f32_to_bf16(v[j]); }
         }
       }
@@ -482,6 +534,44 @@ skinny_kernel(SParams p)
       o[9] = xcc;
     }
   }
+}
+
+template <int BITS, int ROWS>
+hipError_t launch_rows(const SParams& p, const GemmPlan& plan, hipStream_t stream)
+{
+  const dim3 grid((unsigned)((p.N + kCols - 1) / kCols), (unsigned)plan.splits,
+                  (unsigned)((p.M + ROWS - 1) / ROWS));
+  if (plan.splits > 1) {
+    hipLaunchKernelGGL((skinny_kernel<BITS, true, ROWS>), grid, dim3(kThreads), 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((skinny_kernel<BITS, false, ROWS>), grid, dim3(kThreads), 0, stream, p);
+  }
+  return hipGetLastError();
+}
+
+template <int BITS>
+hipError_t launch_bits(const SParams& p, const GemmPlan& plan, int rows, hipStream_t stream)
+{
+  return rows == 32   ? launch_rows<BITS, 32>(p, plan, stream)
+         : rows == 64 ? launch_rows<BITS, 64>(p, plan, stream)
+                      : launch_rows<BITS, 128>(p, plan, stream);
+}
+
+// Token rows per workgroup. A workgroup's time is set by the X rows it pulls
+// from L2, so while the column slices leave CUs idle, fewer rows on more
+// workgroups are faster, although each re-reads its slice of the weight; a
+// second round of workgroups costs more than it gives. w8g64, one call in a
+// captured burst on rotated weights, at 32 / 64 / 128 rows: 126 x 2048 -> 2048
+// (64 slices) 7.2 / 8.2 / 10.1 us; -> 4096 13.3 / 8.8 / 10.7; -> 6144 19.2 /
+// 15.4 / 11.6; -> 8192 25.6 / 16.9 / 12.6. Rows past M are work for nothing:
+// 32 tokens 4096 -> 12288 26.2 / 28.4 / 34.5, 64 tokens 2048 -> 8192 14.4 /
+// 9.8 / 11.9.
+int rows_for(int M, int N, int splits, int cu_count)
+{
+  const long cols = (long)((N + kCols - 1) / kCols) * splits;
+  if (M <= 32 || (M + 31) / 32 * cols <= cu_count) { return 32; }
+  if (M <= 64 || (M + 63) / 64 * cols <= cu_count) { return 64; }
+  return 128;
 }
 
 }  // namespace
@@ -540,35 +630,23 @@ hipError_t launch_skinny(const GemmDesc& d, const GemmPlan& plan, float* workspa
   p.gcols = d.bits == 16 ? 0 : d.K / d.group;
   p.k_chunk = plan.k_chunk;
   p.stamps = stamps;
-  const dim3 grid((unsigned)((d.N + kCols - 1) / kCols), (unsigned)plan.splits, 1);
   const bool split = plan.splits > 1;
+  hipError_t e = hipSuccess;
   if (stamps != nullptr) {
-    // the phase-stamp instantiation (w8 only), for the probe entry point
+    // the phase-stamp instantiation (w8, 128 rows), for the probe entry point
+    const dim3 grid((unsigned)((d.N + kCols - 1) / kCols), (unsigned)plan.splits, 1);
     if (split) {
-      hipLaunchKernelGGL((skinny_kernel<8, true, true>), grid, dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL((skinny_kernel<8, true, kRows, true>), grid, dim3(kThreads), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((skinny_kernel<8, false, true>), grid, dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL((skinny_kernel<8, false, kRows, true>), grid, dim3(kThreads), 0, stream, p);
     }
-  } else if (d.bits == 8) {
-    if (split) {
-      hipLaunchKernelGGL((skinny_kernel<8, true>), grid, dim3(kThreads), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((skinny_kernel<8, false>), grid, dim3(kThreads), 0, stream, p);
-    }
-  } else if (d.bits == 16) {
-    if (split) {
-      hipLaunchKernelGGL((skinny_kernel<16, true>), grid, dim3(kThreads), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((skinny_kernel<16, false>), grid, dim3(kThreads), 0, stream, p);
-    }
+    e = hipGetLastError();
   } else {
-    if (split) {
-      hipLaunchKernelGGL((skinny_kernel<4, true>), grid, dim3(kThreads), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((skinny_kernel<4, false>), grid, dim3(kThreads), 0, stream, p);
-    }
+    const int rows = rows_for(d.M, d.N, plan.splits, plan.cu_count);
+    e = d.bits == 8    ? launch_bits<8>(p, plan, rows, stream)
+        : d.bits == 16 ? launch_bits<16>(p, plan, rows, stream)
+                       : launch_bits<4>(p, plan, rows, stream);
   }
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess || !split) { return e; }
   return launch_splitk_reduce(workspace, plan.splits, d.bias, p.bias_type, d.epilogue, d.y_in,
                               d.y, d.M, d.N, stream);
