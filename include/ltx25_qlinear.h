@@ -224,9 +224,15 @@ int ltx25_dequant_once_takes(int M, int K, int N);
 
 /* Tile families of the GEMM behind ltx25_linear / ltx25_linear_q:
  *   TALL    256 x 256 output tiles, all of K per workgroup (the video GEMMs)
- *   MID     128 x 128 tiles, K split across workgroups until they cover the
- *           CUs once, f32 partials summed in split order by a second launch
- *   SKINNY  at most 128 tokens: 32-column slices of 128, 64 or 32 rows, K
+ *   MID     the shapes between: under AUTO and from K = 1024, panels of 32 to
+ *           128 rows x 32 or 64 columns that split K between a workgroup's
+ *           waves (and, at large K, across workgroups) where one round of
+ *           workgroups holds them; else, and when forced, 128 x 128 tiles, K
+ *           split across workgroups until they cover the CUs once. Splits
+ *           across workgroups write f32 partials that a second launch sums in
+ *           split order
+ *   SKINNY  at most 128 tokens, while one round of workgroups holds them or no
+ *           panel does: 32-column slices of 128, 64 or 32 rows, K
  *           split between the 8 waves (and across workgroups above K = 2048)
  * ltx25_set_tile forces one for every later linear and for the second GEMM
  * of the LoRA pair (AUTO restores the planner); a forced SKINNY falls back to the planner for shapes it cannot

@@ -96,10 +96,10 @@ ROWS = [  # M, K, N, bits, group, bias
     (31, 64, 8224, 8, 64, "none"),        # 32 rows, more slices than CUs
     (33, 576, 4096, 8, 64, "bf16"),       # 2 x 128 slices: 32 rows, ragged second tile
     (33, 576, 4128, 8, 64, "f32"),        # 2 x 129: 64 rows
-    (64, 1600, 8200, 4, 32, "f32"),       # 64 rows, N not whole slices
+    (64, 960, 8200, 4, 32, "f32"),        # 64 rows, N not whole slices
     (65, 448, 4096, 8, 32, "none"),       # 2 x 128: 64 rows, one row in the second tile
     (97, 1600, 4128, 8, 64, "bf16"),      # 128 rows
-    (128, 2112, 4100, 16, 64, "f32"),     # dense, split 2: 128 rows, N % 8 != 0
+    (128, 2112, 4090, 16, 64, "f32"),     # dense, split 2: 128 rows, N % 8 != 0
     (96, 2112, 2044, 4, 64, "f32"),       # split 2: 64 rows, f32 partials four at a time
     (127, 2048, 2048, 16, 64, "none"),    # 4 x 64: 32 rows, every ring slot used
 ]

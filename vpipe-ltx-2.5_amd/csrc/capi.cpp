@@ -637,7 +637,7 @@ FoldPlan plan_fold(int M, int K, int N, int rank, int bits, int cu_count, const 
     return f;
   }
   const int tile = g_tile.load(std::memory_order_relaxed);
-  f.plan = ltx25::plan_gemm(M, N, kt, 16, cu_count, tile);
+  f.plan = ltx25::plan_gemm(M, N, kt, 16, cu_count, tile, false);
   if (f.plan.tile == 2) { return f; }
   f.r_plan = ltx25::plan_gemm(M, rk, K, 16, cu_count);
   // the merge's shape rule (A's alignment and the group size are checked

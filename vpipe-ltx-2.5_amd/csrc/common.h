@@ -123,6 +123,10 @@ struct GemmPlan {
   int splits = 1;    // split-K factor
   int k_chunk = 0;   // K elements per split (multiple of 64)
   size_t workspace_bytes = 0;   // f32 partials when splits > 1
+  // tile 1 only: rows and columns of a workgroup of panel.hip, which splits
+  // K between its waves; 0 for the 128 x 128 tile
+  int panel_rows = 0;
+  int panel_cols = 0;
   int cu_count = 256;           // CUs of the device planned for (persistent grids)
 };
 
@@ -130,17 +134,29 @@ struct GemmPlan {
 // `force` (the LTX25_TILE_* values): 0 the planner's choice; 1 the
 // 256 x 256 tile; 2 the 128 x 128 split-K tile; 3 the M <= 128 kernel
 // where it takes the shape, else the planner's choice.
-GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force = 0);
+// `panels` false: without panel.hip's plans (the two-part activation).
+GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force = 0,
+                   bool panels = true);
 hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
                        float* workspace, hipStream_t stream);
 // The M <= 128 route (skinny.hip): 32 output columns per workgroup, K split
 // between its 8 waves, and across workgroups above 2048. Fills `plan` and
-// returns true when it takes the shape (up to 3 workgroups per CU).
+// returns true when it takes the shape (up to 3 workgroups per CU);
+// skinny_workgroups is the grid it would launch.
+long skinny_workgroups(int M, int N, const GemmPlan& plan);
 bool plan_skinny(int M, int N, int K, int bits, int cu_count, GemmPlan& plan);
 // `stamps` non-null (w8 only): the phase-stamp instantiation, ten words per
 // wave at [(split * ceil(N / 32) + tile) * 8 + wave] * 10 (ltx25_probe_skinny_phases)
 hipError_t launch_skinny(const GemmDesc& d, const GemmPlan& plan, float* workspace,
                          hipStream_t stream, unsigned long long* stamps = nullptr);
+// The panel kernel (panel.hip): panel_rows x panel_cols outputs per workgroup,
+// K split between its waves. Any N; no two-part activation. plan_panel picks
+// the panel and the K splits for which one round of workgroups is expected to
+// end soonest, and returns false when none fits the CUs in one round. The plan
+// does not depend on the weight's format.
+bool plan_panel(int M, int N, int K, int cu_count, GemmPlan& plan);
+hipError_t launch_panel(const GemmDesc& d, const GemmPlan& plan, float* workspace,
+                        hipStream_t stream);
 // The dense bf16 GEMM of the 256 x 256 tile on v_mfma_f32_16x16x32_bf16
 // (tall.hip): the dequant-once arm and dense weights, also with the LoRA
 // fold's two-part activation [x | r] (kx a multiple of 64), or with y_in

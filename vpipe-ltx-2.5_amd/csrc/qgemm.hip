@@ -813,11 +813,22 @@ int ilog2(int v)
 
 }  // namespace
 
-GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force)
+GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force, bool panels)
 {
   GemmPlan plan;
   plan.cu_count = cu_count;
-  if ((force == 0 || force == 3) && plan_skinny(M, N, K, bits, cu_count, plan)) { return plan; }
+  if ((force == 0 || force == 3) && plan_skinny(M, N, K, bits, cu_count, plan)) {
+    // The M <= 128 kernel while its workgroups fit the CUs once; past that a
+    // panel where one fits: 126 x 4096 -> 8192 29.2 us on two rounds of the
+    // former, 19.0 on the latter; 1 x 4096 -> 8192 18.3 and 11.3; 126 x 2048 ->
+    // 16384 24.3 and 18.7.
+    GemmPlan panel = plan;
+    if (force == 0 && panels && skinny_workgroups(M, N, plan) > cu_count &&
+        plan_panel(M, N, K, cu_count, panel)) {
+      return panel;
+    }
+    return plan;
+  }
   const long tall_tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
   // a forced M <= 128 kernel that cannot take the shape leaves the choice
   // to the planner
@@ -827,6 +838,7 @@ GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force)
     plan.k_chunk = K;
     return plan;
   }
+  if ((force == 0 || force == 3) && panels && plan_panel(M, N, K, cu_count, plan)) { return plan; }
   plan.tile = 1;
   const long tiles = (long)((M + 127) / 128) * ((N + kMidBN - 1) / kMidBN);
   // Split K until the workgroups cover the CUs once, with at least 512 of K
@@ -907,6 +919,7 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
     return hipErrorInvalidValue;   // the M <= 128 kernel reads all N weight rows
   }
   if (plan.tile == 2) { return launch_skinny(d, plan, workspace, stream); }
+  if (plan.panel_rows > 0 && d.x2 == nullptr) { return launch_panel(d, plan, workspace, stream); }
   if (tall_dense_takes(d, plan) || tall_w8_takes(d, plan)) { return launch_tall_dense(d, stream); }
   KParams kp = {};
   kp.x = d.x;

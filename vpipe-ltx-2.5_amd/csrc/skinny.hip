@@ -601,6 +601,12 @@ bool plan_skinny(int M, int N, int K, int bits, int cu_count, GemmPlan& plan)
   return true;
 }
 
+long skinny_workgroups(int M, int N, const GemmPlan& plan)
+{
+  const int rows = rows_for(M, N, plan.splits, plan.cu_count);
+  return (long)((N + kCols - 1) / kCols) * plan.splits * ((M + rows - 1) / rows);
+}
+
 hipError_t launch_skinny(const GemmDesc& d, const GemmPlan& plan, float* workspace,
                          hipStream_t stream, unsigned long long* stamps)
 {
