@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import orc
-from gpu_util import dev_bf16, dev_f32, host_bits, host_f32, make_qweight, rng_normal, say
+from gpu_util import dev_bf16, dev_bytes, dev_f32, host_bits, host_f32, make_qweight, rng_normal, say
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
@@ -82,6 +82,71 @@ def test_quantize_rows_at_half_integer_quotients(pkg):
     q_ref, s_ref = orc.i8_quantize_rows(x)
     assert np.array_equal(sc.cpu().numpy(), s_ref)
     assert np.array_equal(q.cpu().numpy(), q_ref)
+
+
+@pytest.mark.parametrize("K", [8, 1000, 1032, 2056, 4096, 4104, 8192, 8200])
+def test_quantize_rows_edges(pkg, K):
+    """Every instance of the register cache, partly filled, on rows of one value, of denormals
+    (1 / scale overflows), of the largest values, and on rows with NaN (passed over by the
+    maximum; their own quotients clamp to -127) and infinities (scale infinity: finite values
+    give 0, the infinities a NaN quotient)."""
+    rng = np.random.default_rng(32 + K)
+    x = orc.bf16_to_f32(orc.bf16_rne(rng_normal(rng, (12, K))))
+    x[0] = 0.0
+    x[0, K - 1] = -3.0
+    x[1] *= 2.0 ** -131
+    x[2] *= 1e-40
+    x[3] *= 5e37
+    x = orc.bf16_rne(x.astype(np.float32))
+    at = rng.integers(0, K, 4)
+    nan, inf = x.copy(), x.copy()
+    nan[4:8, at] = 0x7fc0
+    nan[5, at] = 0xffff
+    inf[8, at[0]] = 0x7f80
+    inf[9, at] = 0xff80
+    say(f"i8 quantize rows edges K={K}")
+    q, s = (t.cpu().numpy() for t in quantize_rows_dev(pkg, dev_bf16(x), 12, K))
+    q_ref, s_ref = orc.i8_quantize_rows(x)
+    assert np.array_equal(s, s_ref)
+    assert np.array_equal(q, q_ref)
+    zeroed = nan.copy()
+    zeroed[4:8, at] = 0
+    q_ref, s_ref = orc.i8_quantize_rows(zeroed)
+    q_ref[4:8, at] = np.where(s_ref[4:8, None] > 0, -127, 0)
+    q, s = (t.cpu().numpy() for t in quantize_rows_dev(pkg, dev_bf16(nan), 12, K))
+    assert np.array_equal(s, s_ref)
+    assert np.array_equal(q, q_ref)
+    q, s = (t.cpu().numpy() for t in quantize_rows_dev(pkg, dev_bf16(inf), 12, K))
+    for r, cols in ((8, at[:1]), (9, at)):
+        want = np.zeros(K, np.int8)
+        want[cols] = -127
+        assert np.isinf(s[r]) and np.array_equal(q[r], want)
+
+
+@pytest.mark.parametrize("bits,group", [(8, 64), (8, 32), (4, 64), (4, 32)])
+def test_quantize_qweight_extreme_codes(pkg, bits, group):
+    """The absmax comes from each chunk's least and greatest code: negative scales, zero scales,
+    zero points of either sign, rows whose maximum sits at one end or the other, chunk counts
+    that leave lanes idle."""
+    N, K = 37, 1344
+    rng = np.random.default_rng(33 + bits + group)
+    codes = rng.integers(0, 1 << bits, (N, K), dtype=np.uint8)
+    codes[0] = 0
+    codes[1] = (1 << bits) - 1
+    scales = orc.bf16_rne((rng_normal(rng, (N, K // group), 0.02)).astype(np.float32))
+    biases = orc.bf16_rne((rng_normal(rng, (N, K // group), 1.0)).astype(np.float32))
+    scales[2] = 0
+    words = orc.pack(codes, bits)
+    _, wb = orc.dequant(words, scales, biases, N, K, bits, group)
+    qw = pkg.QWeight(dev_bytes(words), dev_bf16(scales), dev_bf16(biases), bits, group)
+    wq = torch.empty((N, K), dtype=torch.int8, device="cuda")
+    sw = torch.empty((N,), dtype=torch.float32, device="cuda")
+    say(f"i8 quantize of extreme codes w{bits}g{group}")
+    pkg.i8_quantize_qweight(qw, wq, sw, N, K)
+    torch.cuda.synchronize()
+    q_ref, s_ref = orc.i8_quantize_rows(wb.reshape(N, K))
+    assert np.array_equal(sw.cpu().numpy(), s_ref)
+    assert np.array_equal(wq.cpu().numpy(), q_ref)
 
 
 @pytest.mark.parametrize("N,K,bits,group", [

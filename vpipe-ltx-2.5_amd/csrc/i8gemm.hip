@@ -11,49 +11,72 @@
 // src/ltx25-metal-ops.cc:386-391; contract at src/ltx25-metal-ops.h:810-817).
 #include "common.h"
 
+#include <type_traits>
+
 namespace ltx25 {
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kRowsPerBlock = kThreads / 64;   // one wave per row
 
+// Both quantizers are bound by memory (the row in, its int8 out) once their
+// arithmetic, two passes over values that stay in registers, keeps up: at 8160
+// x 4096 a plain copy of the bytes is 20 us, so every value has about 18 VALU
+// instructions in all.
+
 // 16-byte chunks a lane keeps in registers between the absmax pass and the
-// quantize pass (K up to 8192 bf16 or 16384 w8 codes); chunks past them are
-// read again for the second pass.
-constexpr int kCacheChunks = 16;
+// quantize pass: the instance for a row's K keeps no more than it needs, up to
+// kMaxChunks (K up to 8192 bf16, 16384 w8 codes); chunks past them are read again
+// for the second pass.
+constexpr int kMaxChunks = 16;
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b)
+{
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a),
+                                                                __builtin_bit_cast(u16x2, b)));
+}
+
+__device__ __forceinline__ uint32_t pk_min_u16(uint32_t a, uint32_t b)
+{
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a),
+                                                                __builtin_bit_cast(u16x2, b)));
+}
 
 // q = clamp(rint(v / s), -127, 127) with v / s correctly rounded, given
 // rs = 1 / s rounded, for four values packed low byte first. t = v * rs is
-// within 2^-24 |v / s| (1 + 2^-24) of the quotient, i.e. within 2^-15 for
-// |t| < 256; so rint(t) = rint(v / s) unless t lies within 2^-13 of a
-// half-integer. Those values, and any t that is not a finite number below
-// 256 (s tiny, v or s not finite), take the division itself. The test for
-// that fallback is made once for the four values (a test per value was a
-// branch per value around the rarely taken division); s <= 0 gives 0.
+// within 2^-21.9 |v / s| of the quotient (rs keeps at least 21 bits), i.e.
+// within 2^-14.9 for |t| <= 127; so rint(t) = rint(v / s) unless t lies within
+// 2^-13 of a half-integer, and a quotient past 127 clamps to the same end.
+// t + 1.5 * 2^23 rounds to the integer and holds it in its low bits. Values
+// near a half-integer take the division itself, tested once for the four; so
+// does every value when 1 / s overflows (rs not finite). A NaN gives -127 on
+// either way; s <= 0 gives 0.
 __device__ __forceinline__ uint32_t q8x4(const float* v, float s, float rs)
 {
+  constexpr float kMagic = 12582912.0f;   // 1.5 * 2^23
   if (!(s > 0.0f)) { return 0u; }
-  float r[4];
-  int slow = 0;
+  uint32_t bits[4];
+  float off = rs < __builtin_inff() ? 0.0f : 1.0f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const float t = v[j] * rs;
-    r[j] = rintf(t);
-    slow |= (int)!(fabsf(t) < 256.0f) | (int)(fabsf(t - r[j]) > 0.5f - 0x1p-13f);
+    const float t = fminf(fmaxf(v[j] * rs, -127.0f), 127.0f);
+    const float m = t + kMagic;
+    bits[j] = __float_as_uint(m);
+    off = fmaxf(off, fabsf(t - (m - kMagic)));
   }
-  if (slow) {
+  if (off > 0.5f - 0x1p-13f) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float t = v[j] * rs;
-      if (!(fabsf(t) < 256.0f) || fabsf(t - r[j]) > 0.5f - 0x1p-13f) { r[j] = rintf(v[j] / s); }
+      bits[j] = __float_as_uint(fminf(fmaxf(rintf(v[j] / s), -127.0f), 127.0f) + kMagic);
     }
   }
-  uint32_t out = 0u;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    out |= ((uint32_t)(int)fminf(fmaxf(r[j], -127.0f), 127.0f) & 0xffu) << (8 * j);
-  }
-  return out;
+  // the four low bytes: v_perm picks bytes 0..3 of its second operand, 4..7 of its first
+  const uint32_t lo = __builtin_amdgcn_perm(bits[1], bits[0], 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(bits[3], bits[2], 0x04000c0cu);
+  return lo | hi;
 }
 
 __device__ __forceinline__ float wave_absmax(float amax)
@@ -67,8 +90,12 @@ __device__ __forceinline__ float wave_absmax(float amax)
 // One wave per row: absmax, then q = clamp(rint(x / s), -127, 127),
 // s = absmax / 127. Works on bf16 activations (values exact in f32). Lane l
 // takes 16-byte chunks l, l + 64, ...: every load instruction of the wave
-// covers 1 KB of the row, up to 16 of them in flight per lane, and the
-// row's maximum is a shuffle reduction (no LDS, no barrier).
+// covers 1 KB of the row, NC of them in flight per lane, and the row's
+// maximum is a shuffle reduction (no LDS, no barrier). The absmax runs on the
+// bf16 bits, two a time, sign bits cleared: their order is the values' order;
+// a row with a NaN (bits past infinity's) takes its maximum again in floats,
+// which passes NaNs over.
+template <int NC>
 __global__ void __launch_bounds__(kThreads)
 i8_quantize_rows_kernel(const uint16_t* x, int8_t* q, float* scale, int M, int K)
 {
@@ -78,46 +105,57 @@ i8_quantize_rows_kernel(const uint16_t* x, int8_t* q, float* scale, int M, int K
   const uint16_t* xr = x + (size_t)m * K;
   int8_t* qr = q + (size_t)m * K;
   const int chunks = K / 8;
-  uint4 cache[kCacheChunks];
-  float amax = 0.0f;
-  auto absmax8 = [&](const uint4& v) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  u32x4 cache[NC];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      amax = fmaxf(amax, fabsf(bf16_to_f32((uint16_t)(w[j] & 0xffffu))));
-      amax = fmaxf(amax, fabsf(bf16_to_f32((uint16_t)(w[j] >> 16))));
-    }
+  for (int c = 0; c < NC; ++c) {
+    const int i = lane + c * 64;
+    cache[c] = u32x4{0u, 0u, 0u, 0u};
+    if (i < chunks) { cache[c] = *(const u32x4*)(xr + (size_t)i * 8); }
+  }
+  uint32_t mx = 0u;
+  auto absmax8 = [&](const u32x4& v) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { mx = pk_max_u16(mx, v[j] & 0x7fff7fffu); }
   };
 #pragma unroll
-  for (int c = 0; c < kCacheChunks; ++c) {
-    const int i = lane + c * 64;
-    if (i < chunks) { cache[c] = *(const uint4*)(xr + (size_t)i * 8); }
+  for (int c = 0; c < NC; ++c) { absmax8(cache[c]); }
+  for (int i = lane + NC * 64; i < chunks; i += 64) {
+    absmax8(*(const u32x4*)(xr + (size_t)i * 8));
   }
+  const uint32_t top = mx >> 16 > (mx & 0xffffu) ? mx >> 16 : mx & 0xffffu;
+  // bits of non-negative floats order as the floats do
+  float amax = __uint_as_float(top << 16);
+  if (__any(top > 0x7f80u)) {
+    amax = 0.0f;
+    for (int i = lane; i < chunks; i += 64) {
+      const u32x4 v = *(const u32x4*)(xr + (size_t)i * 8);
 #pragma unroll
-  for (int c = 0; c < kCacheChunks; ++c) {
-    if (lane + c * 64 < chunks) { absmax8(cache[c]); }
-  }
-  for (int i = lane + kCacheChunks * 64; i < chunks; i += 64) {
-    absmax8(*(const uint4*)(xr + (size_t)i * 8));
+      for (int j = 0; j < 4; ++j) {
+        amax = fmaxf(amax, fabsf(bf16_to_f32((uint16_t)(v[j] & 0xffffu))));
+        amax = fmaxf(amax, fabsf(bf16_to_f32((uint16_t)(v[j] >> 16))));
+      }
+    }
   }
   amax = wave_absmax(amax);
   const float s = amax / 127.0f;
   const float rs = 1.0f / s;
   if (lane == 0) { scale[m] = s; }
-  auto quant8 = [&](const uint4& v, int i) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  auto quant8 = [&](const u32x4& v, int i) {
     float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { f[j] = bf16_to_f32((uint16_t)(w[j >> 1] >> (16 * (j & 1)))); }
+    for (int j = 0; j < 4; ++j) {
+      f[2 * j] = __uint_as_float(v[j] << 16);
+      f[2 * j + 1] = __uint_as_float(v[j] & 0xffff0000u);
+    }
     *(uint2*)(qr + (size_t)i * 8) = make_uint2(q8x4(f, s, rs), q8x4(f + 4, s, rs));
   };
 #pragma unroll
-  for (int c = 0; c < kCacheChunks; ++c) {
+  for (int c = 0; c < NC; ++c) {
     const int i = lane + c * 64;
     if (i < chunks) { quant8(cache[c], i); }
   }
-  for (int i = lane + kCacheChunks * 64; i < chunks; i += 64) {
-    quant8(*(const uint4*)(xr + (size_t)i * 8), i);
+  for (int i = lane + NC * 64; i < chunks; i += 64) {
+    quant8(*(const u32x4*)(xr + (size_t)i * 8), i);
   }
 }
 
@@ -125,7 +163,9 @@ i8_quantize_rows_kernel(const uint16_t* x, int8_t* q, float* scale, int M, int K
 // w = bf16(fma(scale, q, qbias)): one wave per row, one 16-byte load of
 // codes (16 w8 or 32 w4 codes, all in one group) per chunk, kept in
 // registers between the absmax and the quantize pass; 16-byte int8 stores.
-template <int BITS>
+// Within a group w is monotone in its code (the fma and the rounding are), so
+// a chunk's absmax is that of its least and greatest code, found on the codes.
+template <int BITS, int NC>
 __global__ void __launch_bounds__(kThreads)
 i8_quantize_qweight_kernel(const uint8_t* codes, const uint16_t* scales,
                            const uint16_t* qbias, int gshift, int gcols,
@@ -140,54 +180,73 @@ i8_quantize_qweight_kernel(const uint8_t* codes, const uint16_t* scales,
   const uint16_t* brow = qbias + (size_t)n * gcols;
   int8_t* qr = q + (size_t)n * K;
   const int chunks = K / CPC;
-  uint4 cache[kCacheChunks];
-  float amax = 0.0f;
-  // the CPC dequantized values of chunk i, in order, into v
-  auto dequant = [&](const uint4& c, int i, float* v) {
-    const int g = (i * CPC) >> gshift;
-    const float s = bf16_to_f32(srow[g]);
-    const float b = bf16_to_f32(brow[g]);
-    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+  u32x4 cache[NC];
+  float sc[NC], zp[NC];
 #pragma unroll
-    for (int j = 0; j < CPC; ++j) {
-      uint32_t code;
-      if constexpr (BITS == 8) {
-        code = (w[j >> 2] >> (8 * (j & 3))) & 0xffu;
-      } else {
-        code = (w[j >> 3] >> (4 * (j & 7))) & 0xfu;
-      }
-      v[j] = bf16_to_f32(f32_to_bf16(fmaf(s, (float)code, b)));
+  for (int c = 0; c < NC; ++c) {
+    const int i = lane + c * 64;
+    cache[c] = u32x4{0u, 0u, 0u, 0u};
+    sc[c] = zp[c] = 0.0f;
+    if (i < chunks) {
+      cache[c] = *(const u32x4*)(cr + (size_t)i * 16);
+      sc[c] = bf16_to_f32(srow[(i * CPC) >> gshift]);
+      zp[c] = bf16_to_f32(brow[(i * CPC) >> gshift]);
     }
-  };
-  auto absmax_chunk = [&](const uint4& c, int i) {
-    float v[CPC];
-    dequant(c, i, v);
-#pragma unroll
-    for (int j = 0; j < CPC; ++j) { amax = fmaxf(amax, fabsf(v[j])); }
-  };
-#pragma unroll
-  for (int c = 0; c < kCacheChunks; ++c) {
-    const int i = lane + c * 64;
-    if (i < chunks) { cache[c] = *(const uint4*)(cr + (size_t)i * 16); }
   }
+  float amax = 0.0f;
+  auto absmax_chunk = [&](const u32x4& c, float s, float b) {
+    uint32_t lo = 0xffffffffu, hi = 0u;   // two u16 lanes of codes each
+    auto two = [&](uint32_t v) {
+      lo = pk_min_u16(lo, v);
+      hi = pk_max_u16(hi, v);
+    };
 #pragma unroll
-  for (int c = 0; c < kCacheChunks; ++c) {
-    const int i = lane + c * 64;
-    if (i < chunks) { absmax_chunk(cache[c], i); }
-  }
-  for (int i = lane + kCacheChunks * 64; i < chunks; i += 64) {
-    absmax_chunk(*(const uint4*)(cr + (size_t)i * 16), i);
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (BITS == 8) {
+        two(c[j] & 0x00ff00ffu);
+        two((c[j] >> 8) & 0x00ff00ffu);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) { two((c[j] >> (4 * t)) & 0x000f000fu); }
+      }
+    }
+    const uint32_t l = min(lo >> 16, lo & 0xffffu);
+    const uint32_t h = max(hi >> 16, hi & 0xffffu);
+    amax = fmaxf(amax, fabsf(bf16_to_f32(f32_to_bf16(fmaf(s, (float)l, b)))));
+    amax = fmaxf(amax, fabsf(bf16_to_f32(f32_to_bf16(fmaf(s, (float)h, b)))));
+  };
+#pragma unroll
+  for (int c = 0; c < NC; ++c) { absmax_chunk(cache[c], sc[c], zp[c]); }   // past the row: 0
+  for (int i = lane + NC * 64; i < chunks; i += 64) {
+    absmax_chunk(*(const u32x4*)(cr + (size_t)i * 16), bf16_to_f32(srow[(i * CPC) >> gshift]),
+                 bf16_to_f32(brow[(i * CPC) >> gshift]));
   }
   amax = wave_absmax(amax);
   const float s = amax / 127.0f;
   const float rs = 1.0f / s;
   if (lane == 0) { scale[n] = s; }
-  auto quant_chunk = [&](const uint4& c, int i) {
-    float v[CPC];
-    dequant(c, i, v);
+  auto quant_chunk = [&](const u32x4& c, float gs, float gb, int i) {
     uint32_t packed[CPC / 4];
 #pragma unroll
-    for (int t = 0; t < CPC / 4; ++t) { packed[t] = q8x4(v + 4 * t, s, rs); }
+    for (int t = 0; t < CPC / 4; ++t) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const int k = 4 * t + j;   // codes k and k + 1
+        uint32_t c0, c1;
+        if constexpr (BITS == 8) {
+          c0 = (c[k >> 2] >> (8 * (k & 3))) & 0xffu;
+          c1 = (c[k >> 2] >> (8 * (k & 3) + 8)) & 0xffu;
+        } else {
+          c0 = (c[k >> 3] >> (4 * (k & 7))) & 0xfu;
+          c1 = (c[k >> 3] >> (4 * (k & 7) + 4)) & 0xfu;
+        }
+        const uint32_t w = pack_bf16x2(fmaf(gs, (float)c0, gb), fmaf(gs, (float)c1, gb));
+        v[j] = __uint_as_float(w << 16);
+        v[j + 1] = __uint_as_float(w & 0xffff0000u);
+      }
+      packed[t] = q8x4(v, s, rs);
+    }
 #pragma unroll
     for (int t = 0; t < CPC / 16; ++t) {
       *(uint4*)(qr + (size_t)i * CPC + 16 * t) =
@@ -195,12 +254,30 @@ i8_quantize_qweight_kernel(const uint8_t* codes, const uint16_t* scales,
     }
   };
 #pragma unroll
-  for (int c = 0; c < kCacheChunks; ++c) {
+  for (int c = 0; c < NC; ++c) {
     const int i = lane + c * 64;
-    if (i < chunks) { quant_chunk(cache[c], i); }
+    if (i < chunks) { quant_chunk(cache[c], sc[c], zp[c], i); }
   }
-  for (int i = lane + kCacheChunks * 64; i < chunks; i += 64) {
-    quant_chunk(*(const uint4*)(cr + (size_t)i * 16), i);
+  for (int i = lane + NC * 64; i < chunks; i += 64) {
+    quant_chunk(*(const u32x4*)(cr + (size_t)i * 16), bf16_to_f32(srow[(i * CPC) >> gshift]),
+                bf16_to_f32(brow[(i * CPC) >> gshift]), i);
+  }
+}
+
+// go(integral_constant): the smallest instance whose lanes hold a row of
+// `chunks` 16-byte chunks, or the largest
+template <typename F>
+void with_chunks(int chunks, F&& go)
+{
+  const int per_lane = (chunks + 63) / 64;
+  if (per_lane <= 2) {
+    go(std::integral_constant<int, 2>{});
+  } else if (per_lane <= 4) {
+    go(std::integral_constant<int, 4>{});
+  } else if (per_lane <= 8) {
+    go(std::integral_constant<int, 8>{});
+  } else {
+    go(std::integral_constant<int, kMaxChunks>{});
   }
 }
 
@@ -217,7 +294,10 @@ hipError_t launch_i8_quantize_rows(const uint16_t* x, int8_t* q, float* s,
                                    int M, int K, hipStream_t stream)
 {
   const dim3 grid((unsigned)((M + kRowsPerBlock - 1) / kRowsPerBlock));
-  hipLaunchKernelGGL(i8_quantize_rows_kernel, grid, dim3(kThreads), 0, stream, x, q, s, M, K);
+  with_chunks(K / 8, [&](auto nc) {
+    hipLaunchKernelGGL((i8_quantize_rows_kernel<decltype(nc)::value>), grid, dim3(kThreads), 0,
+                       stream, x, q, s, M, K);
+  });
   return hipGetLastError();
 }
 
@@ -230,13 +310,16 @@ hipError_t launch_i8_quantize_qweight(const void* codes,
   const int gshift = ilog2(group);
   const int gcols = K / group;
   const dim3 grid((unsigned)((N + kRowsPerBlock - 1) / kRowsPerBlock));
-  if (bits == 8) {
-    hipLaunchKernelGGL(i8_quantize_qweight_kernel<8>, grid, dim3(kThreads), 0, stream,
-                       (const uint8_t*)codes, scales, qbias, gshift, gcols, q, s, N, K);
-  } else {
-    hipLaunchKernelGGL(i8_quantize_qweight_kernel<4>, grid, dim3(kThreads), 0, stream,
-                       (const uint8_t*)codes, scales, qbias, gshift, gcols, q, s, N, K);
-  }
+  with_chunks(K / (128 / bits), [&](auto nc) {
+    constexpr int NC = decltype(nc)::value;
+    if (bits == 8) {
+      hipLaunchKernelGGL((i8_quantize_qweight_kernel<8, NC>), grid, dim3(kThreads), 0, stream,
+                         (const uint8_t*)codes, scales, qbias, gshift, gcols, q, s, N, K);
+    } else {
+      hipLaunchKernelGGL((i8_quantize_qweight_kernel<4, NC>), grid, dim3(kThreads), 0, stream,
+                         (const uint8_t*)codes, scales, qbias, gshift, gcols, q, s, N, K);
+    }
+  });
   return hipGetLastError();
 }
 
