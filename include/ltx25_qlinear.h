@@ -280,10 +280,14 @@ int ltx25_linear_route(int M, int K, int N, int bits, ltx25_route* out);
  * - rank < 96 with M >= 512, K % 64 == 0, rank % 8 == 0 and the vector
  *   path's conditions (below): r on the dense GEMM into that scratch, then
  *   the fused kernel's y pass reading it;
- * - otherwise one fused kernel per 512 adapter columns (16-byte aligned x,
- *   a and y with K % 8 == 0 and N % 8 == 0 take its vector path; when the
- *   rank is not a multiple of 8, b is first copied with its rows
- *   zero-padded to one).
+ * - otherwise the fused kernel, one launch per 512 adapter columns (16-byte
+ *   aligned x, a and y with K % 8 == 0 and N % 8 == 0 take its vector path;
+ *   when the rank is not a multiple of 8, b is first copied with its rows
+ *   zero-padded to one). On the vector path with K % 64 == 0 it leaves x . a^T
+ *   to a dense GEMM ahead of it (into the library's scratch) where K >= 1536 or
+ *   M >= 512, rank <= 512; and from rank 96 and K = 512 (N % 8 == 0) both
+ *   products run on the dense GEMM, in the pair's manner, below the pair's 256
+ *   tokens too.
  * `r` ([M][rank] bf16) and `d` ([M][N]) are the reference signature's
  * caller scratch; either may be NULL. A 16-byte aligned `r` receives
  * r = bf16(x . a^T) on the r-first route, and on the pair when rank is a
@@ -301,10 +305,11 @@ int ltx25_lora_add(void* stream, const void* x, const void* a, const void* b,
 #define LTX25_LORA_NONE 0
 #define LTX25_LORA_PAIR 1    /* two dense GEMMs, the second seeded from y */
 #define LTX25_LORA_RFIRST 2  /* r on the dense GEMM, then the fused y pass */
-#define LTX25_LORA_FUSED 3   /* one fused kernel per 512 adapter columns */
+#define LTX25_LORA_FUSED 3   /* the fused kernel and its plans (ltx25_lora_add); when
+                              * forced, always one launch per 512 adapter columns */
 
-/* 1 when ltx25_lora_add takes the GEMM pair for this shape (with
- * allocator-aligned pointers) under the current switches, else 0.
+/* 1 when ltx25_lora_add's route is the GEMM pair (LTX25_LORA_PAIR) for this
+ * shape (with allocator-aligned pointers) under the current switches, else 0.
  * Replaces MetalOps::lora_on_matrix_cores (src/ltx25-metal-ops.h:134-139;
  * src/ltx25-metal-ops.cc:921-936). Host-only. */
 int ltx25_lora_on_matrix_cores(int M, int K, int N, int rank);
@@ -344,8 +349,9 @@ int ltx25_lora_route(const void* x, const void* a, const void* b, const void* y,
  *   - otherwise as rank-rounded-to-64 more K: y = epi([x | r] . [W | B]^T
  *     + bias), r = bf16(x . A^T), one rounding of the output;
  * where the reference rounds the linear and the delta separately.
- * Elsewhere it runs ltx25_linear_q, ltx25_lora_add, then ltx25_gelu_tanh
- * for LTX25_EPI_GELU_TANH. a is bf16 [rank][K], b bf16 [N][rank];
+ * Elsewhere it gives the bits of ltx25_linear_q, ltx25_lora_add, then
+ * ltx25_gelu_tanh for LTX25_EPI_GELU_TANH (inside the adapter's last kernel
+ * where that kernel is the fused one). a is bf16 [rank][K], b bf16 [N][rank];
  * rank 0 is a plain linear. */
 int ltx25_linear_q_lora(void* stream, const void* x, const ltx25_qweight* w, const void* bias,
                         int bias_dtype, const void* a, const void* b, int rank, void* y, int M,

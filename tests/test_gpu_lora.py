@@ -169,6 +169,45 @@ def test_lora_is_deterministic(pkg, dev):
     assert np.array_equal(outs[0], outs[1])
 
 
+# the plans under the FUSED answer: r by the dense GEMM ahead of the y phase (from K = 1536),
+# both products on the dense GEMM (from rank 96 and K = 512), one pass below; at each line's
+# sides, ranks that are not multiples of 8 or 64, one token, ragged N
+PLANS = [  # M, K, N, rank
+    (128, 1536, 1032, 32), (128, 1472, 1032, 32), (1, 4096, 520, 5), (33, 2048, 8, 90),
+    (255, 2048, 4104, 17), (700, 512, 264, 6), (20, 1600, 512, 95), (255, 512, 264, 96),
+    (3, 512, 1000, 450), (255, 448, 264, 96), (70, 1600, 200, 512), (64, 1600, 200, 520),
+    (40, 1536, 1000, 1), (300, 1536, 96, 12),
+]
+
+
+@pytest.mark.parametrize("M,K,N,rank", PLANS)
+def test_fused_plans_against_oracle(pkg, dev, M, K, N, rank):
+    say(f"lora_add plan M={M} K={K} N={N} rank={rank}")
+    assert run_and_check(pkg, f"plan {M} {K} {N} {rank}", M, K, N, rank) == ROUTE[F]
+
+
+@pytest.mark.parametrize("M,K,N,rank", PLANS + [(45, 64, 30, 6)])
+def test_gelu_after_the_adapter_is_the_sequence(pkg, dev, M, K, N, rank):
+    """linear_q_lora where the fold does not take: the GELU inside the adapter's last kernel
+    gives the bits of linear_q, lora_add, gelu_tanh."""
+    from gpu_util import make_qweight, rng_normal
+    if pkg.lora_fold_takes(M, K, N, rank, 8):
+        pytest.skip("the fold takes it")
+    rng = np.random.default_rng(M + K + N + rank)
+    qw = make_qweight(pkg, rng_normal(rng, (N, K), 0.02), 8, 64)[0]
+    x, a, b, _ = draws(f"gelu {M} {K} {N} {rank}", M, K, N, rank)
+    xd, ad, bd = (dev_bf16(orc.bf16_rne(t * s)) for t, s in ((x, 1.0), (a, 0.1), (b, 0.1)))
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    seq = torch.empty_like(y)
+    say(f"linear_q_lora + GELU M={M} K={K} N={N} rank={rank}")
+    pkg.linear_q_lora(xd, qw, None, ad, bd, rank, y, M, K, N, pkg.EPI_GELU_TANH)
+    pkg.linear_q(xd, qw, None, seq, M, K, N)
+    pkg.lora_add(xd, ad, bd, seq, M, K, N, rank)
+    pkg.gelu_tanh(seq, seq)
+    torch.cuda.synchronize()
+    assert np.array_equal(host_bits(y), host_bits(seq))
+
+
 # the reference's caller scratch r ([M][rank]): the r-first route, and the GEMM pair at a
 # rank that is a multiple of 64, compute r into it instead of the library's scratch
 CALLER_R = [("r first: rank 40, ragged M", 777, 1024, 2048, 40, RF),

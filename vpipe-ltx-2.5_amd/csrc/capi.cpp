@@ -517,11 +517,10 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
 {
   const int rk = (rank + 63) & ~63;
   // A's rows past `rank` read as zeros (the GEMM's weight-row bound), so A
-  // is copied only when it is not 16-byte aligned or the r GEMM plans the
-  // M <= 128 kernel, which takes whole weights only; B gets zero columns up
+  // is copied only when it is not 16-byte aligned; B gets zero columns up
   // to rk. The caller's r ([M][rank]) holds r when it has rk columns.
   const ltx25::GemmPlan r_plan = ltx25::plan_gemm(M, rk, K, 16, ds->cu_count);
-  const bool pad_a = !aligned16(a) || (rk != rank && r_plan.tile == 2);
+  const bool pad_a = !aligned16(a);
   const bool pad_b = rk != rank || !aligned16(b);
   const bool own_r = r_caller == nullptr || rk != rank || !aligned16(r_caller);
   const size_t a_bytes = pad_a ? align256((size_t)rk * K * 2) : 0;
@@ -585,6 +584,119 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
     if (e != hipSuccess) { return hip_fail(e, "lora gemm launch"); }
   }
   return LTX25_OK;
+}
+
+// FUSED's two other plans under AUTO (a forced FUSED is always the one-pass
+// kernel). That kernel computes r = x . A^T once per row block and column split,
+// from 16-byte loads of 32 rows each, so its time grows with K and, past rank 32
+// or so, with the rank. From kLoraAheadMinK of K r comes from the dense GEMM, as
+// on the r-first route, and the kernel runs its y phase: rank 32, 128 x 4096 ->
+// 16384 22.8 us in one pass, 15.6 so; rank 40, 24 x 15360 -> 13264 79.5 and
+// 16.1; 246 x 2816 -> 208, rank 24 14.0 and 9.6 (at K = 1024, 9 tokens, 8.9 and
+// 10.7). From rank kLoraPairMinRank and kLoraWideMinK both products run on the
+// dense GEMM, as in the pair: rank 448, 64 x 1024 -> 1024 67.5 us in one pass,
+// 10.4 so; rank 128, 128 x 4096 -> 4096 66.5 and 14.5; rank 200, 126 x 8192 ->
+// 2048 189 and 22.5.
+constexpr int kLoraAheadMinK = 1536;
+constexpr int kLoraWideMinK = 512;
+
+// ltx25_lora_add; with `gelu`, y = bf16(gelu(bf16(y + delta))) as a GELU pass
+// after it would leave y, inside the y phase where that is the last to write y.
+int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* y, void* r, int M,
+             int K, int N, int rank, bool gelu)
+{
+  // The reference returns without encoding anything for an empty shape
+  // (src/ltx25-metal-ops.cc:996).
+  if (M <= 0 || K <= 0 || N <= 0 || rank <= 0) { return LTX25_OK; }
+  if (x == nullptr || a == nullptr || b == nullptr || y == nullptr) {
+    return fail(LTX25_E_INVAL, "x, a, b or y is null");
+  }
+  if ((((uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)y) & 1u) != 0) {
+    return fail(LTX25_E_INVAL, "a bf16 tensor is not 2-byte aligned");
+  }
+  const int route = lora_route(M, K, N, rank, x, a, y);
+  if (route < 0) { return LTX25_E_UNSUPPORTED; }
+  DeviceState* ds = nullptr;
+  const int rc = current_device(&ds);
+  if (rc != LTX25_OK) { return rc; }
+  auto gelu_pass = [&]() { return gelu ? ltx25_gelu_tanh(st, y, y, (size_t)M * N) : LTX25_OK; };
+  const int rank8 = (rank + 7) & ~7;
+  const bool vec = lora_vec_ok(M, K, N, rank, x, a, y);
+  const bool planned =
+      route == LTX25_LORA_FUSED &&
+      g_lora_force.load(std::memory_order_relaxed) == LTX25_LORA_AUTO && vec && K % 64 == 0;
+  const bool wide = planned && rank >= kLoraPairMinRank && K >= kLoraWideMinK &&
+                    lora_pair_ok(M, K, N, rank, x, y);
+  if (route == LTX25_LORA_PAIR || wide) {
+    const int rc2 = lora_pair(ds, st, x, a, b, y, wide ? nullptr : r, M, K, N, rank);
+    return rc2 != LTX25_OK ? rc2 : gelu_pass();
+  }
+  const bool ahead = route == LTX25_LORA_RFIRST ||
+                     (planned && rank <= ltx25::kLoraMaxRank && below_limit((size_t)M * rank8 * 2) &&
+                      (K >= kLoraAheadMinK || M >= kLoraRFirstMinM));
+  const uint16_t* pa = (const uint16_t*)a;
+  const uint16_t* pb = (const uint16_t*)b;
+  int ldb = rank;
+  if (vec && (rank != rank8 || !aligned16(b))) {
+    {
+      std::lock_guard<std::mutex> lk(g_mu);
+      const int rc2 = grow(&ds->lora_b, &ds->lora_b_bytes, (size_t)N * rank8 * 2);
+      if (rc2 != LTX25_OK) { return rc2; }
+    }
+    const hipError_t e = ltx25::launch_lora_pad(pb, N, rank, rank, (uint16_t*)ds->lora_b, rank8,
+                                                st);
+    if (e != hipSuccess) { return hip_fail(e, "lora pad launch"); }
+    pb = (const uint16_t*)ds->lora_b;
+    ldb = rank8;
+  }
+  if (ahead) {
+    // r = bf16(x . A^T) once with the dense GEMM (A is the [rank][K] weight of
+    // that linear, zero rows up to rank8), then the fused kernel's second
+    // phase reads it -- instead of recomputing x . A^T for every column
+    // split of a row block. Same roundings (r rounded once to bf16).
+    // r goes to the caller's buffer on the r-first route when it has one
+    // ([M][rank], 16-byte aligned), else to the library's scratch
+    uint16_t* rb = route == LTX25_LORA_RFIRST ? (uint16_t*)r : nullptr;
+    if (rb == nullptr || !aligned16(rb)) {
+      std::lock_guard<std::mutex> lk(g_mu);
+      const int rc2 = grow(&ds->lora_mm, &ds->lora_mm_bytes, (size_t)M * rank8 * 2);
+      if (rc2 != LTX25_OK) { return rc2; }
+      rb = (uint16_t*)ds->lora_mm;
+    }
+    ltx25::GemmDesc gd;
+    gd.x = (const uint16_t*)x;
+    gd.w = pa;
+    gd.bits = 16;
+    gd.group = 64;
+    gd.y = rb;
+    gd.M = M;
+    gd.N = rank8;
+    gd.wn = rank;
+    gd.K = K;
+    const ltx25::GemmPlan plan = ltx25::plan_gemm(M, rank8, K, 16, ds->cu_count);
+    float* ws = nullptr;
+    if (plan.workspace_bytes > 0) {
+      std::lock_guard<std::mutex> lk(g_mu);
+      const int rc2 = grow(&ds->ws, &ds->ws_bytes, plan.workspace_bytes);
+      if (rc2 != LTX25_OK) { return rc2; }
+      ws = (float*)ds->ws;
+    }
+    hipError_t e = ltx25::launch_gemm(gd, plan, ws, st);
+    if (e != hipSuccess) { return hip_fail(e, "lora r gemm launch"); }
+    e = ltx25::launch_lora((const uint16_t*)x, pa, pb, (uint16_t*)y, M, K, N, rank8, ldb, vec,
+                           ds->cu_count, st, rb, gelu);
+    if (e != hipSuccess) { return hip_fail(e, "lora launch"); }
+    return LTX25_OK;
+  }
+  for (int c = 0; c < rank; c += ltx25::kLoraMaxRank) {
+    const bool last = c + ltx25::kLoraMaxRank >= rank;
+    const int rp = last ? rank - c : ltx25::kLoraMaxRank;
+    const hipError_t e = ltx25::launch_lora((const uint16_t*)x, pa + (size_t)c * K, pb + c,
+                                            (uint16_t*)y, M, K, N, rp, ldb, vec, ds->cu_count, st,
+                                            nullptr, gelu && vec && last);
+    if (e != hipSuccess) { return hip_fail(e, "lora launch"); }
+  }
+  return vec ? LTX25_OK : gelu_pass();
 }
 
 // The LoRA fold: the adapter rides inside the linear's own GEMM as extra K,
@@ -712,8 +824,8 @@ int run_fold(DeviceState* ds, hipStream_t st, const FoldPlan& f, const void* x,
   const int kt = K + rk;
   // A [rank][K] is read as an [rk][K] weight whose rows past `rank` are
   // zeros (the buffer range stops at A's end); copied with zero rows only
-  // when it is not 16-byte aligned or the r GEMM plans the M <= 128 kernel
-  const bool pad_a = !aligned16(a) || f.r_plan.tile == 2;
+  // when it is not 16-byte aligned
+  const bool pad_a = !aligned16(a);
   const size_t a_bytes = pad_a ? align256((size_t)rk * K * 2) : 0;
   const size_t r_bytes = align256((size_t)M * rk * 2);
   uint16_t* wd = nullptr;
@@ -1003,86 +1115,7 @@ int ltx25_lora_add(void* stream, const void* x, const void* a, const void* b,
                    void* y, void* r, void* d, int M, int K, int N, int rank)
 {
   (void)d;
-  // The reference returns without encoding anything for an empty shape
-  // (src/ltx25-metal-ops.cc:996).
-  if (M <= 0 || K <= 0 || N <= 0 || rank <= 0) { return LTX25_OK; }
-  if (x == nullptr || a == nullptr || b == nullptr || y == nullptr) {
-    return fail(LTX25_E_INVAL, "x, a, b or y is null");
-  }
-  if ((((uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)y) & 1u) != 0) {
-    return fail(LTX25_E_INVAL, "a bf16 tensor is not 2-byte aligned");
-  }
-  const int route = lora_route(M, K, N, rank, x, a, y);
-  if (route < 0) { return LTX25_E_UNSUPPORTED; }
-  DeviceState* ds = nullptr;
-  const int rc = current_device(&ds);
-  if (rc != LTX25_OK) { return rc; }
-  if (route == LTX25_LORA_PAIR) {
-    return lora_pair(ds, (hipStream_t)stream, x, a, b, y, r, M, K, N, rank);
-  }
-  const int rank8 = (rank + 7) & ~7;
-  const bool vec = lora_vec_ok(M, K, N, rank, x, a, y);
-  const uint16_t* pa = (const uint16_t*)a;
-  const uint16_t* pb = (const uint16_t*)b;
-  int ldb = rank;
-  if (vec && (rank != rank8 || !aligned16(b))) {
-    {
-      std::lock_guard<std::mutex> lk(g_mu);
-      const int rc2 = grow(&ds->lora_b, &ds->lora_b_bytes, (size_t)N * rank8 * 2);
-      if (rc2 != LTX25_OK) { return rc2; }
-    }
-    const hipError_t e = ltx25::launch_lora_pad(pb, N, rank, rank, (uint16_t*)ds->lora_b, rank8,
-                                                (hipStream_t)stream);
-    if (e != hipSuccess) { return hip_fail(e, "lora pad launch"); }
-    pb = (const uint16_t*)ds->lora_b;
-    ldb = rank8;
-  }
-  if (route == LTX25_LORA_RFIRST) {
-    // Many tokens: r = bf16(x . A^T) once with the dense GEMM (A is the
-    // [rank][K] weight of that linear), then the fused kernel's second
-    // phase reads it -- instead of recomputing x . A^T for every column
-    // split of a row block. Same roundings (r rounded once to bf16).
-    // r goes to the caller's buffer when it has one ([M][rank], 16-byte
-    // aligned), else to the library's scratch
-    uint16_t* rb = (uint16_t*)r;
-    if (rb == nullptr || !aligned16(rb)) {
-      std::lock_guard<std::mutex> lk(g_mu);
-      const int rc2 = grow(&ds->lora_mm, &ds->lora_mm_bytes, (size_t)M * rank * 2);
-      if (rc2 != LTX25_OK) { return rc2; }
-      rb = (uint16_t*)ds->lora_mm;
-    }
-    ltx25::GemmDesc gd;
-    gd.x = (const uint16_t*)x;
-    gd.w = pa;
-    gd.bits = 16;
-    gd.group = 64;
-    gd.y = rb;
-    gd.M = M;
-    gd.N = rank;
-    gd.K = K;
-    const ltx25::GemmPlan plan = ltx25::plan_gemm(M, rank, K, 16, ds->cu_count);
-    float* ws = nullptr;
-    if (plan.workspace_bytes > 0) {
-      std::lock_guard<std::mutex> lk(g_mu);
-      const int rc2 = grow(&ds->ws, &ds->ws_bytes, plan.workspace_bytes);
-      if (rc2 != LTX25_OK) { return rc2; }
-      ws = (float*)ds->ws;
-    }
-    hipError_t e = ltx25::launch_gemm(gd, plan, ws, (hipStream_t)stream);
-    if (e != hipSuccess) { return hip_fail(e, "lora r gemm launch"); }
-    e = ltx25::launch_lora((const uint16_t*)x, pa, pb, (uint16_t*)y, M, K, N, rank, ldb, vec,
-                           ds->cu_count, (hipStream_t)stream, rb);
-    if (e != hipSuccess) { return hip_fail(e, "lora launch"); }
-    return LTX25_OK;
-  }
-  for (int c = 0; c < rank; c += ltx25::kLoraMaxRank) {
-    const int rp = rank - c < ltx25::kLoraMaxRank ? rank - c : ltx25::kLoraMaxRank;
-    const hipError_t e = ltx25::launch_lora((const uint16_t*)x, pa + (size_t)c * K, pb + c,
-                                            (uint16_t*)y, M, K, N, rp, ldb, vec,
-                                            ds->cu_count, (hipStream_t)stream);
-    if (e != hipSuccess) { return hip_fail(e, "lora launch"); }
-  }
-  return LTX25_OK;
+  return run_lora((hipStream_t)stream, x, a, b, y, r, M, K, N, rank, false);
 }
 
 int ltx25_lora_fold_takes(int M, int K, int N, int rank, int bits)
@@ -1135,10 +1168,7 @@ int ltx25_linear_q_lora(void* stream, const void* x, const ltx25_qweight* w, con
   // GELU (src/ltx25-block-metal.cc:639-645).
   int rc = run_linear(st, x, w, bias, bias_dtype, y, M, K, N, LTX25_EPI_NONE);
   if (rc != LTX25_OK) { return rc; }
-  rc = ltx25_lora_add(stream, x, a, b, y, nullptr, nullptr, M, K, N, rank);
-  if (rc != LTX25_OK) { return rc; }
-  if (epilogue == LTX25_EPI_GELU_TANH) { return ltx25_gelu_tanh(stream, y, y, (size_t)M * N); }
-  return LTX25_OK;
+  return run_lora(st, x, a, b, y, nullptr, M, K, N, rank, epilogue == LTX25_EPI_GELU_TANH);
 }
 
 int ltx25_probe_read(void* stream, const void* src, size_t bytes, void* sink, int blocks)

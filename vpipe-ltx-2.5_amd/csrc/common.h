@@ -100,9 +100,9 @@ struct GemmDesc {
   // [kx, K) are x2 [M][K - kx]; kx a multiple of 64. Null x2: X = x [M][K].
   const uint16_t* x2 = nullptr;
   int kx = 0;
-  // Rows of the weight present in memory (0: all N); rows past it read as
-  // zeros (the 256 x 256 and 128 x 128 tiles). The fold's r GEMM reads A
-  // [rank][K] as a [rk][K] weight this way.
+  // Rows of a dense weight present in memory (0: all N); rows past it read as
+  // zeros. The LoRA routes' r GEMMs read A [rank][K] as a [rk][K] weight this
+  // way.
   int wn = 0;
   const void* w = nullptr;          // u8/u32 codes, or bf16 dense
   const uint16_t* scales = nullptr;
@@ -198,13 +198,14 @@ hipError_t launch_splitk_reduce(const float* partial, int splits, const void* bi
 // aligned pointers, every operand under 2 GiB, and B's columns zero from
 // `rank` up to the next multiple of 8).
 // With `r_in` set ([M][rank] bf16, rank % 8 == 0, vector path only) the
-// launch skips the x . A^T phase and reads r from it.
+// launch skips the x . A^T phase and reads r from it. `gelu` (vector path):
+// y = bf16(gelu(bf16(y + delta))), the bits of a GELU pass after the launch.
 constexpr int kLoraMaxRank = 512;
 int lora_splits(int M, int N, int rank, int cu_count, bool pre_r);
 hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
                        uint16_t* y, int M, int K, int N, int rank, int ldb,
                        bool vec, int cu_count, hipStream_t stream,
-                       const uint16_t* r_in = nullptr);
+                       const uint16_t* r_in = nullptr, bool gelu = false);
 // B [rows][cols] (row stride ld_src) -> `width` columns of each dst row
 // (row stride ld_dst; width 0 = ld_dst) with zeros past `cols`: the vector
 // path's copy of an adapter whose rank is not a multiple of 8, and the

@@ -99,8 +99,9 @@ __device__ __forceinline__ bf16x8 frag8s(const uint16_t* p, int row, int rows, i
 }
 
 // RB = 32-column blocks of rank this instance covers (rank <= 32 * RB);
-// PRE_R: r comes from p.r_in instead of phase 1.
-template <int RB, bool VEC, bool PRE_R>
+// PRE_R: r comes from p.r_in instead of phase 1. GELU (vector path): y is
+// GELU-tanh of the rounded sum.
+template <int RB, bool VEC, bool PRE_R, bool GELU>
 __global__ __launch_bounds__(kLoraThreads) void lora_kernel(LoraParams p)
 {
   constexpr int RP = 32 * RB;        // rank padded to the MFMA block
@@ -330,6 +331,12 @@ __global__ __launch_bounds__(kLoraThreads) void lora_kernel(LoraParams p)
             u32x2 o;
             o.x = pack_bf16x2(c[4 * g + 0], c[4 * g + 1]);
             o.y = pack_bf16x2(c[4 * g + 2], c[4 * g + 3]);
+            if constexpr (GELU) {
+              o.x = pack_bf16x2(gelu_tanh(__uint_as_float(o.x << 16)),
+                                gelu_tanh(__uint_as_float(o.x & 0xffff0000u)));
+              o.y = pack_bf16x2(gelu_tanh(__uint_as_float(o.y << 16)),
+                                gelu_tanh(__uint_as_float(o.y & 0xffff0000u)));
+            }
             *(u32x2*)(yt + g * 8) = o;
           }
         }
@@ -373,14 +380,16 @@ __global__ __launch_bounds__(kLoraThreads) void lora_kernel(LoraParams p)
 }
 
 template <int RB>
-hipError_t launch_rb(const LoraParams& p, bool vec, dim3 grid, hipStream_t stream)
+hipError_t launch_rb(const LoraParams& p, bool vec, bool gelu, dim3 grid, hipStream_t stream)
 {
   if (p.r_in != nullptr) {
-    lora_kernel<RB, true, true><<<grid, kLoraThreads, 0, stream>>>(p);
+    gelu ? lora_kernel<RB, true, true, true><<<grid, kLoraThreads, 0, stream>>>(p)
+         : lora_kernel<RB, true, true, false><<<grid, kLoraThreads, 0, stream>>>(p);
   } else if (vec) {
-    lora_kernel<RB, true, false><<<grid, kLoraThreads, 0, stream>>>(p);
+    gelu ? lora_kernel<RB, true, false, true><<<grid, kLoraThreads, 0, stream>>>(p)
+         : lora_kernel<RB, true, false, false><<<grid, kLoraThreads, 0, stream>>>(p);
   } else {
-    lora_kernel<RB, false, false><<<grid, kLoraThreads, 0, stream>>>(p);
+    lora_kernel<RB, false, false, false><<<grid, kLoraThreads, 0, stream>>>(p);
   }
   return hipGetLastError();
 }
@@ -654,22 +663,25 @@ hipError_t launch_lora_pad(const uint16_t* src, int rows, int cols, int ld_src, 
 // block (x and all of A again), so a wide adapter gets just enough
 // workgroups to cover the CUs once; a narrow one, whose phase 2 is bound by
 // y traffic and wants waves in flight, gets two per CU. Never fewer than
-// 1024 columns per workgroup.
+// 1024 columns per workgroup, or the 512 of one super-block stride where r is
+// given and nothing is recomputed.
 int lora_splits(int M, int N, int rank, int cu_count, bool pre_r)
 {
   const int mtiles = (M + kLoraRows - 1) / kLoraRows;
   const int per_cu = rank > 128 && !pre_r ? 1 : 2;
   const int want = per_cu * cu_count / mtiles;
-  const int cap = (N + 1023) / 1024;
+  const int cap = pre_r ? (N + 511) / 512 : (N + 1023) / 1024;
   return want < 1 ? 1 : (want < cap ? want : cap);
 }
 
 hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
                        uint16_t* y, int M, int K, int N, int rank, int ldb,
-                       bool vec, int cu_count, hipStream_t stream, const uint16_t* r_in)
+                       bool vec, int cu_count, hipStream_t stream, const uint16_t* r_in,
+                       bool gelu)
 {
   if (rank <= 0 || rank > kLoraMaxRank) { return hipErrorInvalidValue; }
   if (r_in != nullptr && (!vec || rank % 8 != 0)) { return hipErrorInvalidValue; }
+  if (gelu && !vec) { return hipErrorInvalidValue; }
   const int splits = lora_splits(M, N, rank, cu_count, r_in != nullptr);
   int n_split = (N + splits - 1) / splits;
   // whole super-block strides (4 waves x 128 columns) where N allows
@@ -679,11 +691,11 @@ hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
   LoraParams p{r_in, x, a, b, y, M, K, N, rank, ldb, n_split};
   const dim3 grid((unsigned)((M + kLoraRows - 1) / kLoraRows), (unsigned)gy);
   const int rb = (rank + 31) / 32;
-  if (rb <= 1) { return launch_rb<1>(p, vec, grid, stream); }
-  if (rb <= 2) { return launch_rb<2>(p, vec, grid, stream); }
-  if (rb <= 4) { return launch_rb<4>(p, vec, grid, stream); }
-  if (rb <= 8) { return launch_rb<8>(p, vec, grid, stream); }
-  return launch_rb<16>(p, vec, grid, stream);
+  if (rb <= 1) { return launch_rb<1>(p, vec, gelu, grid, stream); }
+  if (rb <= 2) { return launch_rb<2>(p, vec, gelu, grid, stream); }
+  if (rb <= 4) { return launch_rb<4>(p, vec, gelu, grid, stream); }
+  if (rb <= 8) { return launch_rb<8>(p, vec, gelu, grid, stream); }
+  return launch_rb<16>(p, vec, gelu, grid, stream);
 }
 
 }  // namespace ltx25

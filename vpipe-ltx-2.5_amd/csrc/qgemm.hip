@@ -915,8 +915,8 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
       (plan.tile == 2 || d.bits != 16 || d.kx <= 0 || d.kx >= d.K || d.kx % kBK != 0)) {
     return hipErrorInvalidValue;   // the two-part activation: dense weights, MFMA tiles
   }
-  if (plan.tile == 2 && d.wn > 0 && d.wn < d.N) {
-    return hipErrorInvalidValue;   // the M <= 128 kernel reads all N weight rows
+  if (d.wn > 0 && d.wn < d.N && d.bits != 16) {
+    return hipErrorInvalidValue;   // a weight with fewer rows than N: dense only
   }
   if (plan.tile == 2) { return launch_skinny(d, plan, workspace, stream); }
   if (plan.panel_rows > 0 && d.x2 == nullptr) { return launch_panel(d, plan, workspace, stream); }

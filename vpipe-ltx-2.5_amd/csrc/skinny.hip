@@ -74,6 +74,7 @@ struct SParams {
   uint16_t* y;
   float* partial;           // [splits][M][N] when split
   int M, N, K;
+  int wn;                   // weight rows in memory; rows past them read as zeros
   int gshift, gcols;
   int k_chunk;              // K per workgroup (multiple of 64)
   int bias_type, epilogue;
@@ -190,7 +191,7 @@ skinny_kernel(SParams p)
 
   const size_t wrow_bytes = (size_t)p.K * BITS / 8;   // bits 16: bf16 rows
   const __amdgpu_buffer_rsrc_t xr = rsrc(p.x, (size_t)p.M * p.K * 2);
-  const __amdgpu_buffer_rsrc_t wr = rsrc(p.wq, (size_t)p.N * wrow_bytes);
+  const __amdgpu_buffer_rsrc_t wr = rsrc(p.wq, (size_t)p.wn * wrow_bytes);
   const __amdgpu_buffer_rsrc_t sr = rsrc(p.scales, (size_t)p.N * p.gcols * 2);
   const __amdgpu_buffer_rsrc_t qr = rsrc(p.qbias, (size_t)p.N * p.gcols * 2);
 
@@ -630,6 +631,7 @@ hipError_t launch_skinny(const GemmDesc& d, const GemmPlan& plan, float* workspa
   p.M = d.M;
   p.N = d.N;
   p.K = d.K;
+  p.wn = d.bits == 16 && d.wn > 0 && d.wn < d.N ? d.wn : d.N;
   int gs = 0;
   while ((1 << gs) < d.group) { ++gs; }
   p.gshift = d.bits == 16 ? 0 : gs;
