@@ -99,3 +99,89 @@ def test_row_slabs_past_2gib(pkg, quantized):
     got = host_f32(y)[rows]
     assert orc.max_rel(got, ref) <= 1e-2
     assert orc.rel_l2(got, ref) < 3e-3
+
+
+# where the planner leaves the 128 x 128 tile with one K split for larger ones: 128 x 256 tiles
+# (dense weights) and 256 x 256 tiles that do not fill the CUs; 1, 2, 3 and many K steps, ragged
+# M and N
+LARGER = [  # M, K, N, tile
+    (1024, 64, 8192, 2), (300, 128, 16392, 2), (897, 192, 8008, 2), (1000, 1088, 8192, 2),
+    (257, 320, 16000, 2), (700, 64, 16384, 1), (900, 128, 12296, 1), (641, 960, 13000, 1),
+]
+
+
+@pytest.mark.parametrize("M,K,N,tile", LARGER)
+@pytest.mark.parametrize("bias,epi", [("f32", 0), ("bf16", 1), (None, 1)])
+def test_larger_tiles_give_the_same_bits(pkg, M, K, N, tile, bias, epi):
+    """AUTO's choice against the forced 128 x 128 and 256 x 256 tiles: the same sums in the same
+    K order, so the same bits; dense, w8 and w4."""
+    rng = np.random.default_rng(M + K + N)
+    x = dev_bf16(orc.bf16_rne(rng_normal(rng, (M, K))))
+    b = None if bias is None else rng_normal(rng, (N,), 0.05)
+    bd = None if b is None else dev_f32(b) if bias == "f32" else dev_bf16(orc.bf16_rne(b))
+    for bits, group in ((16, 64), (8, 64), (4, 32)):
+        w = rng_normal(rng, (N, K), 0.05)
+        if bits == 16:
+            keep = dev_bf16(orc.bf16_rne(w))
+            cw = pkg.dense_weight(keep)
+        else:
+            qw = make_qweight(pkg, w, bits, group)[0]
+            cw = qw.c()
+        assert pkg.linear_route(M, K, N, bits)["tile"] == tile
+        outs = []
+        for force in (pkg.TILE_AUTO, pkg.TILE_MID, pkg.TILE_TALL):
+            pkg.set_tile(force)
+            y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+            say(f"larger tiles {M}x{K}->{N} w{bits} bias={bias} epi={epi} forced={force} "
+                f"route={pkg.linear_route(M, K, N, bits)}")
+            pkg.linear_qc(x, cw, bd, y, M, K, N, epi)
+            torch.cuda.synchronize()
+            outs.append(host_bits(y))
+        pkg.set_tile(pkg.TILE_AUTO)
+        assert np.array_equal(outs[0], outs[1])
+        assert np.array_equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("M,K,N", [(1024, 128, 8192), (300, 256, 16392), (1000, 1152, 8200),
+                                   (1500, 384, 9000)])
+def test_larger_int8_tiles_are_exact(pkg, M, K, N):
+    """int8 on 128 x 256 tiles and on 256 x 256 tiles that do not fill the CUs: int32 accumulators
+    and bf16 outputs exact."""
+    rng = np.random.default_rng(M + K)
+    xq = torch.from_numpy(rng.integers(-127, 128, (M, K), dtype=np.int8)).cuda()
+    wq = torch.from_numpy(rng.integers(-127, 128, (N, K), dtype=np.int8)).cuda()
+    sx = torch.from_numpy(rng.random(M, dtype=np.float32) * 0.01).cuda()
+    sw = torch.from_numpy(rng.random(N, dtype=np.float32) * 0.01).cuda()
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    acc = torch.empty((M, N), dtype=torch.int32, device="cuda")
+    say(f"larger int8 tiles {M}x{K}->{N}")
+    pkg.i8_gemm(xq, sx, wq, sw, None, y, acc, M, K, N)
+    torch.cuda.synchronize()
+    exact = (xq.double() @ wq.double().t())
+    assert torch.equal(acc.double(), exact)
+    want = acc.float() * (sx[:, None] * sw[None, :])
+    assert torch.equal(y, want.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rank", [100, 192])
+def test_larger_tiles_under_the_lora_pair(pkg, rank):
+    """The pair's second GEMM, accumulators seeded from y, and the fold's two-part activation on
+    128 x 256 tiles: the bits of the forced 256 x 256 tile."""
+    M, K, N = 1024, 256, 8192
+    rng = np.random.default_rng(rank)
+    x, a, b = (dev_bf16(orc.bf16_rne(rng_normal(rng, s, 0.1))) for s in ((M, K), (rank, K), (N, rank)))
+    y0 = dev_bf16(orc.bf16_rne(rng_normal(rng, (M, N))))
+    qw = make_qweight(pkg, rng_normal(rng, (N, K), 0.05), 8, 64)[0]
+    assert pkg.lora_on_matrix_cores(M, K, N, rank) and pkg.lora_fold_takes(M, K, N, rank, 8)
+    outs = []
+    for force in (pkg.TILE_AUTO, pkg.TILE_TALL):
+        pkg.set_tile(force)
+        y = y0.clone()
+        say(f"larger tiles under the LoRA pair, rank {rank}, forced={force}")
+        pkg.lora_add(x, a, b, y, M, K, N, rank)
+        f = torch.empty_like(y)
+        pkg.linear_q_lora(x, qw, None, a, b, rank, f, M, K, N, pkg.EPI_GELU_TANH)
+        torch.cuda.synchronize()
+        outs.append((host_bits(y), host_bits(f)))
+    assert np.array_equal(outs[0][0], outs[1][0])
+    assert np.array_equal(outs[0][1], outs[1][1])

@@ -127,6 +127,8 @@ struct GemmPlan {
   // K between its waves; 0 for the 128 x 128 tile
   int panel_rows = 0;
   int panel_cols = 0;
+  // tile 1 only: a dense weight runs on 128 x 256 tiles of the 256 x 256 kernel
+  bool half_tall = false;
   int cu_count = 256;           // CUs of the device planned for (persistent grids)
 };
 
@@ -139,6 +141,10 @@ GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force = 0,
                    bool panels = true);
 hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
                        float* workspace, hipStream_t stream);
+// Rows of the ping-pong kernel's tile that an unsplit GEMM is best served by:
+// 256, 128, or 0 where the 128 x 128 tile is (dense weights and int8 operands;
+// codes, dequantized in registers, have no 128-row one).
+int tall_rows(int M, int N, int cu_count);
 // The M <= 128 route (skinny.hip): 32 output columns per workgroup, K split
 // between its 8 waves, and across workgroups above 2048. Fills `plan` and
 // returns true when it takes the shape (up to 3 workgroups per CU);
@@ -169,16 +175,17 @@ bool tall_dense_takes(const GemmDesc& d, const GemmPlan& plan);
 bool tall_w8_takes(const GemmDesc& d, const GemmPlan& plan);
 // `stamps` non-null (bf16 without the two-part activation, or the int8
 // launcher below): the phase-stamp instantiation, eight words per wave at
-// (tile * 8 + wave) * 8 (ltx25_probe_tall_phases)
-hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream,
+// (tile * 8 + wave) * 8 (ltx25_probe_tall_phases). `bm`: rows of the tile, 256, or
+// 128 for a dense weight (plan.half_tall).
+hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm = 256,
                              unsigned long long* stamps = nullptr);
 // The int8 tier's GEMM on the same tile (tall.hip, v_mfma_i32_16x16x64_i8):
-// N % 8 == 0, K a multiple of 128. launch_i8_gemm routes there when the
-// 256 x 256 tiles fill the GPU and it takes the shape.
+// N % 8 == 0, K a multiple of 128. launch_i8_gemm routes there, with 256- or
+// 128-row tiles, where tall_rows says so and it takes the shape.
 bool tall_i8_takes(int M, int N, int K);
 hipError_t launch_tall_i8(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
                           const void* bias, int bias_type, int epilogue, uint16_t* y,
-                          int32_t* acc, int M, int K, int N, hipStream_t stream,
+                          int32_t* acc, int M, int K, int N, hipStream_t stream, int bm = 256,
                           unsigned long long* stamps = nullptr);
 // The no-allocation linear's split-K scratch (noalloc.hip): a fixed device
 // array of kNoAllocScratchBytes per GPU. noalloc_scratch() returns the

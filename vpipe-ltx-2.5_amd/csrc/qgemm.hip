@@ -832,7 +832,9 @@ GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force, bool 
   const long tall_tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
   // a forced M <= 128 kernel that cannot take the shape leaves the choice
   // to the planner
-  if (force == 1 || ((force == 0 || force == 3) && M > 128 && tall_tiles >= cu_count)) {
+  const bool plans = force == 0 || force == 3;
+  const int rows = plans && M > 128 && N % 8 == 0 ? tall_rows(M, N, cu_count) : 0;
+  if (force == 1 || rows == 256 || (plans && M > 128 && tall_tiles >= cu_count)) {
     plan.tile = 0;
     plan.splits = 1;
     plan.k_chunk = K;
@@ -854,7 +856,27 @@ GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force, bool 
   plan.splits = s;
   plan.k_chunk = chunk;
   plan.workspace_bytes = s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+  plan.half_tall = rows == 128 && s == 1;
   return plan;
+}
+
+// The 256 x 256 tiles while they fill the CUs. Fewer of them still beat the 128 x
+// 128 tile once that needs more than the two workgroups per CU it runs at a
+// time, since every output then moves twice the operand bytes from L2: 700 x 4096
+// -> 16384 (192 tiles of 256 x 256) dense 88 against 122 us, w8 96 and 135, w4 102
+// and 131; int8 3000 x 4096 -> 4096 47 and 58. Below that, where the 128 x 128
+// tiles need the second workgroup, 128 x 256 tiles in one round: 1024 x 4096 -> 8192
+// dense 63 against 75 us (256 x 256: 77), 300 x 4096 -> 16384 60 and 69, int8 1024 x
+// 4096 -> 8192 35 and 41. With one workgroup per CU the 128 x 128 tile is ahead:
+// 8160 x 4096 -> 512 41 against 51, as are 256 x 256 tiles past one round of 128 x
+// 256 ones: 2040 x 4096 -> 8192 100 against 123.
+int tall_rows(int M, int N, int cu_count)
+{
+  const long mid = (long)((M + 127) / 128) * ((N + 127) / 128);
+  const long half = (long)((M + 127) / 128) * ((N + 255) / 256);
+  const long tall = (long)((M + 255) / 256) * ((N + 255) / 256);
+  if (tall >= cu_count || mid > 2L * cu_count) { return 256; }
+  return mid > cu_count && half <= cu_count ? 128 : 0;
 }
 
 hipError_t launch_i8_gemm(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
@@ -882,10 +904,12 @@ hipError_t launch_i8_gemm(const int8_t* xq, const float* sx, const int8_t* wq, c
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
     cus = 256;
   }
-  // the tall tile when it fills the GPU, else 128 x 128
+  // the tall tile when it fills the GPU or serves it better, else 128 x 128
   const bool fills = (long)((M + 255) / 256) * ((N + 255) / 256) >= cus;
-  if (fills && tall_i8_takes(M, N, K)) {
-    return launch_tall_i8(xq, sx, wq, sw, bias, kp.bias_type, epilogue, y, acc, M, K, N, stream);
+  const int rows = tall_rows(M, N, cus);
+  if (rows > 0 && tall_i8_takes(M, N, K)) {
+    return launch_tall_i8(xq, sx, wq, sw, bias, kp.bias_type, epilogue, y, acc, M, K, N, stream,
+                          rows);
   }
   if (fills) {
     kp.tiles_m = (M + 255) / 256;
@@ -920,7 +944,9 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
   }
   if (plan.tile == 2) { return launch_skinny(d, plan, workspace, stream); }
   if (plan.panel_rows > 0 && d.x2 == nullptr) { return launch_panel(d, plan, workspace, stream); }
-  if (tall_dense_takes(d, plan) || tall_w8_takes(d, plan)) { return launch_tall_dense(d, stream); }
+  if (tall_dense_takes(d, plan) || tall_w8_takes(d, plan)) {
+    return launch_tall_dense(d, stream, plan.half_tall ? 128 : 256);
+  }
   KParams kp = {};
   kp.x = d.x;
   kp.x2 = d.x2;

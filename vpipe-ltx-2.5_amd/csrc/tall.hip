@@ -137,12 +137,13 @@ __device__ __forceinline__ void unroll(F&& f)
 // tiles a round of workgroups finishes together then store scattered
 // 512-byte segments of each output row, not runs of adjacent ones (1.9%
 // faster on the 8160 x 4096 -> 16384 GEMM, 0.5% on 16384 -> 4096).
+template <int BM>
 __device__ __forceinline__ void tile_of(const TallParams& p, int& m0, int& n0)
 {
   int tm, tn;
   map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
   if (p.tiles_n % 5 != 0) { tn = (tn * 5) % p.tiles_n; }
-  m0 = tm * kBM;
+  m0 = tm * BM;
   n0 = tn * kBN;
 }
 
@@ -152,12 +153,13 @@ __device__ __forceinline__ void tile_of(const TallParams& p, int& m0, int& n0)
 // 0, 1, 2. The staged output tile of the epilogue reuses it.
 constexpr int kOp = 256 * kSB;
 constexpr int kXOff = 0;
-constexpr int kWOff = 2 * kOp;
 constexpr int kPPLds = 5 * kOp;
 static_assert(kPPLds == 160 * 1024, "the stages fill the LDS");
 static_assert(kBM * kEP * 2 <= kPPLds, "the staged tile fits the stages");
 
-template <int MODE, bool FOLD, bool STAMPS = false>
+// BM: rows of the tile, 256 or 128. The 128 x 256 tile is the same schedule with
+// half the rows per group.
+template <int MODE, bool FOLD, bool STAMPS = false, int BM = kBM>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 tall_kernel(TallParams p)
 {
@@ -166,7 +168,14 @@ tall_kernel(TallParams p)
   static_assert(!STAMPS || !FOLD, "the phase stamps are built without the two-part activation");
   constexpr bool I8 = MODE == kModeI8;
   constexpr int kEB = I8 ? 1 : 2;   // bytes per element
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kPPLds];
+  constexpr int kGR = BM / 2;       // output rows of a group
+  constexpr int kNI = kGR / 16;     // its 16-row blocks
+  constexpr int kXL = kGR / 32;     // X load instructions per wave and step
+  constexpr int kXOp = BM * kSB;    // bytes of an X stage
+  constexpr int kWOff = 2 * kXOp;
+  constexpr int kLds = kWOff + 3 * kOp;
+  static_assert(kLds <= kPPLds && BM * kEP * 2 <= kLds, "the stages and the staged tile fit");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
   // phase stamps: shader clock at entry, step 0 landed, K loop done, output
   // staged in LDS, stores complete; 100 MHz clock at entry and at the end
   unsigned long long st[5] = {0, 0, 0, 0, 0};
@@ -180,10 +189,10 @@ tall_kernel(TallParams p)
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = wave >> 2;      // group: output rows 128 g .. 128 g + 127
+  const int g = wave >> 2;      // group: output rows kGR g .. kGR g + kGR - 1
   const int wn = wave & 3;      // output columns 64 wn .. 64 wn + 63
   int m0, n0;
-  tile_of(p, m0, n0);
+  tile_of<BM>(p, m0, n0);
   const uint32_t row_bytes = (uint32_t)p.K * kEB;
   const int n = (int)(row_bytes / kSB);   // K steps
 
@@ -191,11 +200,11 @@ tall_kernel(TallParams p)
   // of the tile; lane l lands at byte 16 l of the instruction's 1 KB (row
   // 8 q + l / 8, slot l % 8) and fetches the row's piece (l % 8) ^ (row % 8),
   // a lane constant since 8 q is a multiple of 8. A wave of group 0 issues X
-  // instructions 16 + 4 wn + i (the half group 1 reads), one of group 1
-  // instructions 4 wn + i; wave w issues weight instructions 4 w + i.
+  // instructions kGR / 8 + kXL wn + i (the half group 1 reads), one of group 1
+  // instructions kXL wn + i; wave w issues weight instructions 4 w + i.
   const uint32_t swz = (uint32_t)(((lane & 7) ^ ((lane >> 3) & 7)) * 16);
-  const int xq = (g == 0 ? 16 : 0) + 4 * wn;
-  const int xq_own = (g == 0 ? 0 : 16) + 4 * wn;   // the half the wave's group reads
+  const int xq = (g == 0 ? kGR / 8 : 0) + kXL * wn;
+  const int xq_own = (g == 0 ? 0 : kGR / 8) + kXL * wn;   // the half the wave's group reads
   const int wq = 4 * wave;
   const uint32_t xrow = (uint32_t)(m0 + 8 * xq + (lane >> 3));
   const uint32_t xrow_own = (uint32_t)(m0 + 8 * xq_own + (lane >> 3));
@@ -218,18 +227,18 @@ tall_kernel(TallParams p)
   const uint32_t xv2_own = FOLD ? xrow_own * rb2 + swz : 0u;
   // `own`: the X half this wave's group reads (the prologue's step 0)
   auto load_x = [&](int s, bool own, int q0) {
-    uint8_t* const base = lds + kXOff + (s & 1) * kOp + q0 * 1024;
+    uint8_t* const base = lds + kXOff + (s & 1) * kXOp + q0 * 1024;
     if (!FOLD || s < fsteps) {
       const uint32_t v0 = own ? xv1_own : xv1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < kXL; ++i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xr1, (lds_u32*)(base + i * 1024), 16,
                                                  (int)(v0 + 8u * i * rb1), s * kSB, 0, 0);
       }
     } else {
       const uint32_t v0 = own ? xv2_own : xv2;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < kXL; ++i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xr2, (lds_u32*)(base + i * 1024), 16,
                                                  (int)(v0 + 8u * i * rb2), (s - fsteps) * kSB, 0,
                                                  0);
@@ -251,25 +260,25 @@ tall_kernel(TallParams p)
   // 16 int8 of a 16x16x64 one), at slot piece ^ (l % 8)
   const int fo0 = (lane & 15) * kSB + ((((lane >> 4)) ^ (lane & 7)) * 16);
   const int fo1 = (lane & 15) * kSB + (((4 + (lane >> 4)) ^ (lane & 7)) * 16);
-  const int xbase = kXOff + g * 128 * kSB;
+  const int xbase = kXOff + g * kGR * kSB;
   const int wbase = kWOff + wn * 64 * kSB;
-  i32x4v afr[2][8], bfr[2][4];
+  i32x4v afr[2][kNI], bfr[2][4];
   auto read_frags = [&](int xst, int wst) {
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
       const int fo = sl ? fo1 : fo0;
-      const uint8_t* const sa = lds + xbase + xst * kOp + fo;
+      const uint8_t* const sa = lds + xbase + xst * kXOp + fo;
       const uint8_t* const sb = lds + wbase + wst * kOp + fo;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) { afr[sl][i] = *(const i32x4v*)(sa + i * 16 * kSB); }
+      for (int i = 0; i < kNI; ++i) { afr[sl][i] = *(const i32x4v*)(sa + i * 16 * kSB); }
 #pragma unroll
       for (int j = 0; j < 4; ++j) { bfr[sl][j] = *(const i32x4v*)(sb + j * 16 * kSB); }
     }
   };
   using AccT = std::conditional_t<I8, i32x4v, f32x4v>;
-  AccT acc[8][4];
+  AccT acc[kNI][4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < kNI; ++i) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -288,8 +297,8 @@ tall_kernel(TallParams p)
       const int lrow = lane & 15;
       const int lcol = (lane >> 4) * 4;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int m = m0 + g * 128 + i * 16 + lrow;
+      for (int i = 0; i < kNI; ++i) {
+        const int m = m0 + g * kGR + i * 16 + lrow;
         if (m >= p.M) { continue; }
         const uint16_t* const yrow = p.y_in + (size_t)m * p.N;
 #pragma unroll
@@ -309,7 +318,7 @@ tall_kernel(TallParams p)
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < kNI; ++i) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if constexpr (I8) {
@@ -334,8 +343,8 @@ tall_kernel(TallParams p)
   if (n > 1) {
     load_w(1, 1);
     if (g == 1) { load_x(1, false, xq); }
-    // step 0 landed: group 0 leaves W(1) (4) in flight, group 1 W(1) and X(1) (8)
-    if (g == 0) { LTX25_VMCNT(4); } else { LTX25_VMCNT(8); }
+    // step 0 landed: group 0 leaves W(1) (4) in flight, group 1 W(1) and X(1)
+    if (g == 0) { LTX25_VMCNT(4); } else { LTX25_VMCNT(4 + kXL); }
   } else {
     LTX25_VMCNT(0);
   }
@@ -375,15 +384,15 @@ tall_kernel(TallParams p)
     if (g == 0) {
       if (s >= 1) {
         if (m2) {
-          LTX25_VMCNT(12);
+          LTX25_VMCNT(8 + kXL);
         } else if (m1) {
-          LTX25_VMCNT(8);
+          LTX25_VMCNT(4 + kXL);
         } else {
           LTX25_VMCNT(0);
         }
       }
     } else if (m2) {
-      LTX25_VMCNT(8);
+      LTX25_VMCNT(4 + kXL);
     } else {
       LTX25_VMCNT(0);
     }
@@ -395,9 +404,9 @@ tall_kernel(TallParams p)
     __builtin_amdgcn_sched_barrier(0);
     if (g == 0) {
       if (m2) {
-        LTX25_VMCNT(8);
+        LTX25_VMCNT(4 + kXL);
       } else if (m1) {
-        LTX25_VMCNT(4);
+        LTX25_VMCNT(kXL);
       } else {
         LTX25_VMCNT(0);
       }
@@ -419,7 +428,7 @@ tall_kernel(TallParams p)
   // scales -- are loaded together before any is used, at indices clamped
   // into range (a column or row past the end is never stored): no branch
   // sits between the loads, so they are waited for once, not one by one.
-  float b4s[4][4], sw4s[4][4], sxm[8];
+  float b4s[4][4], sw4s[4][4], sxm[kNI];
   {
     int ncl[4][4];
 #pragma unroll
@@ -458,8 +467,8 @@ tall_kernel(TallParams p)
         for (int t = 0; t < 4; ++t) { sw4s[j][t] = p.sw[ncl[j][t]]; }
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int m = m0 + g * 128 + i * 16 + lrow;
+      for (int i = 0; i < kNI; ++i) {
+        const int m = m0 + g * kGR + i * 16 + lrow;
         sxm[i] = p.sx[m < p.M ? m : p.M - 1];
       }
       if (p.acc_out != nullptr) {
@@ -468,8 +477,8 @@ tall_kernel(TallParams p)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int m = m0 + g * 128 + i * 16 + lrow;
+          for (int i = 0; i < kNI; ++i) {
+            const int m = m0 + g * kGR + i * 16 + lrow;
             const int nn = n0 + wn * 64 + j * 16 + lcol;
             if (m < p.M && nn < p.N) {
               int32_t* arow = p.acc_out + (size_t)m * p.N + nn;
@@ -494,8 +503,8 @@ tall_kernel(TallParams p)
     for (int j = 0; j < 4; ++j) {
       const int c = wn * 64 + j * 16 + lcol;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int r = g * 128 + i * 16 + lrow;
+      for (int i = 0; i < kNI; ++i) {
+        const int r = g * kGR + i * 16 + lrow;
         float v[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -530,7 +539,7 @@ tall_kernel(TallParams p)
   LTX25_TSTAMP(st[3])
   constexpr int CPR = kBN / 8;   // 16-byte chunks per output row
 #pragma unroll 4
-  for (int q = tid; q < kBM * CPR; q += kThreads) {
+  for (int q = tid; q < BM * CPR; q += kThreads) {
     const int r = q / CPR;
     const int c = (q % CPR) * 8;
     const int m = m0 + r;
@@ -606,7 +615,7 @@ tall_w8_kernel(TallParams p)
   const int wm = wave >> 2;
   const int wn = wave & 3;
   int m0, n0;
-  tile_of(p, m0, n0);
+  tile_of<kBM>(p, m0, n0);
   const uint32_t row_bytes = (uint32_t)p.K * 2u;
   const int nsteps = p.K / kBK;
   auto pad_at = [&](int first, int c) -> float* {
@@ -852,7 +861,7 @@ tall_w8_kernel(TallParams p)
 constexpr size_t kTwoGib = (size_t)1 << 31;
 constexpr size_t kFourGib = (size_t)1 << 32;
 
-hipError_t launch_tall(const TallParams& p, int mode, hipStream_t stream)
+hipError_t launch_tall(const TallParams& p, int mode, int bm, hipStream_t stream)
 {
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
   if (p.stamps != nullptr) {
@@ -861,6 +870,16 @@ hipError_t launch_tall(const TallParams& p, int mode, hipStream_t stream)
       hipLaunchKernelGGL((tall_kernel<kModeI8, false, true>), grid, dim3(kThreads), 0, stream, p);
     } else if (mode == kModeBf16 && p.x2 == nullptr) {
       hipLaunchKernelGGL((tall_kernel<kModeBf16, false, true>), grid, dim3(kThreads), 0, stream, p);
+    } else {
+      return hipErrorInvalidValue;
+    }
+  } else if (bm == 128) {
+    if (mode == kModeI8) {
+      hipLaunchKernelGGL((tall_kernel<kModeI8, false, false, 128>), grid, dim3(kThreads), 0, stream, p);
+    } else if (mode == kModeBf16 && p.x2 != nullptr) {
+      hipLaunchKernelGGL((tall_kernel<kModeBf16, true, false, 128>), grid, dim3(kThreads), 0, stream, p);
+    } else if (mode == kModeBf16) {
+      hipLaunchKernelGGL((tall_kernel<kModeBf16, false, false, 128>), grid, dim3(kThreads), 0, stream, p);
     } else {
       return hipErrorInvalidValue;
     }
@@ -884,7 +903,7 @@ bool tall_dense_takes(const GemmDesc& d, const GemmPlan& plan)
   // accumulating output beside the two-part activation or off 8-byte
   // alignment. The per-lane byte offsets are 32-bit, rows past the last
   // tile's end included.
-  return plan.tile == 0 && plan.splits == 1 && d.bits == 16 &&
+  return (plan.tile == 0 || plan.half_tall) && plan.splits == 1 && d.bits == 16 &&
          (d.x2 == nullptr || (d.kx > 0 && d.kx < d.K && d.kx % kBK == 0)) &&
          (d.y_in == nullptr || (d.x2 == nullptr && ((uintptr_t)d.y_in & 7u) == 0)) &&
          d.N % 8 == 0 && d.K % kBK == 0 && d.K >= kBK &&
@@ -900,8 +919,12 @@ bool tall_w8_takes(const GemmDesc& d, const GemmPlan& plan)
          (size_t)(d.M + kBM) * d.K * 2 < kFourGib && (size_t)(d.N + kBN) * d.K < kFourGib;
 }
 
-hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, unsigned long long* stamps)
+hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm,
+                             unsigned long long* stamps)
 {
+  if ((bm != kBM && bm != kBM / 2) || (bm != kBM && (d.bits != 16 || stamps != nullptr))) {
+    return hipErrorInvalidValue;
+  }
   if (d.bits == 8) {
     GemmPlan plan;
     plan.tile = 0;
@@ -926,7 +949,7 @@ hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, unsigned lon
     p.epilogue = d.epilogue;
     p.tiles_m = (d.M + kBM - 1) / kBM;
     p.tiles_n = (d.N + kBN - 1) / kBN;
-    return launch_tall(p, kModeW8, stream);
+    return launch_tall(p, kModeW8, kBM, stream);
   }
   if (d.M < 1 || d.N < 8 || d.N % 8 != 0 || d.K < kBK || d.K % kBK != 0 || d.bits != 16 ||
       (size_t)d.M * d.K * 2 >= kTwoGib || (size_t)d.N * d.K * 2 >= kTwoGib ||
@@ -949,10 +972,10 @@ hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, unsigned lon
   p.wn = d.wn > 0 && d.wn < d.N ? d.wn : d.N;
   p.bias_type = d.bias != nullptr ? d.bias_type : kBiasNone;
   p.epilogue = d.epilogue;
-  p.tiles_m = (d.M + kBM - 1) / kBM;
+  p.tiles_m = (d.M + bm - 1) / bm;
   p.tiles_n = (d.N + kBN - 1) / kBN;
   p.stamps = stamps;
-  return launch_tall(p, kModeBf16, stream);
+  return launch_tall(p, kModeBf16, bm, stream);
 }
 
 bool tall_i8_takes(int M, int N, int K)
@@ -964,9 +987,12 @@ bool tall_i8_takes(int M, int N, int K)
 
 hipError_t launch_tall_i8(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
                           const void* bias, int bias_type, int epilogue, uint16_t* y,
-                          int32_t* acc, int M, int K, int N, hipStream_t stream,
+                          int32_t* acc, int M, int K, int N, hipStream_t stream, int bm,
                           unsigned long long* stamps)
 {
+  if ((bm != kBM && bm != kBM / 2) || (bm != kBM && stamps != nullptr)) {
+    return hipErrorInvalidValue;
+  }
   if (M < 1 || !tall_i8_takes(M, N, K) || (size_t)M * N * 2 >= kTwoGib) {
     return hipErrorInvalidValue;
   }
@@ -984,10 +1010,10 @@ hipError_t launch_tall_i8(const int8_t* xq, const float* sx, const int8_t* wq, c
   p.wn = N;
   p.bias_type = bias != nullptr ? bias_type : kBiasNone;
   p.epilogue = epilogue;
-  p.tiles_m = (M + kBM - 1) / kBM;
+  p.tiles_m = (M + bm - 1) / bm;
   p.tiles_n = (N + kBN - 1) / kBN;
   p.stamps = stamps;
-  return launch_tall(p, kModeI8, stream);
+  return launch_tall(p, kModeI8, bm, stream);
 }
 
 }  // namespace ltx25
