@@ -425,6 +425,29 @@ __global__ void lora_pad_kernel(const uint16_t* __restrict__ src, int rows, int 
   *(uint4*)(dst + r * (size_t)ld_dst + c) = v;
 }
 
+// at[k][i] = i < rank ? a[i][k] : 0 for i < rk: one 64 x 64 tile per workgroup,
+// through LDS so that both sides move whole 128-byte rows.
+__global__ void __launch_bounds__(256)
+lora_transpose_kernel(const uint16_t* __restrict__ a, int rank, int K, uint16_t* __restrict__ at,
+                      int rk)
+{
+  __shared__ uint16_t tile[64][66];
+  const int k0 = blockIdx.x * 64;
+  const int i0 = blockIdx.y * 64;
+  const int c = threadIdx.x & 63;
+  const int r0 = threadIdx.x >> 6;
+#pragma unroll
+  for (int r = 0; r < 64; r += 4) {
+    const int i = i0 + r + r0;
+    tile[r + r0][c] = i < rank ? a[(size_t)i * K + k0 + c] : 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 64; r += 4) {
+    at[(size_t)(k0 + r + r0) * rk + i0 + c] = tile[c][r + r0];
+  }
+}
+
 // ---- the adapter merged into the dequant-once expansion ----------------
 //   W'[n][k] = bf16(fma(scale, code, zero point) + sum_{i < rank} B[n][i] A[i][k])
 // The linear then runs over W' at its own K. (x . A^T) . B^T = x . (B . A)^T,
@@ -642,6 +665,17 @@ hipError_t launch_dequant_merge(const uint8_t* codes, const uint16_t* scales,
   } else {
     go(std::integral_constant<int, 64>{});
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_lora_transpose(const uint16_t* a, int rank, int K, uint16_t* at, int rk,
+                                 hipStream_t stream)
+{
+  if (rank < 1 || rk < rank || rk % 64 != 0 || K < 64 || K % 64 != 0) {
+    return hipErrorInvalidValue;
+  }
+  lora_transpose_kernel<<<dim3((unsigned)(K / 64), (unsigned)(rk / 64)), 256, 0, stream>>>(
+      a, rank, K, at, rk);
   return hipGetLastError();
 }
 
