@@ -858,14 +858,11 @@ int run_fold(DeviceState* ds, hipStream_t st, const FoldPlan& f, const void* x,
       wd = (uint16_t*)ds->deq;
       base = (char*)ds->lora_mm;
     }
-    hipError_t e = ltx25::launch_lora_transpose((const uint16_t*)a, rank, K, (uint16_t*)base, rk, st);
-    if (e != hipSuccess) { return hip_fail(e, "fold: A transpose launch"); }
-    const uint16_t* pb = (const uint16_t*)b;
-    if (pad_b) {
-      e = ltx25::launch_lora_pad(pb, N, rank, rank, (uint16_t*)(base + at_bytes), rk, st);
-      if (e != hipSuccess) { return hip_fail(e, "fold: B pad launch"); }
-      pb = (const uint16_t*)(base + at_bytes);
-    }
+    uint16_t* const bp = pad_b ? (uint16_t*)(base + at_bytes) : nullptr;
+    hipError_t e = ltx25::launch_lora_operands((const uint16_t*)a, (const uint16_t*)b, rank, K, N,
+                                               (uint16_t*)base, bp, rk, st);
+    if (e != hipSuccess) { return hip_fail(e, "fold: merge operands launch"); }
+    const uint16_t* const pb = pad_b ? bp : (const uint16_t*)b;
     e = ltx25::launch_tall_merge(w->codes, (const uint16_t*)w->scales, (const uint16_t*)w->qbias,
                                  w->bits, w->group, pb, (const uint16_t*)base, rk, wd, N, K, st);
     if (e != hipSuccess) { return hip_fail(e, "fold: merge gemm launch"); }

@@ -226,10 +226,11 @@ hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
 // folded linear's weight tail.
 hipError_t launch_lora_pad(const uint16_t* src, int rows, int cols, int ld_src, uint16_t* dst,
                            int ld_dst, hipStream_t stream, int width = 0);
-// A [rank][K] -> at [K][rk] with zeros past `rank` (rk a multiple of 64, K % 64 ==
-// 0, any 2-byte aligned A).
-hipError_t launch_lora_transpose(const uint16_t* a, int rank, int K, uint16_t* at, int rk,
-                                 hipStream_t stream);
+// launch_tall_merge's operands: A [rank][K] -> at [K][rk] and, unless bp is null, B
+// [N][rank] -> bp [N][rk], zeros past `rank` (rk a multiple of 64, K % 64 == 0, A and B
+// at any 2-byte alignment).
+hipError_t launch_lora_operands(const uint16_t* a, const uint16_t* b, int rank, int K, int N,
+                                uint16_t* at, uint16_t* bp, int rk, hipStream_t stream);
 // The dequant-once expansion with the adapter merged in (lora.hip):
 // out [N][K] = bf16(fma(scale, code, zero point) + B . A), A bf16
 // [rank][K], B bf16 [N][ldb] (columns from rank to ldb zero).

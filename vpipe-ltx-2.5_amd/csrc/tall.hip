@@ -296,8 +296,12 @@ tall_kernel(TallParams p)
   // the hand-counted vmcnt waits below only ever wait longer for them.
   if constexpr (SEED != 0) {
     // The output is a weight: its codes dequantized in the accumulators' layout,
-    // w = fma(scale, code, zero point), four codes of one group a load. All
-    // loads go out before the first is used.
+    // w = fma(scale, code, zero point). A lane needs, of block j, the quad of
+    // columns that its 16-lane row q = lane / 16 names; it loads the 16 codes of
+    // block q, so that a load covers 16 whole 64-code (w8) or 32-byte (w4) runs, and
+    // the four rows exchange quads (a 4 x 4 transpose of dwords by row swaps).
+    // The 4096 x 4096 merge at rank 450 takes 35 us so; loaded quad by quad, 16
+    // bytes of 16 rows an instruction, 39.
     static_assert(MODE == kModeBf16 && !FOLD && !STAMPS, "the merge is the plain bf16 mode");
     const int lrow = lane & 15;
     const int lcol = (lane >> 4) * 4;
@@ -305,18 +309,21 @@ tall_kernel(TallParams p)
     const __amdgpu_buffer_rsrc_t cr = make_rsrc(p.codes, (size_t)p.M * code_row);
     const __amdgpu_buffer_rsrc_t sr = make_rsrc(p.scales, (size_t)p.M * p.gcols * 2);
     const __amdgpu_buffer_rsrc_t zr = make_rsrc(p.qbias, (size_t)p.M * p.gcols * 2);
+    typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
     uint32_t cv[kNI][4], sv[kNI][2], zv[kNI][2];
 #pragma unroll
     for (int i = 0; i < kNI; ++i) {
       const uint32_t m = (uint32_t)(m0 + g * kGR + i * 16 + lrow);
+      const uint32_t off = m * code_row + (uint32_t)(n0 + wn * 64 + lcol * 4) * SEED / 8;
+      if constexpr (SEED == 8) {
+        const i32x4v v = __builtin_amdgcn_raw_buffer_load_b128(cr, (int)off, 0, 0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t off = m * code_row + (uint32_t)(n0 + wn * 64 + j * 16 + lcol) * SEED / 8;
-        if constexpr (SEED == 8) {
-          cv[i][j] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(cr, (int)off, 0, 0);
-        } else {
-          cv[i][j] = __builtin_amdgcn_raw_buffer_load_b16(cr, (int)off, 0, 0);
-        }
+        for (int j = 0; j < 4; ++j) { cv[i][j] = (uint32_t)v[j]; }
+      } else {
+        const u32x2v v =
+            __builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(cr, (int)off, 0, 0));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { cv[i][j] = (v[j >> 1] >> (16 * (j & 1))) & 0xffffu; }
       }
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
@@ -327,8 +334,23 @@ tall_kernel(TallParams p)
         zv[i][q] = __builtin_amdgcn_raw_buffer_load_b16(zr, (int)off, 0, 0);
       }
     }
+    // rows 2, 3 of the first against rows 0, 1 of the second; then rows 1, 3 against 0, 2
+    auto swap32 = [](uint32_t& a, uint32_t& b) {
+      const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+      a = r[0];
+      b = r[1];
+    };
+    auto swap16 = [](uint32_t& a, uint32_t& b) {
+      const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+      a = r[0];
+      b = r[1];
+    };
 #pragma unroll
     for (int i = 0; i < kNI; ++i) {
+      swap32(cv[i][0], cv[i][2]);
+      swap32(cv[i][1], cv[i][3]);
+      swap16(cv[i][0], cv[i][1]);
+      swap16(cv[i][2], cv[i][3]);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float sc = __uint_as_float(sv[i][j >> 1] << 16);
