@@ -178,19 +178,38 @@ def _ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _stream(stream) -> int | None:
-    if stream is not None:
-        return stream
+_torch = None
+_raw_stream = None
+
+
+def _import_torch():
+    """torch, imported on first use, and how its current stream's handle is read: the accessor
+    that returns the handle alone where torch has it (0.07 us; torch.cuda.current_stream() builds
+    a Stream object, 2.7 of the 8.2 us that a call took on the host)."""
+    global _torch, _raw_stream
     import torch
 
-    return torch.cuda.current_stream().cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    _raw_stream = raw if raw is not None else (
+        lambda device: torch.cuda.current_stream(device).cuda_stream)
+    _torch = torch
+    return torch
+
+
+def _current_stream() -> int:
+    torch = _torch or _import_torch()
+    # current_device() initialises torch's CUDA state, as current_stream() does
+    return _raw_stream(torch.cuda.current_device())
+
+
+def _stream(stream) -> int | None:
+    return stream if stream is not None else _current_stream()
 
 
 def bias_dtype_of(bias) -> int:
     if bias is None:
         return DT_NONE
-    import torch
-
+    torch = _torch or _import_torch()
     if bias.dtype == torch.bfloat16:
         return DT_BF16
     if bias.dtype == torch.float32:
@@ -422,9 +441,8 @@ def _pack_stream(stream):
     that host-side validation runs (and fails) without touching a device."""
     if stream is not None:
         return stream
-    import torch
-
-    return torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else None
+    torch = _torch or _import_torch()
+    return _current_stream() if torch.cuda.is_available() else None
 
 
 class Pack:
