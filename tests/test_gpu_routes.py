@@ -185,3 +185,83 @@ def test_larger_tiles_under_the_lora_pair(pkg, rank):
         outs.append((host_bits(y), host_bits(f)))
     assert np.array_equal(outs[0][0], outs[1][0])
     assert np.array_equal(outs[0][1], outs[1][1])
+
+
+# a last round of 256 x 256 tiles that leaves half of the CUs idle or more goes out as 128 x 256
+# tiles of the last columns or rows: ragged M and N on both sides of the cut. The forced 128 x 128
+# tile gives the same sums in one launch.
+ROUNDS = [  # M, K, N
+    (2040, 2048, 12288),   # 8 x 48: 32 columns of tiles, then 16
+    (6000, 2048, 4096),    # 24 x 16: 16 rows of tiles, then 8
+    (4500, 2112, 4360),    # 18 x 18, N past the last whole column
+    (2570, 2048, 6664),    # 11 x 27: 256 + 41
+]
+
+
+@pytest.mark.parametrize("M,K,N", ROUNDS)
+@pytest.mark.parametrize("bias,epi", [("f32", 1), ("bf16", 0)])
+def test_the_last_round_gives_the_same_bits(pkg, M, K, N, bias, epi):
+    rng = np.random.default_rng(M + K + N)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn((N, K), device="cuda", generator=g) * 0.05).to(torch.bfloat16)
+    b = rng_normal(rng, (N,), 0.05)
+    bd = dev_f32(b) if bias == "f32" else dev_bf16(orc.bf16_rne(b))
+    assert pkg.linear_route(M, K, N, 16)["tile"] == pkg.TILE_TALL
+    outs = []
+    for force in (pkg.TILE_AUTO, pkg.TILE_MID):
+        pkg.set_tile(force)
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        say(f"last round {M}x{K}->{N} bias={bias} epi={epi} forced={force}")
+        pkg.linear_qc(x, pkg.dense_weight(w), bd, y, M, K, N, epi)
+        torch.cuda.synchronize()
+        outs.append(y)
+    pkg.set_tile(pkg.TILE_AUTO)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("M,K,N", [(2040, 4096, 12296), (6000, 4096, 4096)])
+def test_the_last_int8_round_is_exact(pkg, M, K, N):
+    rng = np.random.default_rng(M + K)
+    xq = torch.from_numpy(rng.integers(-127, 128, (M, K), dtype=np.int8)).cuda()
+    wq = torch.from_numpy(rng.integers(-127, 128, (N, K), dtype=np.int8)).cuda()
+    sx = torch.from_numpy(rng.random(M, dtype=np.float32) * 0.01).cuda()
+    sw = torch.from_numpy(rng.random(N, dtype=np.float32) * 0.01).cuda()
+    b = torch.from_numpy(rng.random(N, dtype=np.float32)).cuda()
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    acc = torch.empty((M, N), dtype=torch.int32, device="cuda")
+    say(f"last int8 round {M}x{K}->{N}")
+    pkg.i8_gemm(xq, sx, wq, sw, b, y, acc, M, K, N)
+    torch.cuda.synchronize()
+    assert torch.equal(acc.double(), xq.double() @ wq.double().t())
+    want = torch.addcmul(b.double()[None, :], acc.double(),
+                         (sx[:, None] * sw[None, :]).double())   # one fma, then one rounding
+    assert torch.equal(y, want.float().to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N", [(2040, 12288), (6000, 4096)])
+def test_the_last_round_under_the_lora_pair(pkg, M, N):
+    """y-seeded accumulators (rank 2048 as the second GEMM's K) and the two-part activation: the
+    forced 128 x 128 tile's bits."""
+    K, rank = 2048, 2048
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    x, a, b, y0 = ((torch.randn(s, device="cuda", generator=g) * 0.1).to(torch.bfloat16)
+                   for s in ((M, K), (rank, K), (N, rank), (M, N)))
+    rng = np.random.default_rng(M)
+    qw = make_qweight(pkg, rng_normal(rng, (N, K), 0.05), 8, 64)[0]
+    assert pkg.lora_on_matrix_cores(M, K, N, rank)
+    outs = []
+    for force in (pkg.TILE_AUTO, pkg.TILE_MID):
+        pkg.set_tile(force)
+        y = y0.clone()
+        f = torch.empty_like(y)
+        say(f"last round under the LoRA pair {M}x{K}->{N} forced={force}")
+        pkg.lora_add(x, a, b, y, M, K, N, rank)
+        pkg.linear_q_lora(x, qw, None, a, b, rank, f, M, K, N, 0)
+        torch.cuda.synchronize()
+        outs.append((y, f))
+    pkg.set_tile(pkg.TILE_AUTO)
+    assert torch.equal(outs[0][0].view(torch.int16), outs[1][0].view(torch.int16))
+    assert torch.equal(outs[0][1].view(torch.int16), outs[1][1].view(torch.int16))

@@ -1383,7 +1383,7 @@ int ltx25_probe_tall_phases(void* stream, const void* x, const void* w_bf16, con
   d.M = M;
   d.N = N;
   d.K = K;
-  const hipError_t e = ltx25::launch_tall_dense(d, (hipStream_t)stream, 256,
+  const hipError_t e = ltx25::launch_tall_dense(d, (hipStream_t)stream, 256, 0,
                                                 (unsigned long long*)stamps);
   return e == hipSuccess ? LTX25_OK : hip_fail(e, "tall phase-stamp launch");
 }
@@ -1416,7 +1416,7 @@ int ltx25_probe_tall_i8_phases(void* stream, const int8_t* xq, const float* sx, 
   const hipError_t e = ltx25::launch_tall_i8(xq, sx, wq, sw, bias,
                                              bias != nullptr ? bias_dtype : ltx25::kBiasNone,
                                              ltx25::kEpiNone, (uint16_t*)y, nullptr, M, K, N,
-                                             (hipStream_t)stream, 256, (unsigned long long*)stamps);
+                                             (hipStream_t)stream, 256, 0, (unsigned long long*)stamps);
   return e == hipSuccess ? LTX25_OK : hip_fail(e, "tall i8 phase-stamp launch");
 }
 

@@ -176,9 +176,10 @@ bool tall_w8_takes(const GemmDesc& d, const GemmPlan& plan);
 // `stamps` non-null (bf16 without the two-part activation, or the int8
 // launcher below): the phase-stamp instantiation, eight words per wave at
 // (tile * 8 + wave) * 8 (ltx25_probe_tall_phases). `bm`: rows of the tile, 256, or
-// 128 for a dense weight (plan.half_tall).
+// 128 for a dense weight (plan.half_tall). With the device's cu_count a last round
+// of 256-row tiles that would leave CUs idle goes out as 128-row ones.
 hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm = 256,
-                             unsigned long long* stamps = nullptr);
+                             int cu_count = 0, unsigned long long* stamps = nullptr);
 // The dequant-once expansion with an adapter of any rank merged in, as a GEMM
 // on the same tile: out [N][K] = bf16(fma(scale, code, zero point) + b . at^T), b
 // bf16 [N][rk], at (A transposed) bf16 [K][rk], rk a multiple of 64; bits 8 or
@@ -193,7 +194,7 @@ bool tall_i8_takes(int M, int N, int K);
 hipError_t launch_tall_i8(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
                           const void* bias, int bias_type, int epilogue, uint16_t* y,
                           int32_t* acc, int M, int K, int N, hipStream_t stream, int bm = 256,
-                          unsigned long long* stamps = nullptr);
+                          int cu_count = 0, unsigned long long* stamps = nullptr);
 // The no-allocation linear's split-K scratch (noalloc.hip): a fixed device
 // array of kNoAllocScratchBytes per GPU. noalloc_scratch() returns the
 // current device's copy, resolving its address on the first call there.

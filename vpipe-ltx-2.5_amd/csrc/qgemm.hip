@@ -909,7 +909,7 @@ hipError_t launch_i8_gemm(const int8_t* xq, const float* sx, const int8_t* wq, c
   const int rows = tall_rows(M, N, cus);
   if (rows > 0 && tall_i8_takes(M, N, K)) {
     return launch_tall_i8(xq, sx, wq, sw, bias, kp.bias_type, epilogue, y, acc, M, K, N, stream,
-                          rows);
+                          rows, cus);
   }
   if (fills) {
     kp.tiles_m = (M + 255) / 256;
@@ -945,7 +945,7 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
   if (plan.tile == 2) { return launch_skinny(d, plan, workspace, stream); }
   if (plan.panel_rows > 0 && d.x2 == nullptr) { return launch_panel(d, plan, workspace, stream); }
   if (tall_dense_takes(d, plan) || tall_w8_takes(d, plan)) {
-    return launch_tall_dense(d, stream, plan.half_tall ? 128 : 256);
+    return launch_tall_dense(d, stream, plan.half_tall ? 128 : 256, plan.cu_count);
   }
   KParams kp = {};
   kp.x = d.x;

@@ -97,6 +97,10 @@ struct TallParams {
   // the phase-stamp instantiation only (ltx25_probe_tall_phases): eight
   // words per wave at (tile * 8 + wave) * 8
   unsigned long long* stamps;
+  // 128-row tiles: the first column. Last, so that the 256-row kernels load their
+  // arguments as without it: with one more scalar load they start 8 bytes off, and
+  // 8160 x 4096 x 4096 took 1% longer.
+  int n_first;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, size_t bytes)
@@ -195,6 +199,8 @@ tall_kernel(TallParams p)
   const int wn = wave & 3;      // output columns 64 wn .. 64 wn + 63
   int m0, n0;
   tile_of<BM>(p, m0, n0);
+  // the last round of a launch in two (launch_rounds): the columns left to it
+  if constexpr (BM != kBM) { n0 += p.n_first; }
   const uint32_t row_bytes = (uint32_t)p.K * kEB;
   const int n = (int)(row_bytes / kSB);   // K steps
 
@@ -965,6 +971,58 @@ hipError_t launch_tall(const TallParams& p, int mode, int bm, hipStream_t stream
   return hipGetLastError();
 }
 
+// 256-row tiles, in two launches where the last round of them would leave half of
+// the CUs idle or more: whole rounds take the first columns (or rows), and the
+// rest goes out as 128 x 256 tiles, which fit one round. At K = 4096 a last round of
+// r tiles takes about 58 + 0.16 r us, 2 r half tiles 40 + 0.18 r and the second
+// launch 3 us, so from 2048 of K (4096 int8). Dense 2040 x 4096 -> 12288 (384 tiles)
+// 174 -> 165 us, 5000 x 8192 -> 4096 (320) 316 -> 284; int8 8160 x 8192 -> 4352 (544)
+// 260 -> 244. The same bits.
+hipError_t launch_rounds(const TallParams& p, int mode, int cu_count, hipStream_t stream)
+{
+  const size_t eb = mode == kModeI8 ? 1 : 2;
+  const size_t row = (size_t)p.K * eb;   // bytes of a weight row, and of an activation's
+  const long tiles = (long)p.tiles_m * p.tiles_n;
+  if (cu_count <= 0 || tiles < cu_count || tiles % cu_count == 0 || row < 4096) {
+    return launch_tall(p, mode, kBM, stream);
+  }
+  const long full = tiles / cu_count * cu_count;
+  const int half_m = (p.M + 127) / 128;
+  const int cols = (int)(full / p.tiles_m);   // N-tiles in whole rounds, all rows
+  const int rows = (int)(full / p.tiles_n);   // or M-tiles, all columns
+  const bool by_cols = cols >= 1 && (long)half_m * (p.tiles_n - cols) <= cu_count;
+  const bool by_rows = rows >= 1 && (long)(half_m - 2 * rows) * p.tiles_n <= cu_count;
+  // the one whose first launch is fuller
+  const bool take_rows =
+      by_rows && (!by_cols || (long)rows * p.tiles_n > (long)cols * p.tiles_m);
+  if (!by_cols && !by_rows) { return launch_tall(p, mode, kBM, stream); }
+  TallParams a = p;
+  TallParams b = p;
+  if (take_rows) {
+    const size_t m1 = (size_t)rows * kBM;
+    a.M = (int)m1;
+    a.tiles_m = rows;
+    b.M = p.M - (int)m1;
+    if (p.x2 != nullptr) {
+      b.x = (const uint8_t*)p.x + m1 * p.kx * eb;
+      b.x2 = (const uint8_t*)p.x2 + m1 * (p.K - p.kx) * eb;
+    } else {
+      b.x = (const uint8_t*)p.x + m1 * row;
+    }
+    b.y = p.y + m1 * p.N;
+    if (p.y_in != nullptr) { b.y_in = p.y_in + m1 * p.N; }
+    if (p.sx != nullptr) { b.sx = p.sx + m1; }
+    if (p.acc_out != nullptr) { b.acc_out = p.acc_out + m1 * p.N; }
+  } else {
+    a.tiles_n = cols;
+    b.tiles_n = p.tiles_n - cols;
+    b.n_first = cols * kBN;
+  }
+  b.tiles_m = (b.M + 127) / 128;
+  const hipError_t e = launch_tall(a, mode, kBM, stream);
+  return e != hipSuccess ? e : launch_tall(b, mode, kBM / 2, stream);
+}
+
 }  // namespace
 
 bool tall_dense_takes(const GemmDesc& d, const GemmPlan& plan)
@@ -989,7 +1047,7 @@ bool tall_w8_takes(const GemmDesc& d, const GemmPlan& plan)
          (size_t)(d.M + kBM) * d.K * 2 < kFourGib && (size_t)(d.N + kBN) * d.K < kFourGib;
 }
 
-hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm,
+hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm, int cu_count,
                              unsigned long long* stamps)
 {
   if ((bm != kBM && bm != kBM / 2) || (bm != kBM && (d.bits != 16 || stamps != nullptr))) {
@@ -1045,7 +1103,8 @@ hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm,
   p.tiles_m = (d.M + bm - 1) / bm;
   p.tiles_n = (d.N + kBN - 1) / kBN;
   p.stamps = stamps;
-  return launch_tall(p, kModeBf16, bm, stream);
+  return bm == kBM && stamps == nullptr ? launch_rounds(p, kModeBf16, cu_count, stream)
+                                        : launch_tall(p, kModeBf16, bm, stream);
 }
 
 hipError_t launch_tall_merge(const void* codes, const uint16_t* scales, const uint16_t* qbias,
@@ -1101,7 +1160,7 @@ bool tall_i8_takes(int M, int N, int K)
 hipError_t launch_tall_i8(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
                           const void* bias, int bias_type, int epilogue, uint16_t* y,
                           int32_t* acc, int M, int K, int N, hipStream_t stream, int bm,
-                          unsigned long long* stamps)
+                          int cu_count, unsigned long long* stamps)
 {
   if ((bm != kBM && bm != kBM / 2) || (bm != kBM && stamps != nullptr)) {
     return hipErrorInvalidValue;
@@ -1126,7 +1185,8 @@ hipError_t launch_tall_i8(const int8_t* xq, const float* sx, const int8_t* wq, c
   p.tiles_m = (M + bm - 1) / bm;
   p.tiles_n = (N + kBN - 1) / kBN;
   p.stamps = stamps;
-  return launch_tall(p, kModeI8, bm, stream);
+  return bm == kBM && stamps == nullptr ? launch_rounds(p, kModeI8, cu_count, stream)
+                                        : launch_tall(p, kModeI8, bm, stream);
 }
 
 }  // namespace ltx25
