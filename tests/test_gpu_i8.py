@@ -370,3 +370,76 @@ def test_tier_with_gelu_at_the_ffn_shape(pkg):
         pkg.set_i8_gemm(False)
     r = ((tier.float() - base.float()).norm() / base.float().norm()).item()
     assert 1e-5 < r < 3e-2, f"rel-L2 {r:.3e}"
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+def test_quantize_qweight_edges(pkg, bits):
+    """Rows whose scale's reciprocal overflows or is below the normal range, and NaN and infinite
+    scales and zero points: as the quotient of each dequantized value, a NaN to -127."""
+    group, N, K = 64, 12, 1344
+    rng = np.random.default_rng(37 + bits)
+    codes = rng.integers(0, 1 << bits, (N, K), dtype=np.uint8)
+    codes[:, ::7] = 0
+    sc = rng_normal(rng, (N, K // group), 0.02)
+    zp = rng_normal(rng, (N, K // group), 1.0)
+    for row, f in ((0, 2.0 ** -124), (1, 2.0 ** -131), (2, 1e-40), (3, 1e38), (4, 2.0 ** 119)):
+        sc[row] *= f
+        zp[row] *= f
+    sc[5, 3], sc[6, 20], zp[7, 0] = np.nan, np.inf, -np.inf
+    sc[8, 2], zp[8, 2] = np.inf, -np.inf
+    zp[9, 5] = np.nan
+    scales, biases = orc.bf16_rne(sc.astype(np.float32)), orc.bf16_rne(zp.astype(np.float32))
+    words = orc.pack(codes, bits)
+    with np.errstate(all="ignore"):
+        s32, z32 = (np.repeat(orc.bf16_to_f32(a), group, axis=1).astype(np.float64)
+                    for a in (scales, biases))
+        # 8 + 8 bits of product and a sum: one rounding to bf16 from the exact value in float64,
+        # of which the float32 step in between is exact or far from a bf16 tie here
+        v = orc.bf16_to_f32(orc.bf16_rne((s32 * codes + z32).astype(np.float32)))
+        v = np.where(np.isnan(s32 * codes + z32), np.float32(np.nan), v.reshape(N, K))
+        s_ref = (np.fmax.reduce(np.abs(v), axis=1) / np.float32(127.0)).astype(np.float32)
+        t = v / s_ref[:, None]
+        q_ref = np.where(np.isnan(t), -127, np.clip(np.rint(t), -127, 127)).astype(np.int8)
+    qw = pkg.QWeight(dev_bytes(words), dev_bf16(scales), dev_bf16(biases), bits, group)
+    wq = torch.empty((N, K), dtype=torch.int8, device="cuda")
+    sw = torch.empty((N,), dtype=torch.float32, device="cuda")
+    say(f"i8 quantize of weight edges w{bits}")
+    pkg.i8_quantize_qweight(qw, wq, sw, N, K)
+    torch.cuda.synchronize()
+    assert np.array_equal(sw.cpu().numpy(), s_ref)
+    assert np.array_equal(wq.cpu().numpy(), q_ref)
+
+
+# the tier quantizes both operands in one launch: the chunks per lane at each K's instance, past
+# the registers, the last workgroup with rows of both; the output is that of the separate entries
+@pytest.mark.parametrize("bits", [16, 8, 4])
+@pytest.mark.parametrize("M,K,N", [(1025, 1024, 18), (1031, 2048, 33), (1024, 4224, 16),
+                                   (1026, 8192, 19), (1027, 16896, 17)])
+def test_tier_quantizes_as_the_separate_entries(pkg, bits, M, K, N):
+    say(f"i8 tier operands w{bits} {M}x{K}->{N}")
+    rng = np.random.default_rng(M + K + bits)
+    x = dev_bf16(orc.bf16_rne(rng_normal(rng, (M, K))))
+    wf = rng_normal(rng, (N, K), 0.02)
+    b = dev_f32(rng_normal(rng, (N,), 0.01))
+    xq, sx = quantize_rows_dev(pkg, x, M, K)
+    if bits == 16:
+        w = dev_bf16(orc.bf16_rne(wf))
+        wq, sw = quantize_rows_dev(pkg, w, N, K)
+    else:
+        qw = make_qweight(pkg, wf, bits, 64)[0]
+        wq = torch.empty((N, K), dtype=torch.int8, device="cuda")
+        sw = torch.empty((N,), dtype=torch.float32, device="cuda")
+        pkg.i8_quantize_qweight(qw, wq, sw, N, K)
+    want, _ = i8_run(pkg, xq, sx, wq, sw, b, M, K, N, want_acc=False)
+    got = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    pkg.set_i8_gemm(True)
+    try:
+        assert pkg.i8_takes(M, K, N)
+        if bits == 16:
+            pkg.linear(x, w, b, got, M, K, N)
+        else:
+            pkg.linear_q(x, qw, b, got, M, K, N)
+        torch.cuda.synchronize()
+    finally:
+        pkg.set_i8_gemm(False)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

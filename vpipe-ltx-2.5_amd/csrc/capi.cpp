@@ -424,16 +424,10 @@ int run_i8_linear(DeviceState* ds, hipStream_t st, const void* x,
   float* sx = (float*)(base + xq_b);
   int8_t* wq = (int8_t*)(base + xq_b + sx_b);
   float* sw = (float*)(base + xq_b + sx_b + wq_b);
-  hipError_t e = ltx25::launch_i8_quantize_rows((const uint16_t*)x, xq, sx, M, K, st);
-  if (e != hipSuccess) { return hip_fail(e, "i8 quantize (x)"); }
-  if (w->quantized) {
-    e = ltx25::launch_i8_quantize_qweight(w->codes, (const uint16_t*)w->scales,
-                                          (const uint16_t*)w->qbias, w->bits,
-                                          w->group, wq, sw, N, K, st);
-  } else {
-    e = ltx25::launch_i8_quantize_rows((const uint16_t*)w->w, wq, sw, N, K, st);
-  }
-  if (e != hipSuccess) { return hip_fail(e, "i8 quantize (w)"); }
+  hipError_t e = ltx25::launch_i8_quantize_both(
+      w->quantized ? w->codes : w->w, (const uint16_t*)w->scales, (const uint16_t*)w->qbias,
+      w->quantized ? w->bits : 16, w->group, wq, sw, N, (const uint16_t*)x, xq, sx, M, K, st);
+  if (e != hipSuccess) { return hip_fail(e, "i8 quantize"); }
   e = ltx25::launch_i8_gemm(xq, sx, wq, sw, bias, bias != nullptr ? bias_dtype : 0, epilogue,
                             (uint16_t*)y, nullptr, M, K, N, st);
   if (e != hipSuccess) { return hip_fail(e, "i8 gemm launch"); }

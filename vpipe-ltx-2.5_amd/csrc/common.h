@@ -277,6 +277,11 @@ hipError_t launch_i8_quantize_qweight(const void* codes,
                                       const uint16_t* qbias, int bits,
                                       int group, int8_t* q, float* s, int N,
                                       int K, hipStream_t stream);
+// Both of a linear's operands in one launch; bits 16: w holds bf16 rows.
+hipError_t launch_i8_quantize_both(const void* w, const uint16_t* scales, const uint16_t* qbias,
+                                   int bits, int group, int8_t* wq, float* sw, int N,
+                                   const uint16_t* x, int8_t* xq, float* sx, int M, int K,
+                                   hipStream_t stream);
 // y = bf16(epilogue(fma(float(acc), sx[m] * sw[n], bias[n]))), epilogue
 // kEpiNone or kEpiGelu (GELU-tanh in f32 before the one rounding).
 hipError_t launch_i8_gemm(const int8_t* xq, const float* sx,
