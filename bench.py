@@ -575,7 +575,7 @@ def tall_phases_summary(json_path, trace_csv, out, cmd):
     for r in rows:
         name = r["Kernel_Name"].replace("(anonymous namespace)::", "").split("(")[0]
         dur = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
-        if re.search(r"tall_kernel<\d+, false, true>$", name):
+        if re.search(r"tall_kernel<\d+, false, true(, \d+)*>$", name):
             if apart:
                 runs.append([])
             runs[-1].append(dur)
@@ -638,7 +638,7 @@ def skinny_phases_summary(json_path, trace_csv, out, cmd):
     for r in rows:
         name = r["Kernel_Name"].replace("(anonymous namespace)::", "").split("(")[0]
         dur = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
-        if re.search(r"skinny_kernel<\d+, (true|false), true>$", name):
+        if re.search(r"skinny_kernel<\d+, (true|false)(, \d+)?, true>$", name):
             key = (int(r.get("Grid_Size_X", r.get("Grid_Size", 0))), int(r.get("Grid_Size_Y", 1)))
             if apart or runs[-1]["key"] != key:
                 runs.append({"key": key, "main": [], "reduce": []})

@@ -223,7 +223,10 @@ int ltx25_dequant_once_takes(int M, int K, int N);
 /* ---- routing: what a linear runs on, and the A/B switch ------------------------ */
 
 /* Tile families of the GEMM behind ltx25_linear / ltx25_linear_q:
- *   TALL    256 x 256 output tiles, all of K per workgroup (the video GEMMs)
+ *   TALL    256 x 256 output tiles, all of K per workgroup (the video GEMMs);
+ *           dense weights and the int8 tier also run 128 x 256 ones, for
+ *           outputs below a round of workgroups and for a poorly filled
+ *           last round (a launch of its own; the same bits)
  *   MID     the shapes between: under AUTO and from K = 1024, panels of 32 to
  *           128 rows x 32 or 64 columns that split K between a workgroup's
  *           waves (and, at large K, across workgroups) where one round of
@@ -346,6 +349,9 @@ int ltx25_lora_route(const void* x, const void* a, const void* b, const void* y,
  *     y = epi(x . W'^T + bias) at the linear's own K
  *     ((x . A^T) . B^T = x . (B . A)^T); one rounding per weight element
  *     and one of the output;
+ *   - wider adapters and w4 codes, where M is large enough for it to cost
+ *     less than the form below: the same W', by a GEMM whose accumulators
+ *     start from the dequantized codes;
  *   - otherwise as rank-rounded-to-64 more K: y = epi([x | r] . [W | B]^T
  *     + bias), r = bf16(x . A^T), one rounding of the output;
  * where the reference rounds the linear and the delta separately.

@@ -760,7 +760,10 @@ FoldPlan plan_fold(int M, int K, int N, int rank, int bits, int cu_count, const 
   }
   if (!f.merge && K % 64 == 0 && below_limit((size_t)(N + 256) * rk * 2) &&
       below_limit((size_t)(K + 256) * rk * 2) && below_limit((size_t)N * K * 2)) {
-    // expected times in us, from the figures of their kernels on a 256-CU GPU
+    // expected times in us, from the figures of their kernels on a 256-CU GPU: the
+    // merge's operands (6) and its GEMM per round against r's GEMM, the wider main GEMM
+    // and the expansion. 8160 x 4096 -> 4096 at rank 450: 227 us merged, 268 as extra K;
+    // the extra K form stays where few tokens share the merge.
     const double nk = (double)N * K, mrk = (double)M * rk;
     const double rounds = (double)(((long)((N + 255) / 256) * ((K + 255) / 256) + cu_count - 1) / cu_count);
     const double merge_us = 10.0 + rounds * (12.0 + 1.2 * rk / 64);

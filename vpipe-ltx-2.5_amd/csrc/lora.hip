@@ -28,7 +28,9 @@
 // With many tokens the host computes r = bf16(x . A^T) once with the dense
 // GEMM instead (phase 1 here re-reads x and all of A for every column split
 // of a row block) and the kernel runs phase 2 only, reading its 32 rows of
-// r from that buffer (`r_in`, [M][rank], rank % 8 == 0).
+// r from that buffer (`r_in`, [M][rank], rank % 8 == 0). Below 512 tokens it does so
+// where phase 1 is the larger part (K from 1536; from 512 for wide ranks). A linear's
+// GELU can follow the sum in the y phase, instead of a pass of its own.
 
 #include <type_traits>
 

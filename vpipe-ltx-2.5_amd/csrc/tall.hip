@@ -12,6 +12,10 @@
 //     workgroup before the LDS write, with the expansion kernel's
 //     arithmetic, so its results equal the bf16 mode's over the expansion
 //     bit for bit (tall_w8_kernel, below).
+// tall_kernel is also instantiated with 128 rows (the same schedule, half the rows
+// per group), for outputs below a round of 256 x 256 tiles and for a poorly filled
+// last round, and with accumulators that start from a weight's codes (the wide
+// adapter merged into the expansion).
 //
 // bf16 and int8: tall_kernel, an 8-wave ping-pong schedule.
 //   - Waves 0-3 (group 0) own output rows 0..127, waves 4-7 (group 1) rows
