@@ -238,3 +238,65 @@ def test_lora_caller_r_holds_r(pkg, dev, what, M, K, N, rank, route):
     r_ref = orc.bf16_to_f32(xb).astype(np.float64) @ orc.bf16_to_f32(ab).astype(np.float64).T
     assert np.isfinite(r_got).all()
     assert max_rel(r_got, r_ref) <= MAX_REL
+
+
+# the plans' scratch is the stream's own: ranks and K of both two-launch plans
+OWN = [(128, 4096, 1032, 32), (100, 2048, 1000, 200)]
+
+
+def own_operands(M, K, N, rank):
+    x, a, b, y0 = draws(f"own {M} {K} {N} {rank}", M, K, N, rank)
+    return tuple(dev_bf16(orc.bf16_rne(t)) for t in (x, a, b, y0))
+
+
+@pytest.mark.parametrize("M,K,N,rank", OWN)
+def test_plans_under_capture_run_in_one_pass(pkg, dev, M, K, N, rank):
+    """A capture without a call before it: the one-pass kernel, which needs no scratch."""
+    x, a, b, y0 = own_operands(M, K, N, rank)
+    want = y0.clone()
+    pkg.set_lora_route(pkg.LORA_FUSED)
+    pkg.lora_add(x, a, b, want, M, K, N, rank)
+    pkg.set_lora_route(pkg.LORA_AUTO)
+    y, eager = y0.clone(), y0.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    say(f"lora_add captured first M={M} K={K} N={N} rank={rank}")
+    with torch.cuda.graph(graph):
+        pkg.lora_add(x, a, b, y, M, K, N, rank)
+    for _ in range(3):
+        y.copy_(y0)
+        graph.replay()
+        eager.copy_(y0)
+        pkg.lora_add(x, a, b, eager, M, K, N, rank)   # the plan's own scratch meanwhile
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        assert (eager.float() - want.float()).norm() < 3e-3 * want.float().norm()
+
+
+@pytest.mark.parametrize("M,K,N,rank", OWN)
+def test_plans_overlap_on_streams(pkg, dev, M, K, N, rank):
+    """Calls on ten streams at once, more than have scratch of their own: each result is the one
+    it has alone, the plan's or the one-pass kernel's."""
+    n = 10
+    x, a, b, y0 = own_operands(M, K, N, rank)
+    xs = [x * (i + 1) for i in range(n)]
+    alone = []
+    for xi in xs:
+        plan, one = y0.clone(), y0.clone()
+        pkg.lora_add(xi, a, b, plan, M, K, N, rank)
+        pkg.set_lora_route(pkg.LORA_FUSED)
+        pkg.lora_add(xi, a, b, one, M, K, N, rank)
+        pkg.set_lora_route(pkg.LORA_AUTO)
+        alone.append((plan, one))
+    streams = [torch.cuda.Stream() for _ in range(n)]
+    ys = [[y0.clone() for _ in range(6)] for _ in range(n)]
+    torch.cuda.synchronize()
+    say(f"lora_add on {n} streams M={M} K={K} N={N} rank={rank}")
+    for t in range(6):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                pkg.lora_add(xs[i], a, b, ys[i][t], M, K, N, rank)
+    torch.cuda.synchronize()
+    for i in range(n):
+        for y in ys[i]:
+            assert any(torch.equal(y.view(torch.int16), w.view(torch.int16)) for w in alone[i])

@@ -67,6 +67,15 @@ int hip_fail(hipError_t e, const char* what)
 constexpr int kMaxDevices = 64;
 
 // Per-device state: checked once, then the grow-only scratch.
+// Scratch of the streams that ran the fused LoRA's two-launch plans
+constexpr int kLoraSlots = 8;
+struct LoraSlot {
+  bool used = false;
+  hipStream_t stream = nullptr;
+  void* buf = nullptr;
+  size_t bytes = 0;
+};
+
 struct DeviceState {
   bool checked = false;
   bool ok = false;
@@ -82,6 +91,7 @@ struct DeviceState {
   size_t lora_b_bytes = 0;
   void* lora_mm = nullptr;   // LoRA GEMM pair: A padded | r | B padded
   size_t lora_mm_bytes = 0;
+  LoraSlot lora_few[kLoraSlots];   // the fused LoRA's other plans (lora_slot)
 };
 
 std::mutex g_mu;
@@ -506,8 +516,9 @@ int lora_route(int M, int K, int N, int rank, const void* x, const void* a, cons
   return LTX25_LORA_FUSED;
 }
 
+// `own`: scratch of the call's own (lora_few_pair_bytes) instead of the library's.
 int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, const void* b,
-              void* y, void* r_caller, int M, int K, int N, int rank)
+              void* y, void* r_caller, int M, int K, int N, int rank, char* own = nullptr)
 {
   const int rk = (rank + 63) & ~63;
   // A's rows past `rank` read as zeros (the GEMM's weight-row bound), so A
@@ -520,8 +531,8 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
   const size_t a_bytes = pad_a ? align256((size_t)rk * K * 2) : 0;
   const size_t r_bytes = own_r ? align256((size_t)M * rk * 2) : 0;
   const size_t b_bytes = pad_b ? align256((size_t)N * rk * 2) : 0;
-  char* base = nullptr;
-  if (a_bytes + r_bytes + b_bytes > 0) {
+  char* base = own;
+  if (own == nullptr && a_bytes + r_bytes + b_bytes > 0) {
     std::lock_guard<std::mutex> lk(g_mu);
     const int rc = grow(&ds->lora_mm, &ds->lora_mm_bytes, a_bytes + r_bytes + b_bytes);
     if (rc != LTX25_OK) { return rc; }
@@ -568,7 +579,9 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
                   : ltx25::plan_gemm(d.M, d.N, d.K, d.bits, ds->cu_count,
                                      g_tile.load(std::memory_order_relaxed));
     float* ws = nullptr;
-    if (plan.workspace_bytes > 0) {
+    if (own != nullptr) {
+      ws = (float*)(own + a_bytes + r_bytes + b_bytes);
+    } else if (plan.workspace_bytes > 0) {
       std::lock_guard<std::mutex> lk(g_mu);
       const int rc = grow(&ds->ws, &ds->ws_bytes, plan.workspace_bytes);
       if (rc != LTX25_OK) { return rc; }
@@ -591,8 +604,76 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
 // dense GEMM, as in the pair: rank 448, 64 x 1024 -> 1024 67.5 us in one pass,
 // 10.4 so; rank 128, 128 x 4096 -> 4096 66.5 and 14.5; rank 200, 126 x 8192 ->
 // 2048 189 and 22.5.
+// The one-pass kernel needs no scratch (with b as it is), so calls of it may overlap
+// on several streams, be captured unprepared, and never fail for memory. The other
+// plans keep all of that: their scratch belongs to the call's stream (lora_slot), and
+// where there is none the one-pass kernel runs.
 constexpr int kLoraAheadMinK = 1536;
 constexpr int kLoraWideMinK = 512;
+
+// Bytes of lora_pair's scratch with r and the split-K partials in it
+size_t lora_few_pair_bytes(const DeviceState* ds, const void* a, const void* b, int M, int K,
+                           int N, int rank)
+{
+  const int rk = (rank + 63) & ~63;
+  const size_t ws_r = ltx25::plan_gemm(M, rk, K, 16, ds->cu_count).workspace_bytes;
+  const size_t ws_y = ltx25::plan_gemm(M, N, rk, 16, ds->cu_count,
+                                       g_tile.load(std::memory_order_relaxed)).workspace_bytes;
+  return (aligned16(a) ? 0 : align256((size_t)rk * K * 2)) + align256((size_t)M * rk * 2) +
+         (rk == rank && aligned16(b) ? 0 : align256((size_t)N * rk * 2)) +
+         (ws_r > ws_y ? ws_r : ws_y);
+}
+
+// `need` bytes of the stream's own scratch, or null: the stream is being captured (a
+// graph may replay beside later calls on it), is the per-thread one (one handle, many
+// streams), is the ninth to ask, or memory is short. Held by at most kLoraSlots streams
+// of a device, each grown by its own stream's calls. The caller holds g_lora_mu until
+// its launches are queued, so threads that share a stream do not mix theirs.
+std::mutex g_lora_mu;
+char* lora_slot(DeviceState* ds, hipStream_t st, size_t need)
+{
+  if (st == hipStreamPerThread) { return nullptr; }
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess ||
+      status != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  LoraSlot* slot = nullptr;
+  for (LoraSlot& c : ds->lora_few) {
+    if (c.used && c.stream == st) {
+      slot = &c;
+      break;
+    }
+    if (!c.used && slot == nullptr) { slot = &c; }
+  }
+  if (slot == nullptr) { return nullptr; }
+  if (slot->bytes < need) {
+    // another thread's capture is not to be ended by this one's allocation
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    bool ok = true;
+    if (slot->buf != nullptr) {
+      ok = hipStreamSynchronize(st) == hipSuccess;   // its only user
+      if (ok) {
+        (void)hipFree(slot->buf);
+        *slot = LoraSlot();
+      }
+    }
+    void* buf = nullptr;
+    ok = ok && hipMalloc(&buf, need) == hipSuccess;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    slot->used = true;
+    slot->stream = st;
+    slot->buf = buf;
+    slot->bytes = need;
+  }
+  return (char*)slot->buf;
+}
 
 // ltx25_lora_add; with `gelu`, y = bf16(gelu(bf16(y + delta))) as a GELU pass
 // after it would leave y, inside the y phase where that is the last to write y.
@@ -619,15 +700,30 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
   const bool planned =
       route == LTX25_LORA_FUSED &&
       g_lora_force.load(std::memory_order_relaxed) == LTX25_LORA_AUTO && vec && K % 64 == 0;
-  const bool wide = planned && rank >= kLoraPairMinRank && K >= kLoraWideMinK &&
-                    lora_pair_ok(M, K, N, rank, x, y);
+  bool wide = planned && rank >= kLoraPairMinRank && K >= kLoraWideMinK &&
+              lora_pair_ok(M, K, N, rank, x, y);
+  bool ahead = route == LTX25_LORA_RFIRST ||
+               (planned && !wide && rank <= ltx25::kLoraMaxRank &&
+                below_limit((size_t)M * rank8 * 2) &&
+                (K >= kLoraAheadMinK || M >= kLoraRFirstMinM));
+  const bool few = route == LTX25_LORA_FUSED && (wide || ahead);
+  const ltx25::GemmPlan r_plan = ltx25::plan_gemm(M, rank8, K, 16, ds->cu_count);
+  const size_t r_bytes = align256((size_t)M * rank8 * 2);
+  std::unique_lock<std::mutex> held(g_lora_mu, std::defer_lock);
+  char* own = nullptr;
+  if (few) {
+    held.lock();
+    own = lora_slot(ds, st, wide ? lora_few_pair_bytes(ds, a, b, M, K, N, rank)
+                                 : r_bytes + r_plan.workspace_bytes);
+    if (own == nullptr) {
+      held.unlock();
+      wide = ahead = false;
+    }
+  }
   if (route == LTX25_LORA_PAIR || wide) {
-    const int rc2 = lora_pair(ds, st, x, a, b, y, wide ? nullptr : r, M, K, N, rank);
+    const int rc2 = lora_pair(ds, st, x, a, b, y, wide ? nullptr : r, M, K, N, rank, own);
     return rc2 != LTX25_OK ? rc2 : gelu_pass();
   }
-  const bool ahead = route == LTX25_LORA_RFIRST ||
-                     (planned && rank <= ltx25::kLoraMaxRank && below_limit((size_t)M * rank8 * 2) &&
-                      (K >= kLoraAheadMinK || M >= kLoraRFirstMinM));
   const uint16_t* pa = (const uint16_t*)a;
   const uint16_t* pb = (const uint16_t*)b;
   int ldb = rank;
@@ -650,7 +746,7 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     // split of a row block. Same roundings (r rounded once to bf16).
     // r goes to the caller's buffer on the r-first route when it has one
     // ([M][rank], 16-byte aligned), else to the library's scratch
-    uint16_t* rb = route == LTX25_LORA_RFIRST ? (uint16_t*)r : nullptr;
+    uint16_t* rb = own != nullptr ? (uint16_t*)own : (uint16_t*)r;
     if (rb == nullptr || !aligned16(rb)) {
       std::lock_guard<std::mutex> lk(g_mu);
       const int rc2 = grow(&ds->lora_mm, &ds->lora_mm_bytes, (size_t)M * rank8 * 2);
@@ -667,15 +763,16 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     gd.N = rank8;
     gd.wn = rank;
     gd.K = K;
-    const ltx25::GemmPlan plan = ltx25::plan_gemm(M, rank8, K, 16, ds->cu_count);
     float* ws = nullptr;
-    if (plan.workspace_bytes > 0) {
+    if (own != nullptr) {
+      ws = (float*)(own + r_bytes);
+    } else if (r_plan.workspace_bytes > 0) {
       std::lock_guard<std::mutex> lk(g_mu);
-      const int rc2 = grow(&ds->ws, &ds->ws_bytes, plan.workspace_bytes);
+      const int rc2 = grow(&ds->ws, &ds->ws_bytes, r_plan.workspace_bytes);
       if (rc2 != LTX25_OK) { return rc2; }
       ws = (float*)ds->ws;
     }
-    hipError_t e = ltx25::launch_gemm(gd, plan, ws, st);
+    hipError_t e = ltx25::launch_gemm(gd, r_plan, ws, st);
     if (e != hipSuccess) { return hip_fail(e, "lora r gemm launch"); }
     e = ltx25::launch_lora((const uint16_t*)x, pa, pb, (uint16_t*)y, M, K, N, rank8, ldb, vec,
                            ds->cu_count, st, rb, gelu);
