@@ -350,10 +350,8 @@ int ltx25_lora_route(const void* x, const void* a, const void* b, const void* y,
  *     into the expanded weight, W' = bf16(dequant(W) + B . A), then
  *     y = epi(x . W'^T + bias) at the linear's own K
  *     ((x . A^T) . B^T = x . (B . A)^T); one rounding per weight element
- *     and one of the output;
- *   - wider adapters and w4 codes, where M is large enough for it to cost
- *     less than the form below: the same W', by a GEMM whose accumulators
- *     start from the dequantized codes;
+ *     and one of the output (what of B . A lies below its weight's bf16 ulp
+ *     is lost);
  *   - otherwise as rank-rounded-to-64 more K: y = epi([x | r] . [W | B]^T
  *     + bias), r = bf16(x . A^T), one rounding of the output;
  * where the reference rounds the linear and the delta separately.

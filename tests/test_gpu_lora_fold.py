@@ -336,62 +336,30 @@ def test_merge_boundary(pkg, dev, rank, K, bits, group, merges):
     assert np.array_equal(outs[0], outs[1]) != merges
 
 
-# Adapters that the small merge does not take (rank above 64, w4, K % 128 != 0), at enough rows
-# that merging them by a GEMM costs less than the extra K: one past and inside a tile of the
-# weight, ranks that need zero columns and ones that do not, A and B at odd addresses.
-MERGE_GEMM = [  # M, K, N, rank, bits, group, bias, epilogue, elements off 16-byte alignment
-    (8160, 4096, 520, 450, 8, 64, "bf16", 1, 0),
-    (8160, 4096, 300 * 8, 448, 8, 32, None, 0, 0),
-    (20000, 2112, 264, 450, 8, 64, "f32", 0, 3),
-    (30000, 2112, 1000, 65, 8, 32, None, 1, 1),
-    (30000, 2560, 264, 96, 4, 32, "bf16", 0, 0),
-    (20000, 4096, 776, 128, 4, 64, "f32", 1, 5),
-]
-
-
-@pytest.mark.parametrize("M,K,N,rank,bits,group,bias_kind,epi,off", MERGE_GEMM)
-def test_merge_by_a_gemm(pkg, dev, M, K, N, rank, bits, group, bias_kind, epi, off):
-    """Against the oracle's bars on sampled rows, against the same linear over W' = bf16(W + B . A)
-    in f32 on every row (only W' entries next to a rounding boundary differ: rel-L2 < 3e-4, where
-    the extra-K form's own roundings put it past 1e-3), and repeatable bit for bit."""
+# The adapter's own share of the output: x takes its values in pairs (v, -v) and each weight row
+# its columns in equal pairs, so x . W^T is zero and y is the delta alone, B . A being 2% of W. Two
+# roundings to bf16 stand between it and 64 bits, r's and the output's, half an ulp (2^-9) each;
+# the f32 sums add 1e-5. An adapter rounded together with W, as the merge up to rank 64 rounds it,
+# loses what lies below W's ulp: 8e-2 at both shapes.
+@pytest.mark.parametrize("M,K,N,rank,bits,group", [
+    (8160, 4096, 520, 450, 8, 64), (20000, 4096, 264, 128, 4, 64),
+])
+def test_a_small_delta_keeps_its_precision(pkg, dev, M, K, N, rank, bits, group):
     assert pkg.lora_fold_takes(M, K, N, rank, bits)
-    rng = np.random.default_rng(M + K + rank)
+    rng = np.random.default_rng(M + N + rank)
     g = torch.Generator(device="cuda")
-    g.manual_seed(M + N + rank)
-    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
-    qw, codes, scales, biases, wb = make_qweight(pkg, rng_normal(rng, (N, K), 0.02), bits, group)
-    ab = orc.bf16_rne(rng_normal(rng, (rank, K), 0.05))
-    bb = orc.bf16_rne(rng_normal(rng, (N, rank), 0.05))
-
-    def place(bits_u16):
-        t = torch.zeros(bits_u16.size + off + 8, dtype=torch.bfloat16, device="cuda")
-        v = t[off:off + bits_u16.size].view(bits_u16.shape)
-        v.copy_(dev_bf16(bits_u16))
-        return v
-
-    a, b = place(ab), place(bb)
-    bias = rng_normal(rng, (N,), 0.01) if bias_kind is not None else None
-    if bias_kind == "bf16":
-        bias = orc.bf16_to_f32(orc.bf16_rne(bias))
-    bd = _bias_dev(bias, bias_kind)
+    g.manual_seed(M + rank)
+    v = torch.randn((M, K // 2), device="cuda", generator=g).to(torch.bfloat16)
+    x = torch.stack((v, -v), 2).view(M, K)
+    w = np.repeat(rng_normal(rng, (N, K // 2), 0.02), 2, axis=1)
+    qw = make_qweight(pkg, w, bits, group)[0]
+    std = (0.02 * 0.02 / rank ** 0.5) ** 0.5
+    a = dev_bf16(orc.bf16_rne(rng_normal(rng, (rank, K), std)))
+    b = dev_bf16(orc.bf16_rne(rng_normal(rng, (N, rank), std)))
     y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
-    again = torch.empty_like(y)
-    say(f"lora merge GEMM M={M} K={K} N={N} rank={rank} w{bits}g{group} off={off}")
-    pkg.linear_q_lora(x, qw, bd, a, b, rank, y, M, K, N, epi)
-    pkg.linear_q_lora(x, qw, bd, a, b, rank, again, M, K, N, epi)
+    say(f"lora fold, the delta alone: M={M} K={K} N={N} rank={rank} w{bits}g{group}")
+    pkg.linear_q_lora(x, qw, None, a, b, rank, y, M, K, N)
     torch.cuda.synchronize()
-    assert torch.equal(y.view(torch.int16), again.view(torch.int16))
-    wf, _ = orc.dequant(codes, scales, biases, N, K, bits, group)
-    wm = torch.from_numpy(np.asarray(wf, np.float32).reshape(N, K)).cuda().double()
-    wm = (wm + dev_bf16(bb).double() @ dev_bf16(ab).double()).float().to(torch.bfloat16)
-    want = torch.empty_like(y)
-    pkg.linear_qc(x, pkg.dense_weight(wm), bd, want, M, K, N, epi)
-    torch.cuda.synchronize()
-    rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
-    assert rel < 3e-4, rel
-    rows = np.unique(np.linspace(0, M - 1, 24).astype(int))
-    xr = host_bits(x[torch.from_numpy(rows).cuda()])
-    ref = _oracle_rows(xr, wb, ab, bb, bias, epi, np.arange(rows.size))
-    got = orc.bf16_to_f32(host_bits(y[torch.from_numpy(rows).cuda()]))
-    assert orc.max_rel(got, ref) <= MAX_REL
-    assert orc.rel_l2(got, ref) < REL_L2_ORACLE
+    ref = torch.cat([(t.double() @ a.double().t()) @ b.double().t() for t in x.split(2048)])
+    rel = ((y.double() - ref).norm() / ref.norm()).item()
+    assert rel < 2.0 ** -8 + 1e-5, rel

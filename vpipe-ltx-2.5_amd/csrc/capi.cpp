@@ -807,16 +807,11 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
 // extra K; one rounding per weight element and one of the output. Taken up
 // to rank 64 (kMergeMaxRank): above it the merge kernel is LDS-bound and
 // the extra K costs less.
-// Every other adapter is merged by a GEMM of its own, W' = W + B . A with the
-// codes as its seeds (ltx25::launch_tall_merge), where that is expected to cost
-// less than the r GEMM, the expansion and the extra K: its work does not grow
-// with M. Rank 450, 8160 x 4096 -> 4096.
 struct FoldPlan {
   bool takes = false;
   int rk = 0;
   int bits = 0;
   bool merge = false;        // the shape allows the merge (pointers checked at run time)
-  bool merge_gemm = false;   // else: merged by a GEMM
   ltx25::GemmPlan r_plan;
   ltx25::GemmPlan plan;
   ltx25::GemmPlan merge_plan;   // the linear over W' [N][K]
@@ -854,19 +849,6 @@ FoldPlan plan_fold(int M, int K, int N, int rank, int bits, int cu_count, const 
   if (f.merge) {
     f.merge_plan = ltx25::plan_gemm(M, N, K, 16, cu_count, tile);
     f.merge = f.merge_plan.tile != 2;
-  }
-  if (!f.merge && K % 64 == 0 && below_limit((size_t)(N + 256) * rk * 2) &&
-      below_limit((size_t)(K + 256) * rk * 2) && below_limit((size_t)N * K * 2)) {
-    // expected times in us, from the figures of their kernels on a 256-CU GPU: the
-    // merge's operands (6) and its GEMM per round against r's GEMM, the wider main GEMM
-    // and the expansion. 8160 x 4096 -> 4096 at rank 450: 227 us merged, 268 as extra K;
-    // the extra K form stays where few tokens share the merge.
-    const double nk = (double)N * K, mrk = (double)M * rk;
-    const double rounds = (double)(((long)((N + 255) / 256) * ((K + 255) / 256) + cu_count - 1) / cu_count);
-    const double merge_us = 10.0 + rounds * (12.0 + 1.2 * rk / 64);
-    const double extra_us = 8.0 + 2.0 * mrk * K / 0.8e9 + 2.0 * mrk * N / 1.3e9 + nk * 3.0 / 5.0e6;
-    f.merge_plan = ltx25::plan_gemm(M, N, K, 16, cu_count, tile);
-    f.merge_gemm = merge_us < extra_us && f.merge_plan.tile != 2;
   }
   f.rk = rk;
   f.bits = bits;
@@ -913,53 +895,6 @@ int run_fold(DeviceState* ds, hipStream_t st, const FoldPlan& f, const void* x,
         w->group, (const uint16_t*)a, pad_b ? bp : (const uint16_t*)b, rank,
         pad_b ? rank8 : rank, wd, N, K, st);
     if (e != hipSuccess) { return hip_fail(e, "fold: merge launch"); }
-    ltx25::GemmDesc d;
-    d.x = (const uint16_t*)x;
-    d.w = wd;
-    d.bits = 16;
-    d.group = 64;
-    d.bias = bias;
-    d.bias_type = bias != nullptr ? bias_dtype : ltx25::kBiasNone;
-    d.epilogue = epilogue;
-    d.y = (uint16_t*)y;
-    d.M = M;
-    d.N = N;
-    d.K = K;
-    e = ltx25::launch_gemm(d, f.merge_plan, ws, st);
-    if (e != hipSuccess) { return hip_fail(e, "fold: gemm launch"); }
-    return LTX25_OK;
-  }
-  if (f.merge_gemm) {
-    // at = A^T and B, both padded to rk columns, W' = bf16(W + B . A), then the
-    // linear over W'
-    const int rk = f.rk;
-    const size_t at_bytes = align256((size_t)K * rk * 2);
-    const bool pad_b = rk != rank || !aligned16(b);
-    uint16_t* wd = nullptr;
-    char* base = nullptr;
-    float* ws = nullptr;
-    {
-      std::lock_guard<std::mutex> lk(g_mu);
-      int rc = grow(&ds->deq, &ds->deq_bytes, (size_t)N * K * 2);
-      if (rc != LTX25_OK) { return rc; }
-      rc = grow(&ds->lora_mm, &ds->lora_mm_bytes, at_bytes + (pad_b ? (size_t)N * rk * 2 : 0));
-      if (rc != LTX25_OK) { return rc; }
-      if (f.merge_plan.workspace_bytes > 0) {
-        rc = grow(&ds->ws, &ds->ws_bytes, f.merge_plan.workspace_bytes);
-        if (rc != LTX25_OK) { return rc; }
-        ws = (float*)ds->ws;
-      }
-      wd = (uint16_t*)ds->deq;
-      base = (char*)ds->lora_mm;
-    }
-    uint16_t* const bp = pad_b ? (uint16_t*)(base + at_bytes) : nullptr;
-    hipError_t e = ltx25::launch_lora_operands((const uint16_t*)a, (const uint16_t*)b, rank, K, N,
-                                               (uint16_t*)base, bp, rk, st);
-    if (e != hipSuccess) { return hip_fail(e, "fold: merge operands launch"); }
-    const uint16_t* const pb = pad_b ? bp : (const uint16_t*)b;
-    e = ltx25::launch_tall_merge(w->codes, (const uint16_t*)w->scales, (const uint16_t*)w->qbias,
-                                 w->bits, w->group, pb, (const uint16_t*)base, rk, wd, N, K, st);
-    if (e != hipSuccess) { return hip_fail(e, "fold: merge gemm launch"); }
     ltx25::GemmDesc d;
     d.x = (const uint16_t*)x;
     d.w = wd;

@@ -180,13 +180,6 @@ bool tall_w8_takes(const GemmDesc& d, const GemmPlan& plan);
 // of 256-row tiles that would leave CUs idle goes out as 128-row ones.
 hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm = 256,
                              int cu_count = 0, unsigned long long* stamps = nullptr);
-// The dequant-once expansion with an adapter of any rank merged in, as a GEMM
-// on the same tile: out [N][K] = bf16(fma(scale, code, zero point) + b . at^T), b
-// bf16 [N][rk], at (A transposed) bf16 [K][rk], rk a multiple of 64; bits 8 or
-// 4, group 64 or 32, K % 64 == 0, 16-byte aligned codes, b, at and out.
-hipError_t launch_tall_merge(const void* codes, const uint16_t* scales, const uint16_t* qbias,
-                             int bits, int group, const uint16_t* b, const uint16_t* at, int rk,
-                             uint16_t* out, int N, int K, hipStream_t stream);
 // The int8 tier's GEMM on the same tile (tall.hip, v_mfma_i32_16x16x64_i8):
 // N % 8 == 0, K a multiple of 128. launch_i8_gemm routes there, with 256- or
 // 128-row tiles, where tall_rows says so and it takes the shape.
@@ -227,11 +220,6 @@ hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
 // folded linear's weight tail.
 hipError_t launch_lora_pad(const uint16_t* src, int rows, int cols, int ld_src, uint16_t* dst,
                            int ld_dst, hipStream_t stream, int width = 0);
-// launch_tall_merge's operands: A [rank][K] -> at [K][rk] and, unless bp is null, B
-// [N][rank] -> bp [N][rk], zeros past `rank` (rk a multiple of 64, K % 64 == 0, A and B
-// at any 2-byte alignment).
-hipError_t launch_lora_operands(const uint16_t* a, const uint16_t* b, int rank, int K, int N,
-                                uint16_t* at, uint16_t* bp, int rk, hipStream_t stream);
 // The dequant-once expansion with the adapter merged in (lora.hip):
 // out [N][K] = bf16(fma(scale, code, zero point) + B . A), A bf16
 // [rank][K], B bf16 [N][ldb] (columns from rank to ldb zero).

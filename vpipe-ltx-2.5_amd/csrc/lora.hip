@@ -427,49 +427,6 @@ __global__ void lora_pad_kernel(const uint16_t* __restrict__ src, int rows, int 
   *(uint4*)(dst + r * (size_t)ld_dst + c) = v;
 }
 
-// The merge GEMM's operands in one launch. The first a_tiles workgroups: at[k][i] =
-// i < rank ? a[i][k] : 0 for i < rk, a 64 x 64 tile each, through LDS so that both
-// sides move whole 128-byte rows. The others: bp[n][i] = i < rank ? b[n][i] : 0, 64
-// rows of 64 columns each. All loads of a thread go out before its first use.
-__global__ void __launch_bounds__(256)
-lora_operands_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, int rank,
-                     int K, int N, uint16_t* __restrict__ at, uint16_t* __restrict__ bp, int rk,
-                     int a_tiles)
-{
-  __shared__ uint16_t tile[64][66];
-  const int c = threadIdx.x & 63;
-  const int r0 = threadIdx.x >> 6;
-  const int across = rk / 64;
-  const bool of_a = (int)blockIdx.x < a_tiles;
-  const int t = of_a ? (int)blockIdx.x : (int)blockIdx.x - a_tiles;
-  const int i0 = t % across * 64;
-  const int o0 = t / across * 64;   // first k, or first n
-  // clamped, not branched around: a load under a branch is waited for there
-  uint16_t v[16];
-  if (!of_a) {
-    const int i = min(i0 + c, rank - 1);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { v[r] = b[(size_t)min(o0 + 4 * r + r0, N - 1) * rank + i]; }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int n = o0 + 4 * r + r0;
-      if (n < N) { bp[(size_t)n * rk + i0 + c] = i0 + c < rank ? v[r] : (uint16_t)0; }
-    }
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) { v[r] = a[(size_t)min(i0 + 4 * r + r0, rank - 1) * K + o0 + c]; }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    tile[4 * r + r0][c] = i0 + 4 * r + r0 < rank ? v[r] : (uint16_t)0;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    at[(size_t)(o0 + 4 * r + r0) * rk + i0 + c] = tile[c][4 * r + r0];
-  }
-}
-
 // ---- the adapter merged into the dequant-once expansion ----------------
 //   W'[n][k] = bf16(fma(scale, code, zero point) + sum_{i < rank} B[n][i] A[i][k])
 // The linear then runs over W' at its own K. (x . A^T) . B^T = x . (B . A)^T,
@@ -687,19 +644,6 @@ hipError_t launch_dequant_merge(const uint8_t* codes, const uint16_t* scales,
   } else {
     go(std::integral_constant<int, 64>{});
   }
-  return hipGetLastError();
-}
-
-hipError_t launch_lora_operands(const uint16_t* a, const uint16_t* b, int rank, int K, int N,
-                                uint16_t* at, uint16_t* bp, int rk, hipStream_t stream)
-{
-  if (rank < 1 || rk < rank || rk % 64 != 0 || K < 64 || K % 64 != 0 || N < 1) {
-    return hipErrorInvalidValue;
-  }
-  const int a_tiles = K / 64 * (rk / 64);
-  const int b_tiles = bp != nullptr ? (N + 63) / 64 * (rk / 64) : 0;
-  lora_operands_kernel<<<(unsigned)(a_tiles + b_tiles), 256, 0, stream>>>(a, b, rank, K, N, at, bp,
-                                                                          rk, a_tiles);
   return hipGetLastError();
 }
 

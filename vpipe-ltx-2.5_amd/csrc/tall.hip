@@ -14,8 +14,7 @@
 //     bit for bit (tall_w8_kernel, below).
 // tall_kernel is also instantiated with 128 rows (the same schedule, half the rows
 // per group), for outputs below a round of 256 x 256 tiles and for a poorly filled
-// last round, and with accumulators that start from a weight's codes (the wide
-// adapter merged into the expansion).
+// last round.
 //
 // bf16 and int8: tall_kernel, an 8-wave ping-pong schedule.
 //   - Waves 0-3 (group 0) own output rows 0..127, waves 4-7 (group 1) rows
@@ -88,10 +87,9 @@ struct TallParams {
   const float* sx;         // int8 mode: per-row activation scales
   const float* sw;         // int8 mode: per-column weight scales
   int32_t* acc_out;        // int8 mode, optional: the raw int32 accumulators
-  const uint16_t* scales;  // w8 mode: bf16 [N][K / group]; SEED: [M][N / group]
-  const uint16_t* qbias;   // w8 mode: bf16 [N][K / group]; SEED: [M][N / group]
-  int gshift, gcols;       // w8 mode and SEED: log2(group), groups per row
-  const void* codes;       // SEED: the codes [M][N] the accumulators start from
+  const uint16_t* scales;  // w8 mode: bf16 [N][K / group]
+  const uint16_t* qbias;   // w8 mode: bf16 [N][K / group]
+  int gshift, gcols;       // w8 mode: log2(group), K / group
   uint16_t* y;
   const uint16_t* y_in;    // bf16 mode without x2, optional: the accumulators start from it
   int M, N, K;             // K in elements
@@ -168,9 +166,8 @@ static_assert(kPPLds == 160 * 1024, "the stages fill the LDS");
 static_assert(kBM * kEP * 2 <= kPPLds, "the staged tile fits the stages");
 
 // BM: rows of the tile, 256 or 128. The 128 x 256 tile is the same schedule with
-// half the rows per group. SEED (8 or 4): the accumulators start from a weight's
-// codes (the adapter merged into the expansion, launch_tall_merge).
-template <int MODE, bool FOLD, bool STAMPS = false, int BM = kBM, int SEED = 0>
+// half the rows per group.
+template <int MODE, bool FOLD, bool STAMPS = false, int BM = kBM>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 tall_kernel(TallParams p)
 {
@@ -305,75 +302,7 @@ tall_kernel(TallParams p)
   // K loop adds the products to it and the epilogue rounds once, as the
   // template tile does. The loads are issued before any operand load, so
   // the hand-counted vmcnt waits below only ever wait longer for them.
-  if constexpr (SEED != 0) {
-    // The output is a weight: its codes dequantized in the accumulators' layout,
-    // w = fma(scale, code, zero point). A lane needs, of block j, the quad of
-    // columns that its 16-lane row q = lane / 16 names; it loads the 16 codes of
-    // block q, so that a load covers 16 whole 64-code (w8) or 32-byte (w4) runs, and
-    // the four rows exchange quads (a 4 x 4 transpose of dwords by row swaps).
-    // The 4096 x 4096 merge at rank 450 takes 35 us so; loaded quad by quad, 16
-    // bytes of 16 rows an instruction, 39.
-    static_assert(MODE == kModeBf16 && !FOLD && !STAMPS, "the merge is the plain bf16 mode");
-    const int lrow = lane & 15;
-    const int lcol = (lane >> 4) * 4;
-    const uint32_t code_row = (uint32_t)((size_t)p.N * SEED / 8);
-    const __amdgpu_buffer_rsrc_t cr = make_rsrc(p.codes, (size_t)p.M * code_row);
-    const __amdgpu_buffer_rsrc_t sr = make_rsrc(p.scales, (size_t)p.M * p.gcols * 2);
-    const __amdgpu_buffer_rsrc_t zr = make_rsrc(p.qbias, (size_t)p.M * p.gcols * 2);
-    typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
-    uint32_t cv[kNI][4], sv[kNI][2], zv[kNI][2];
-#pragma unroll
-    for (int i = 0; i < kNI; ++i) {
-      const uint32_t m = (uint32_t)(m0 + g * kGR + i * 16 + lrow);
-      const uint32_t off = m * code_row + (uint32_t)(n0 + wn * 64 + lcol * 4) * SEED / 8;
-      if constexpr (SEED == 8) {
-        const i32x4v v = __builtin_amdgcn_raw_buffer_load_b128(cr, (int)off, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { cv[i][j] = (uint32_t)v[j]; }
-      } else {
-        const u32x2v v =
-            __builtin_bit_cast(u32x2v, __builtin_amdgcn_raw_buffer_load_b64(cr, (int)off, 0, 0));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { cv[i][j] = (v[j >> 1] >> (16 * (j & 1))) & 0xffffu; }
-      }
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        // the wave's columns 32 q .. 32 q + 31 are in one group
-        const uint32_t off =
-            (m * (uint32_t)p.gcols + ((uint32_t)(n0 + wn * 64 + 32 * q) >> p.gshift)) * 2u;
-        sv[i][q] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)off, 0, 0);
-        zv[i][q] = __builtin_amdgcn_raw_buffer_load_b16(zr, (int)off, 0, 0);
-      }
-    }
-    // rows 2, 3 of the first against rows 0, 1 of the second; then rows 1, 3 against 0, 2
-    auto swap32 = [](uint32_t& a, uint32_t& b) {
-      const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-      a = r[0];
-      b = r[1];
-    };
-    auto swap16 = [](uint32_t& a, uint32_t& b) {
-      const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-      a = r[0];
-      b = r[1];
-    };
-#pragma unroll
-    for (int i = 0; i < kNI; ++i) {
-      swap32(cv[i][0], cv[i][2]);
-      swap32(cv[i][1], cv[i][3]);
-      swap16(cv[i][0], cv[i][1]);
-      swap16(cv[i][2], cv[i][3]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float sc = __uint_as_float(sv[i][j >> 1] << 16);
-        const float zp = __uint_as_float(zv[i][j >> 1] << 16);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          acc[i][j][t] =
-              fmaf(sc, (float)((cv[i][j] >> (SEED * t)) & ((1u << SEED) - 1u)), zp);
-        }
-      }
-    }
-  } else if constexpr (!I8 && !FOLD) {
+  if constexpr (!I8 && !FOLD) {
     if (p.y_in != nullptr) {
       const int lrow = lane & 15;
       const int lcol = (lane >> 4) * 4;
@@ -1110,49 +1039,6 @@ hipError_t launch_tall_dense(const GemmDesc& d, hipStream_t stream, int bm, int 
   p.stamps = stamps;
   return bm == kBM && stamps == nullptr ? launch_rounds(p, kModeBf16, cu_count, stream)
                                         : launch_tall(p, kModeBf16, bm, stream);
-}
-
-hipError_t launch_tall_merge(const void* codes, const uint16_t* scales, const uint16_t* qbias,
-                             int bits, int group, const uint16_t* b, const uint16_t* at, int rk,
-                             uint16_t* out, int N, int K, hipStream_t stream)
-{
-  if ((bits != 8 && bits != 4) || (group != 64 && group != 32) || N < 1 || K < kBK ||
-      K % kBK != 0 || rk < kBK || rk % kBK != 0 || (size_t)(N + kBM) * rk * 2 >= kTwoGib ||
-      (size_t)(K + kBN) * rk * 2 >= kTwoGib || (size_t)(N + kBM) * K * 2 >= kFourGib ||
-      (size_t)N * K * 2 >= kTwoGib) {
-    return hipErrorInvalidValue;
-  }
-  TallParams p = {};
-  p.x = b;
-  p.w = at;
-  p.codes = codes;
-  p.scales = scales;
-  p.qbias = qbias;
-  p.gshift = group == 64 ? 6 : 5;
-  p.gcols = K / group;
-  p.y = out;
-  p.M = N;
-  p.N = K;
-  p.K = rk;
-  p.kx = rk;
-  p.wn = K;
-  p.bias_type = kBiasNone;
-  p.epilogue = kEpiNone;
-  p.tiles_n = (K + kBN - 1) / kBN;
-  // Half tiles while they all fit one round of a 256-CU GPU: the seeds' loads and
-  // the stores, not the few K steps, are most of a tile's time.
-  const int rows = (N + 127) / 128 * p.tiles_n <= 256 ? 128 : 256;
-  p.tiles_m = (N + rows - 1) / rows;
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
-  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, p); };
-  if (bits == 8) {
-    rows == 128 ? go(tall_kernel<kModeBf16, false, false, 128, 8>)
-                : go(tall_kernel<kModeBf16, false, false, 256, 8>);
-  } else {
-    rows == 128 ? go(tall_kernel<kModeBf16, false, false, 128, 4>)
-                : go(tall_kernel<kModeBf16, false, false, 256, 4>);
-  }
-  return hipGetLastError();
 }
 
 bool tall_i8_takes(int M, int N, int K)
