@@ -1,0 +1,178 @@
+// ltx25_lora_add's host side on a CPU: this program stands in for the HIP runtime calls and the
+// kernel launchers that the library makes (its definitions come first in the symbol search), so
+// that what a call allocates, launches and hands to a launch can be seen without a GPU. The
+// planners are the library's own.
+//
+//   lora_scratch SCENARIO [ARGS]    exits 0 and prints nothing, or says what is wrong
+#include "common.h"
+#include "ltx25_qlinear.h"
+
+#include <dlfcn.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <set>
+#include <string>
+#include <vector>
+
+namespace {
+
+int g_failures = 0;
+
+#define EXPECT(cond, ...)              \
+  do {                                 \
+    if (!(cond)) {                     \
+      ++g_failures;                    \
+      std::printf("line %d: ", __LINE__); \
+      std::printf(__VA_ARGS__);        \
+      std::printf("\n");               \
+    }                                  \
+  } while (0)
+
+// ---- device memory: addresses only, never touched ----
+std::map<uintptr_t, size_t> g_mem;
+uintptr_t g_next = (uintptr_t)1 << 44;
+int g_mallocs = 0, g_device_syncs = 0;
+
+// The bytes left in the allocation that holds p, 0 outside of all
+size_t room(const void* p)
+{
+  auto it = g_mem.upper_bound((uintptr_t)p);
+  if (it == g_mem.begin()) { return 0; }
+  --it;
+  const uintptr_t end = it->first + it->second;
+  return (uintptr_t)p < end ? end - (uintptr_t)p : 0;
+}
+
+// ---- launches ----
+struct Launch {
+  std::string what;
+  hipStream_t stream;
+  std::vector<std::pair<uintptr_t, size_t>> scratch;   // library scratch it reads or writes
+};
+std::vector<Launch> g_launches;
+
+void note(const char* what, hipStream_t st, std::initializer_list<std::pair<const void*, size_t>> use)
+{
+  Launch l{what, st, {}};
+  for (const auto& u : use) {
+    if (u.first == nullptr || u.second == 0 || room(u.first) == 0) { continue; }   // the caller's
+    EXPECT(room(u.first) >= u.second, "%s: %zu bytes at %p, %zu allocated", what, u.second,
+           u.first, room(u.first));
+    l.scratch.push_back({(uintptr_t)u.first, u.second});
+  }
+  g_launches.push_back(l);
+}
+
+int g_plans = 0;                       // made by the present call
+int g_set_after = 0, g_set_tile = 0;   // another thread sets the tile after that many of them
+
+}  // namespace
+
+// ---- the HIP runtime ----
+extern "C" {
+
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int)
+{
+  std::memset(p, 0, sizeof *p);
+  std::strcpy(p->gcnArchName, "gfx950");
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipMalloc(void** p, size_t n)
+{
+  ++g_mallocs;
+  *p = (void*)g_next;
+  g_mem[g_next] = n;
+  g_next += (n + 0xffff) & ~(size_t)0xffff;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) { return g_mem.erase((uintptr_t)p) ? hipSuccess : hipErrorInvalidValue; }
+hipError_t hipDeviceSynchronize() { ++g_device_syncs; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
+{
+  *s = hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
+
+}  // extern "C"
+
+// ---- the kernels' launchers ----
+namespace ltx25 {
+
+GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force, bool panels)
+{
+  using Fn = GemmPlan (*)(int, int, int, int, int, int, bool);
+  static const Fn real = (Fn)dlsym(RTLD_NEXT, "_ZN5ltx259plan_gemmEiiiiiib");
+  if (real == nullptr) { std::printf("no planner in the library\n"); std::exit(2); }
+  const GemmPlan p = real(M, N, K, bits, cu_count, force, panels);
+  if (++g_plans == g_set_after) { ltx25_set_tile(g_set_tile); }
+  return p;
+}
+
+hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan, float* ws, hipStream_t st)
+{
+  EXPECT(plan.workspace_bytes == 0 || room(ws) >= plan.workspace_bytes,
+         "GEMM %d x %d -> %d: %zu bytes of partials, %zu at %p", d.M, d.K, d.N,
+         plan.workspace_bytes, room(ws), (void*)ws);
+  note("gemm", st, {{ws, plan.workspace_bytes}, {d.x, (size_t)d.M * d.K * 2},
+                    {d.w, (size_t)(d.wn > 0 ? d.wn : d.N) * d.K * 2}, {d.y, (size_t)d.M * d.N * 2}});
+  return hipSuccess;
+}
+
+hipError_t launch_lora(const uint16_t*, const uint16_t*, const uint16_t* b, uint16_t*, int M, int,
+                       int N, int rank, int ldb, bool, int, hipStream_t st, const uint16_t* r_in,
+                       bool)
+{
+  note(r_in != nullptr ? "lora y" : "lora", st,
+       {{b, ((size_t)(N - 1) * ldb + rank) * 2}, {r_in, (size_t)M * rank * 2}});
+  return hipSuccess;
+}
+
+hipError_t launch_lora_pad(const uint16_t*, int rows, int, int, uint16_t* dst, int ld_dst,
+                           hipStream_t st, int)
+{
+  note("pad", st, {{dst, (size_t)rows * ld_dst * 2}});
+  return hipSuccess;
+}
+
+}  // namespace ltx25
+
+namespace {
+
+// A call's operands: four addresses that no allocation holds
+int add(hipStream_t st, int M, int K, int N, int rank, int b_off = 0)
+{
+  char* const x = (char*)((uintptr_t)1 << 40);
+  return ltx25_lora_add(st, x, x + (1 << 30), x + (2ul << 30) + b_off, x + (3ul << 30), nullptr,
+                        nullptr, M, K, N, rank);
+}
+
+// The tile switch changes after the call's n-th plan: what runs fits what was reserved for it, also
+// where the y GEMM splits K under one setting and not under the other.
+void tile_switch(int rank, int from, int to, int n)
+{
+  ltx25_set_tile(from);
+  g_set_after = n;
+  g_set_tile = to;
+  EXPECT(add((hipStream_t)0x1000, 128, 2048, 16384, rank) == LTX25_OK, "%s", ltx25_last_error());
+  EXPECT(!g_launches.empty() && g_launches.back().what == "gemm", "not the GEMM pair");
+}
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+  const std::string s = argc > 1 ? argv[1] : "";
+  auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
+  if (s == "tile_switch") { tile_switch(arg(2), arg(3), arg(4), arg(5)); }
+  else { std::printf("unknown scenario %s\n", s.c_str()); return 2; }
+  return g_failures == 0 ? 0 : 1;
+}

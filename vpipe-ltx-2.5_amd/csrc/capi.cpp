@@ -516,30 +516,56 @@ int lora_route(int M, int K, int N, int rank, const void* x, const void* a, cons
   return LTX25_LORA_FUSED;
 }
 
-// `own`: scratch of the call's own (lora_few_pair_bytes) instead of the library's.
-int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, const void* b,
-              void* y, void* r_caller, int M, int K, int N, int rank, char* own = nullptr)
+// The pair's GEMM plans and scratch, A padded | r | B padded | split-K partials.
+// Made once per call, so that the plans which run are those the scratch was
+// sized for: the tile switch may change between two reads of it.
+struct LoraPairPlan {
+  int rk = 0;
+  bool pad_a = false, pad_b = false, own_r = false;
+  size_t a_bytes = 0, r_bytes = 0, b_bytes = 0, ws_bytes = 0;
+  ltx25::GemmPlan r_plan, y_plan;
+  size_t operand_bytes() const { return a_bytes + r_bytes + b_bytes; }
+};
+
+LoraPairPlan plan_lora_pair(const DeviceState* ds, const void* a, const void* b,
+                            const void* r_caller, int M, int K, int N, int rank)
 {
-  const int rk = (rank + 63) & ~63;
+  LoraPairPlan p;
+  p.rk = (rank + 63) & ~63;
   // A's rows past `rank` read as zeros (the GEMM's weight-row bound), so A
   // is copied only when it is not 16-byte aligned; B gets zero columns up
   // to rk. The caller's r ([M][rank]) holds r when it has rk columns.
-  const ltx25::GemmPlan r_plan = ltx25::plan_gemm(M, rk, K, 16, ds->cu_count);
-  const bool pad_a = !aligned16(a);
-  const bool pad_b = rk != rank || !aligned16(b);
-  const bool own_r = r_caller == nullptr || rk != rank || !aligned16(r_caller);
-  const size_t a_bytes = pad_a ? align256((size_t)rk * K * 2) : 0;
-  const size_t r_bytes = own_r ? align256((size_t)M * rk * 2) : 0;
-  const size_t b_bytes = pad_b ? align256((size_t)N * rk * 2) : 0;
+  p.pad_a = !aligned16(a);
+  p.pad_b = p.rk != rank || !aligned16(b);
+  p.own_r = r_caller == nullptr || p.rk != rank || !aligned16(r_caller);
+  p.a_bytes = p.pad_a ? align256((size_t)p.rk * K * 2) : 0;
+  p.r_bytes = p.own_r ? align256((size_t)M * p.rk * 2) : 0;
+  p.b_bytes = p.pad_b ? align256((size_t)N * p.rk * 2) : 0;
+  p.r_plan = ltx25::plan_gemm(M, p.rk, K, 16, ds->cu_count);
+  p.y_plan = ltx25::plan_gemm(M, N, p.rk, 16, ds->cu_count,
+                              g_tile.load(std::memory_order_relaxed));
+  p.ws_bytes = std::max(p.r_plan.workspace_bytes, p.y_plan.workspace_bytes);
+  return p;
+}
+
+// `own`: p.operand_bytes() + p.ws_bytes of the call's own, instead of the
+// library's scratch.
+int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void* x,
+              const void* a, const void* b, void* y, void* r_caller, int M, int K, int N, int rank,
+              char* own = nullptr)
+{
+  const int rk = p.rk;
+  const bool pad_a = p.pad_a, pad_b = p.pad_b;
+  const size_t a_bytes = p.a_bytes, r_bytes = p.r_bytes;
   char* base = own;
-  if (own == nullptr && a_bytes + r_bytes + b_bytes > 0) {
+  if (own == nullptr && p.operand_bytes() > 0) {
     std::lock_guard<std::mutex> lk(g_mu);
-    const int rc = grow(&ds->lora_mm, &ds->lora_mm_bytes, a_bytes + r_bytes + b_bytes);
+    const int rc = grow(&ds->lora_mm, &ds->lora_mm_bytes, p.operand_bytes());
     if (rc != LTX25_OK) { return rc; }
     base = (char*)ds->lora_mm;
   }
   const uint16_t* pa = (const uint16_t*)a;
-  uint16_t* pr = own_r ? (uint16_t*)(base + a_bytes) : (uint16_t*)r_caller;
+  uint16_t* pr = p.own_r ? (uint16_t*)(base + a_bytes) : (uint16_t*)r_caller;
   const uint16_t* pb = (const uint16_t*)b;
   if (pad_a) {
     // A [rank][K] -> [rk][K]: one row of rank*K elements, zero-filled to rk*K
@@ -574,13 +600,10 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
       d.N = N;
       d.K = rk;
     }
-    const ltx25::GemmPlan plan =
-        half == 0 ? r_plan
-                  : ltx25::plan_gemm(d.M, d.N, d.K, d.bits, ds->cu_count,
-                                     g_tile.load(std::memory_order_relaxed));
+    const ltx25::GemmPlan& plan = half == 0 ? p.r_plan : p.y_plan;
     float* ws = nullptr;
     if (own != nullptr) {
-      ws = (float*)(own + a_bytes + r_bytes + b_bytes);
+      ws = (float*)(own + p.operand_bytes());
     } else if (plan.workspace_bytes > 0) {
       std::lock_guard<std::mutex> lk(g_mu);
       const int rc = grow(&ds->ws, &ds->ws_bytes, plan.workspace_bytes);
@@ -610,19 +633,6 @@ int lora_pair(DeviceState* ds, hipStream_t st, const void* x, const void* a, con
 // where there is none the one-pass kernel runs.
 constexpr int kLoraAheadMinK = 1536;
 constexpr int kLoraWideMinK = 512;
-
-// Bytes of lora_pair's scratch with r and the split-K partials in it
-size_t lora_few_pair_bytes(const DeviceState* ds, const void* a, const void* b, int M, int K,
-                           int N, int rank)
-{
-  const int rk = (rank + 63) & ~63;
-  const size_t ws_r = ltx25::plan_gemm(M, rk, K, 16, ds->cu_count).workspace_bytes;
-  const size_t ws_y = ltx25::plan_gemm(M, N, rk, 16, ds->cu_count,
-                                       g_tile.load(std::memory_order_relaxed)).workspace_bytes;
-  return (aligned16(a) ? 0 : align256((size_t)rk * K * 2)) + align256((size_t)M * rk * 2) +
-         (rk == rank && aligned16(b) ? 0 : align256((size_t)N * rk * 2)) +
-         (ws_r > ws_y ? ws_r : ws_y);
-}
 
 // `need` bytes of the stream's own scratch, or null: the stream is being captured (a
 // graph may replay beside later calls on it), is the per-thread one (one handle, many
@@ -709,11 +719,15 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
   const bool few = route == LTX25_LORA_FUSED && (wide || ahead);
   const ltx25::GemmPlan r_plan = ltx25::plan_gemm(M, rank8, K, 16, ds->cu_count);
   const size_t r_bytes = align256((size_t)M * rank8 * 2);
+  LoraPairPlan pair;
+  if (route == LTX25_LORA_PAIR || wide) {
+    pair = plan_lora_pair(ds, a, b, wide ? nullptr : r, M, K, N, rank);
+  }
   std::unique_lock<std::mutex> held(g_lora_mu, std::defer_lock);
   char* own = nullptr;
   if (few) {
     held.lock();
-    own = lora_slot(ds, st, wide ? lora_few_pair_bytes(ds, a, b, M, K, N, rank)
+    own = lora_slot(ds, st, wide ? pair.operand_bytes() + pair.ws_bytes
                                  : r_bytes + r_plan.workspace_bytes);
     if (own == nullptr) {
       held.unlock();
@@ -721,7 +735,7 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     }
   }
   if (route == LTX25_LORA_PAIR || wide) {
-    const int rc2 = lora_pair(ds, st, x, a, b, y, wide ? nullptr : r, M, K, N, rank, own);
+    const int rc2 = lora_pair(ds, st, pair, x, a, b, y, wide ? nullptr : r, M, K, N, rank, own);
     return rc2 != LTX25_OK ? rc2 : gelu_pass();
   }
   const uint16_t* pa = (const uint16_t*)a;
