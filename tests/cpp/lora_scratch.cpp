@@ -166,6 +166,30 @@ void tile_switch(int rank, int from, int to, int n)
   EXPECT(!g_launches.empty() && g_launches.back().what == "gemm", "not the GEMM pair");
 }
 
+// Calls on several streams at once: no two of them use the same bytes of scratch.
+void overlap(int M, int K, int N, int rank, int b_off)
+{
+  for (int i = 0; i < 3; ++i) {
+    for (int s = 1; s <= 4; ++s) {
+      EXPECT(add((hipStream_t)(uintptr_t)(0x1000 * s), M, K, N, rank, b_off) == LTX25_OK, "%s",
+             ltx25_last_error());
+    }
+  }
+  EXPECT(g_launches.size() > 12, "the one-pass kernel alone");
+  for (const Launch& l : g_launches) {
+    for (const Launch& o : g_launches) {
+      if (l.stream == o.stream) { continue; }
+      for (const auto& p : l.scratch) {
+        for (const auto& q : o.scratch) {
+          EXPECT(p.first + p.second <= q.first || q.first + q.second <= p.first,
+                 "%s of one stream and %s of another share scratch", l.what.c_str(),
+                 o.what.c_str());
+        }
+      }
+    }
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -173,6 +197,7 @@ int main(int argc, char** argv)
   const std::string s = argc > 1 ? argv[1] : "";
   auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
   if (s == "tile_switch") { tile_switch(arg(2), arg(3), arg(4), arg(5)); }
+  else if (s == "overlap") { overlap(arg(2), arg(3), arg(4), arg(5), arg(6)); }
   else { std::printf("unknown scenario %s\n", s.c_str()); return 2; }
   return g_failures == 0 ? 0 : 1;
 }

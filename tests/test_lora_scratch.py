@@ -37,3 +37,16 @@ def run(exe, *args):
 def test_the_tile_switch_may_change_during_a_call(exe, rank, before, after):
     for n in range(1, 7):   # after the call's n-th plan
         run(exe, "tile_switch", rank, before, after, n)
+
+
+# the plans under the fused route: r ahead of the y phase, both products on the dense GEMM; ranks
+# and addresses of b that the kernels read as they are, and that need a copy
+PLANS = [  # M, K, N, rank, bytes of b off 16-byte alignment
+    (128, 4096, 1032, 32, 0), (128, 4096, 1032, 32, 2), (128, 2048, 1032, 12, 0),
+    (33, 2048, 4104, 17, 0), (64, 1024, 1024, 450, 0), (100, 2048, 1000, 192, 6),
+]
+
+
+@pytest.mark.parametrize("M,K,N,rank,b_off", PLANS)
+def test_streams_share_no_scratch(exe, M, K, N, rank, b_off):
+    run(exe, "overlap", M, K, N, rank, b_off)

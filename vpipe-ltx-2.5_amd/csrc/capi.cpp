@@ -627,10 +627,11 @@ int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void
 // dense GEMM, as in the pair: rank 448, 64 x 1024 -> 1024 67.5 us in one pass,
 // 10.4 so; rank 128, 128 x 4096 -> 4096 66.5 and 14.5; rank 200, 126 x 8192 ->
 // 2048 189 and 22.5.
-// The one-pass kernel needs no scratch (with b as it is), so calls of it may overlap
-// on several streams, be captured unprepared, and never fail for memory. The other
-// plans keep all of that: their scratch belongs to the call's stream (lora_slot), and
-// where there is none the one-pass kernel runs.
+// The one-pass kernel needs no scratch where it reads b as it is (rank % 8 == 0, b
+// 16-byte aligned): such calls may overlap on several streams, be captured
+// unprepared, and never fail for memory. The other plans keep all of that: their
+// scratch, a padded copy of b included, belongs to the call's stream (lora_slot),
+// and where there is none the one-pass kernel runs.
 constexpr int kLoraAheadMinK = 1536;
 constexpr int kLoraWideMinK = 512;
 
@@ -717,8 +718,10 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
                 below_limit((size_t)M * rank8 * 2) &&
                 (K >= kLoraAheadMinK || M >= kLoraRFirstMinM));
   const bool few = route == LTX25_LORA_FUSED && (wide || ahead);
+  const bool pad_b = vec && (rank != rank8 || !aligned16(b));
   const ltx25::GemmPlan r_plan = ltx25::plan_gemm(M, rank8, K, 16, ds->cu_count);
   const size_t r_bytes = align256((size_t)M * rank8 * 2);
+  const size_t b_bytes = pad_b ? align256((size_t)N * rank8 * 2) : 0;
   LoraPairPlan pair;
   if (route == LTX25_LORA_PAIR || wide) {
     pair = plan_lora_pair(ds, a, b, wide ? nullptr : r, M, K, N, rank);
@@ -728,7 +731,7 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
   if (few) {
     held.lock();
     own = lora_slot(ds, st, wide ? pair.operand_bytes() + pair.ws_bytes
-                                 : r_bytes + r_plan.workspace_bytes);
+                                 : r_bytes + b_bytes + r_plan.workspace_bytes);
     if (own == nullptr) {
       held.unlock();
       wide = ahead = false;
@@ -741,16 +744,17 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
   const uint16_t* pa = (const uint16_t*)a;
   const uint16_t* pb = (const uint16_t*)b;
   int ldb = rank;
-  if (vec && (rank != rank8 || !aligned16(b))) {
-    {
+  if (pad_b) {
+    uint16_t* dst = own != nullptr ? (uint16_t*)(own + r_bytes) : nullptr;
+    if (own == nullptr) {
       std::lock_guard<std::mutex> lk(g_mu);
       const int rc2 = grow(&ds->lora_b, &ds->lora_b_bytes, (size_t)N * rank8 * 2);
       if (rc2 != LTX25_OK) { return rc2; }
+      dst = (uint16_t*)ds->lora_b;
     }
-    const hipError_t e = ltx25::launch_lora_pad(pb, N, rank, rank, (uint16_t*)ds->lora_b, rank8,
-                                                st);
+    const hipError_t e = ltx25::launch_lora_pad(pb, N, rank, rank, dst, rank8, st);
     if (e != hipSuccess) { return hip_fail(e, "lora pad launch"); }
-    pb = (const uint16_t*)ds->lora_b;
+    pb = dst;
     ldb = rank8;
   }
   if (ahead) {
@@ -779,7 +783,7 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     gd.K = K;
     float* ws = nullptr;
     if (own != nullptr) {
-      ws = (float*)(own + r_bytes);
+      ws = (float*)(own + r_bytes + b_bytes);
     } else if (r_plan.workspace_bytes > 0) {
       std::lock_guard<std::mutex> lk(g_mu);
       const int rc2 = grow(&ds->ws, &ds->ws_bytes, r_plan.workspace_bytes);
