@@ -34,7 +34,7 @@ int g_failures = 0;
 // ---- device memory: addresses only, never touched ----
 std::map<uintptr_t, size_t> g_mem;
 uintptr_t g_next = (uintptr_t)1 << 44;
-int g_mallocs = 0, g_device_syncs = 0;
+std::set<hipStream_t> g_capturing;   // streams
 
 // The bytes left in the allocation that holds p, 0 outside of all
 size_t room(const void* p)
@@ -85,19 +85,22 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int)
 }
 hipError_t hipMalloc(void** p, size_t n)
 {
-  ++g_mallocs;
+  if (!g_capturing.empty()) { return hipErrorStreamCaptureUnsupported; }
   *p = (void*)g_next;
   g_mem[g_next] = n;
   g_next += (n + 0xffff) & ~(size_t)0xffff;
   return hipSuccess;
 }
 hipError_t hipFree(void* p) { return g_mem.erase((uintptr_t)p) ? hipSuccess : hipErrorInvalidValue; }
-hipError_t hipDeviceSynchronize() { ++g_device_syncs; return hipSuccess; }
+hipError_t hipDeviceSynchronize()
+{
+  return g_capturing.empty() ? hipSuccess : hipErrorStreamCaptureUnsupported;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
+hipError_t hipStreamIsCapturing(hipStream_t st, hipStreamCaptureStatus* s)
 {
-  *s = hipStreamCaptureStatusNone;
+  *s = g_capturing.count(st) != 0 ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
@@ -190,6 +193,20 @@ void overlap(int M, int K, int N, int rank, int b_off)
   }
 }
 
+// A call, then the same under capture, on its own stream and on another one: it allocates nothing.
+void capture(int M, int K, int N, int rank, int b_off)
+{
+  const hipStream_t st = (hipStream_t)0x1000, other = (hipStream_t)0x2000;
+  EXPECT(add(st, M, K, N, rank, b_off) == LTX25_OK, "%s", ltx25_last_error());
+  for (hipStream_t c : {st, other}) {
+    g_capturing = {c};
+    g_launches.clear();
+    EXPECT(add(c, M, K, N, rank, b_off) == LTX25_OK, "captured: %s", ltx25_last_error());
+    EXPECT(!g_launches.empty() && g_launches.back().what == "lora", "not the one-pass kernel");
+    g_capturing.clear();
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -198,6 +215,7 @@ int main(int argc, char** argv)
   auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
   if (s == "tile_switch") { tile_switch(arg(2), arg(3), arg(4), arg(5)); }
   else if (s == "overlap") { overlap(arg(2), arg(3), arg(4), arg(5), arg(6)); }
+  else if (s == "capture") { capture(arg(2), arg(3), arg(4), arg(5), arg(6)); }
   else { std::printf("unknown scenario %s\n", s.c_str()); return 2; }
   return g_failures == 0 ? 0 : 1;
 }

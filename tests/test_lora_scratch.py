@@ -50,3 +50,8 @@ PLANS = [  # M, K, N, rank, bytes of b off 16-byte alignment
 @pytest.mark.parametrize("M,K,N,rank,b_off", PLANS)
 def test_streams_share_no_scratch(exe, M, K, N, rank, b_off):
     run(exe, "overlap", M, K, N, rank, b_off)
+
+
+@pytest.mark.parametrize("M,K,N,rank,b_off", PLANS)
+def test_a_call_prepares_its_capture(exe, M, K, N, rank, b_off):
+    run(exe, "capture", M, K, N, rank, b_off)

@@ -635,6 +635,13 @@ int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void
 constexpr int kLoraAheadMinK = 1536;
 constexpr int kLoraWideMinK = 512;
 
+// While it lives, this thread's allocations do not end another thread's capture
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // `need` bytes of the stream's own scratch, or null: the stream is being captured (a
 // graph may replay beside later calls on it), is the per-thread one (one handle, many
 // streams), is the ninth to ask, or memory is short. Held by at most kLoraSlots streams
@@ -660,9 +667,7 @@ char* lora_slot(DeviceState* ds, hipStream_t st, size_t need)
   }
   if (slot == nullptr) { return nullptr; }
   if (slot->bytes < need) {
-    // another thread's capture is not to be ended by this one's allocation
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    RelaxedCapture relaxed;
     bool ok = true;
     if (slot->buf != nullptr) {
       ok = hipStreamSynchronize(st) == hipSuccess;   // its only user
@@ -673,7 +678,6 @@ char* lora_slot(DeviceState* ds, hipStream_t st, size_t need)
     }
     void* buf = nullptr;
     ok = ok && hipMalloc(&buf, need) == hipSuccess;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!ok) {
       (void)hipGetLastError();
       return nullptr;
@@ -735,6 +739,15 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     if (own == nullptr) {
       held.unlock();
       wide = ahead = false;
+    } else if (pad_b) {
+      // A capture of this shape later runs the one-pass kernel and cannot
+      // allocate its copy of b: this call does, and goes on if there is no room.
+      RelaxedCapture relaxed;
+      std::lock_guard<std::mutex> lk(g_mu);
+      if (grow(&ds->lora_b, &ds->lora_b_bytes, (size_t)N * rank8 * 2) != LTX25_OK) {
+        (void)hipGetLastError();
+        g_err.clear();
+      }
     }
   }
   if (route == LTX25_LORA_PAIR || wide) {
