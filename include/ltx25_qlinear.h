@@ -290,9 +290,11 @@ int ltx25_linear_route(int M, int K, int N, int bits, ltx25_route* out);
  *   to a dense GEMM ahead of it where K >= 1536 or M >= 512, rank <= 512; and
  *   from rank 96 and K = 512 (N % 8 == 0) both products run on the dense GEMM,
  *   in the pair's manner, below the pair's 256 tokens too. These two keep r and a
- *   padded b in scratch of the call's own stream (up to 8 streams of a device), so
- *   such calls may overlap on several streams; further streams, the per-thread
- *   stream and a stream under capture run the kernel alone. It needs no scratch
+ *   padded b in scratch of the call's own stream, so such calls may overlap on
+ *   several streams. Up to 8 streams of a device hold scratch at a time, and a
+ *   stream whose work has ended gives it up to one that asks. Further streams, the
+ *   per-thread stream and a stream under capture run the kernel alone, which sums
+ *   in another order: the last bits may differ. It needs no scratch
  *   where rank % 8 == 0 and b is 16-byte aligned. Elsewhere its copy of b is in
  *   the library's scratch: calls of it on several streams are to be ordered, and
  *   a capture needs a call of the shape outside the capture before it.

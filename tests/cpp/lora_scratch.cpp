@@ -52,7 +52,7 @@ struct Launch {
   hipStream_t stream;
   std::vector<std::pair<uintptr_t, size_t>> scratch;   // library scratch it reads or writes
 };
-std::vector<Launch> g_launches;
+std::vector<Launch> g_launches;   // and the event calls between them
 
 void note(const char* what, hipStream_t st, std::initializer_list<std::pair<const void*, size_t>> use)
 {
@@ -66,6 +66,8 @@ void note(const char* what, hipStream_t st, std::initializer_list<std::pair<cons
   g_launches.push_back(l);
 }
 
+bool g_busy = false;                   // no stream's work ends
+hipError_t g_error = hipSuccess;       // what hipGetLastError finds
 int g_plans = 0;                       // made by the present call
 int g_set_after = 0, g_set_tile = 0;   // another thread sets the tile after that many of them
 
@@ -97,7 +99,34 @@ hipError_t hipDeviceSynchronize()
   return g_capturing.empty() ? hipSuccess : hipErrorStreamCaptureUnsupported;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
+{
+  static uintptr_t next = 0x100;
+  *e = (hipEvent_t)next++;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t st)
+{
+  g_launches.push_back({"record " + std::to_string((uintptr_t)e), st, {}});
+  return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t st, hipEvent_t e, unsigned)
+{
+  g_launches.push_back({"wait " + std::to_string((uintptr_t)e), st, {}});
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t) { return g_busy ? g_error = hipErrorNotReady : hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t)
+{
+  EXPECT(!g_busy, "the host waits for a stream");
+  return hipSuccess;
+}
+hipError_t hipGetLastError()
+{
+  const hipError_t e = g_error;
+  g_error = hipSuccess;
+  return e;
+}
 hipError_t hipStreamIsCapturing(hipStream_t st, hipStreamCaptureStatus* s)
 {
   *s = g_capturing.count(st) != 0 ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
@@ -125,6 +154,7 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan, float* ws, hipSt
   EXPECT(plan.workspace_bytes == 0 || room(ws) >= plan.workspace_bytes,
          "GEMM %d x %d -> %d: %zu bytes of partials, %zu at %p", d.M, d.K, d.N,
          plan.workspace_bytes, room(ws), (void*)ws);
+  EXPECT(g_error == hipSuccess, "an error is left for the launch's check");
   note("gemm", st, {{ws, plan.workspace_bytes}, {d.x, (size_t)d.M * d.K * 2},
                     {d.w, (size_t)(d.wn > 0 ? d.wn : d.N) * d.K * 2}, {d.y, (size_t)d.M * d.N * 2}});
   return hipSuccess;
@@ -158,6 +188,17 @@ int add(hipStream_t st, int M, int K, int N, int rank, int b_off = 0)
                         nullptr, M, K, N, rank);
 }
 
+// The last kernel
+std::string last_launch()
+{
+  for (size_t i = g_launches.size(); i-- > 0;) {
+    if (g_launches[i].what.find(' ') == std::string::npos || g_launches[i].what == "lora y") {
+      return g_launches[i].what;
+    }
+  }
+  return "";
+}
+
 // The tile switch changes after the call's n-th plan: what runs fits what was reserved for it, also
 // where the y GEMM splits K under one setting and not under the other.
 void tile_switch(int rank, int from, int to, int n)
@@ -166,7 +207,7 @@ void tile_switch(int rank, int from, int to, int n)
   g_set_after = n;
   g_set_tile = to;
   EXPECT(add((hipStream_t)0x1000, 128, 2048, 16384, rank) == LTX25_OK, "%s", ltx25_last_error());
-  EXPECT(!g_launches.empty() && g_launches.back().what == "gemm", "not the GEMM pair");
+  EXPECT(last_launch() == "gemm", "not the GEMM pair");
 }
 
 // Calls on several streams at once: no two of them use the same bytes of scratch.
@@ -202,9 +243,47 @@ void capture(int M, int K, int N, int rank, int b_off)
     g_capturing = {c};
     g_launches.clear();
     EXPECT(add(c, M, K, N, rank, b_off) == LTX25_OK, "captured: %s", ltx25_last_error());
-    EXPECT(!g_launches.empty() && g_launches.back().what == "lora", "not the one-pass kernel");
+    EXPECT(last_launch() == "lora", "not the one-pass kernel");
     g_capturing.clear();
   }
+}
+
+// One stream after another, each idle before the next: every one gets scratch, eight allocations
+// serve them all. With eight of them busy a ninth runs the one-pass kernel, until one is idle.
+void streams_come_and_go()
+{
+  for (int s = 1; s <= 30; ++s) {
+    EXPECT(add((hipStream_t)(uintptr_t)(0x1000 * s), 128, 4096, 1032, 32) == LTX25_OK, "%s",
+           ltx25_last_error());
+    EXPECT(last_launch() == "lora y", "stream %d runs the one-pass kernel", s);
+  }
+  EXPECT(g_mem.size() == 8, "%zu allocations", g_mem.size());
+  g_busy = true;
+  EXPECT(add((hipStream_t)0x100, 128, 4096, 1032, 32) == LTX25_OK, "%s", ltx25_last_error());
+  EXPECT(last_launch() == "lora", "a ninth stream beside eight busy ones: %s",
+         last_launch().c_str());
+  EXPECT(g_error == hipSuccess, "an error is left behind");
+  EXPECT(add((hipStream_t)0x1e000, 128, 4096, 1032, 32) == LTX25_OK, "%s", ltx25_last_error());
+  EXPECT(last_launch() == "lora y", "a busy stream with scratch of its own");
+  g_busy = false;
+  EXPECT(add((hipStream_t)0x100, 128, 8192, 1032, 64) == LTX25_OK, "%s", ltx25_last_error());
+  EXPECT(last_launch() == "lora y", "an idle slot is not taken");
+  EXPECT(g_mem.size() == 8, "%zu allocations", g_mem.size());
+}
+
+// A handle that comes back may be another stream's, while the one that had it still runs: the
+// second call waits for the event that the first recorded behind its launches.
+void recycled_handle(int M, int K, int N, int rank)
+{
+  const hipStream_t st = (hipStream_t)0x1000;
+  g_busy = true;
+  EXPECT(add(st, M, K, N, rank) == LTX25_OK, "%s", ltx25_last_error());
+  const std::string last = g_launches.empty() ? "" : g_launches.back().what;
+  EXPECT(last.rfind("record ", 0) == 0, "no event behind the launches");
+  const std::string e = last.size() > 7 ? last.substr(7) : "";
+  g_launches.clear();
+  EXPECT(add(st, M, K, N, rank) == LTX25_OK, "%s", ltx25_last_error());
+  EXPECT(!g_launches.empty() && g_launches.front().what == "wait " + e, "no wait before launches");
 }
 
 }  // namespace
@@ -216,6 +295,8 @@ int main(int argc, char** argv)
   if (s == "tile_switch") { tile_switch(arg(2), arg(3), arg(4), arg(5)); }
   else if (s == "overlap") { overlap(arg(2), arg(3), arg(4), arg(5), arg(6)); }
   else if (s == "capture") { capture(arg(2), arg(3), arg(4), arg(5), arg(6)); }
+  else if (s == "streams_come_and_go") { streams_come_and_go(); }
+  else if (s == "recycled_handle") { recycled_handle(arg(2), arg(3), arg(4), arg(5)); }
   else { std::printf("unknown scenario %s\n", s.c_str()); return 2; }
   return g_failures == 0 ? 0 : 1;
 }

@@ -273,6 +273,64 @@ def test_plans_under_capture_run_in_one_pass(pkg, dev, M, K, N, rank):
         assert (eager.float() - want.float()).norm() < 3e-3 * want.float().norm()
 
 
+# ranks whose b is copied with its rows padded: r ahead, and both products on the dense GEMM
+COPIED = [(128, 2048, 1032, 12), (33, 2048, 4104, 17), (64, 1024, 1024, 450)]
+
+
+@pytest.mark.parametrize("M,K,N,rank", COPIED)
+def test_plans_before_a_capture(pkg, dev, M, K, N, rank):
+    """A call, then the same captured: the one-pass kernel, whose copy of b the call has allocated."""
+    x, a, b, y0 = own_operands(M, K, N, rank)
+    want, y, eager = y0.clone(), y0.clone(), y0.clone()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    say(f"lora_add before its capture M={M} K={K} N={N} rank={rank}")
+    with torch.cuda.stream(side):
+        pkg.lora_add(x, a, b, eager, M, K, N, rank)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pkg.lora_add(x, a, b, y, M, K, N, rank)
+    pkg.set_lora_route(pkg.LORA_FUSED)
+    pkg.lora_add(x, a, b, want, M, K, N, rank)
+    pkg.set_lora_route(pkg.LORA_AUTO)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        y.copy_(y0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        eager.copy_(y0)
+        pkg.lora_add(x, a, b, eager, M, K, N, rank)
+        torch.cuda.synchronize()
+        assert (eager.float() - want.float()).norm() < 3e-3 * want.float().norm()
+
+
+@pytest.mark.parametrize("M,K,N,rank", OWN + COPIED)
+def test_eight_streams_have_their_plans(pkg, dev, M, K, N, rank):
+    """Eight streams at once, each with an adapter of its own: all idle before, so all hold scratch,
+    and each result has the bits of the plan alone."""
+    n = 8
+    x, a, b, y0 = own_operands(M, K, N, rank)
+    bs = [(b.float() * (1.0 + 0.1 * i)).to(torch.bfloat16) for i in range(n)]
+    alone = []
+    for bi in bs:
+        alone.append(y0.clone())
+        pkg.lora_add(x, a, bi, alone[-1], M, K, N, rank)
+    streams = [torch.cuda.Stream() for _ in range(n)]
+    ys = [[y0.clone() for _ in range(6)] for _ in range(n)]
+    torch.cuda.synchronize()
+    say(f"lora_add, eight streams M={M} K={K} N={N} rank={rank}")
+    for t in range(6):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                pkg.lora_add(x, a, bs[i], ys[i][t], M, K, N, rank)
+    torch.cuda.synchronize()
+    for i in range(n):
+        for y in ys[i]:
+            assert torch.equal(y.view(torch.int16), alone[i].view(torch.int16)), i
+
+
 @pytest.mark.parametrize("M,K,N,rank", OWN)
 def test_plans_overlap_on_streams(pkg, dev, M, K, N, rank):
     """Calls on ten streams at once, more than have scratch of their own: each result is the one

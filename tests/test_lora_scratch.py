@@ -55,3 +55,12 @@ def test_streams_share_no_scratch(exe, M, K, N, rank, b_off):
 @pytest.mark.parametrize("M,K,N,rank,b_off", PLANS)
 def test_a_call_prepares_its_capture(exe, M, K, N, rank, b_off):
     run(exe, "capture", M, K, N, rank, b_off)
+
+
+def test_streams_that_come_and_go_keep_the_plans(exe):
+    run(exe, "streams_come_and_go")
+
+
+@pytest.mark.parametrize("M,K,N,rank", [(128, 4096, 1032, 32), (64, 1024, 1024, 450)])
+def test_a_stream_handle_may_come_back(exe, M, K, N, rank):
+    run(exe, "recycled_handle", M, K, N, rank)
