@@ -36,6 +36,11 @@ CASES = [
     (150, 1024, 40, 16, 64, "bf16", 1),      # dense, 32 x 32
     (1000, 1088, 300, 16, 64, "none", 1),    # dense, 64 x 32
     (160, 4160, 4100, 16, 64, "f32", 1),     # dense, N % 8 == 4
+    (129, 1088, 8190, 8, 64, "bf16", 1),     # the wide panels at few chunks: 128 x 64, 17 chunks
+    (300, 1088, 5000, 4, 32, "f32", 1),
+    (250, 1088, 4100, 16, 64, "none", 1),
+    (260, 1024, 3000, 8, 32, "f32", 1),      # 64 x 64
+    (1500, 2048, 513, 4, 64, "bf16", 1),     # 128 x 32
     (1, 4096, 8192, 8, 64, "f32", 1),        # at most 128 rows where the M <= 128 kernel
     (31, 4160, 12290, 4, 64, "bf16", 1),     #   would need two rounds: 32 x 32, 32 x 64
     (126, 4096, 8192, 8, 32, "none", 1),

@@ -5,8 +5,8 @@ The variant runs the same GEMM plan with its split-K partials in a fixed
 per-GPU device array. Its output must be bit-identical to linear_q_ex's on
 the same operands (the in-register dequant stands in for the dequant-once
 expansion, which produces the same bits). Each pair of calls runs back to
-back, the second on a smaller input, so stale partials of the first call
-sit in the shared array when the second runs. The device's free memory is
+back, the second on a smaller input: where both split K, stale partials of
+the first call sit in the shared array when the second runs. The device's free memory is
 read around every call after set-up (ltx25_init, which resolves this GPU's
 copy of the array; the runtime places it in device memory then): the
 variant must not change it. As a check that
@@ -21,19 +21,22 @@ from gpu_util import make_qweight, rng_normal, say
 
 pytestmark = pytest.mark.gpu
 
-# (name, M, K, N, bits, group, bias dtype, epilogue); first of each pair is the larger input
+# (name, (K splits of both calls), two calls of M, K, N, bits, group, bias dtype, epilogue); the
+# first of a pair is the larger input
 PAIRS = [
-    ("mid split-K then skinny split-K",
-     (256, 2048, 2048, 8, 64, "f32", 1), (64, 4096, 4096, 8, 64, "bf16", 0)),
-    ("skinny split-K then skinny",
+    ("mid split-K (128x128 tile) then skinny split-K", (2, 2),
+     (640, 2048, 6144, 8, 64, "f32", 1), (64, 4096, 4096, 8, 64, "bf16", 0)),
+    ("mid split-K (128x128 tile) then mid split-K (panels)", (2, 7),
+     (640, 2048, 6144, 4, 64, "bf16", 0), (150, 16384, 700, 4, 32, "f32", 1)),
+    ("skinny split-K then skinny", (4, 1),
      (126, 8192, 2048, 8, 64, "bf16", 0), (126, 2048, 2048, 8, 64, None, 1)),
-    ("tall (dequant-once in the entry point) then mid split-K",
-     (4096, 4096, 4096, 8, 64, "bf16", 1), (300, 2048, 2048, 8, 64, "f32", 0)),
-    ("w4 skinny split-K then w4 mid",
+    ("tall (dequant-once in the entry point) then mid split-K", (1, 2),
+     (4096, 4096, 4096, 8, 64, "bf16", 1), (640, 2048, 6144, 8, 64, "f32", 0)),
+    ("w4 skinny split-K then w4 mid", (2, 1),
      (126, 4096, 4096, 4, 32, "f32", 0), (192, 2048, 1024, 4, 32, None, 0)),
     # linear_q_ex expands the w4 weight and runs the 16x16x32 tile; the
     # no-allocation call runs the template's fused 32x32x16 w4 tile
-    ("w4 tall (dequant-once in the entry point vs fused w4 tile) then w4 mid",
+    ("w4 tall (dequant-once in the entry point vs fused w4 tile) then w4 mid", (1, 1),
      (1024, 4096, 4096, 4, 32, None, 1), (512, 1024, 2048, 4, 64, "f32", 0)),
 ]
 
@@ -98,12 +101,11 @@ def _one(pkg, case, seed):
     return route
 
 
-@pytest.mark.parametrize("name,first,second", PAIRS, ids=[p[0] for p in PAIRS])
-def test_noalloc_matches_linear_q_ex(pkg, name, first, second):
+@pytest.mark.parametrize("name,splits,first,second", PAIRS, ids=[p[0] for p in PAIRS])
+def test_noalloc_matches_linear_q_ex(pkg, name, splits, first, second):
     r1 = _one(pkg, first, 11 + first[0])
     r2 = _one(pkg, second, 23 + second[0])
-    # the pair must exercise the shared scratch at least once
-    assert r1["splits"] > 1 or r2["splits"] > 1
+    assert (r1["splits"], r2["splits"]) == splits   # which of them use the shared scratch
 
 
 def test_noalloc_refuses_the_int8_tier(pkg):

@@ -650,11 +650,6 @@ bool plan_panel(int M, int N, int K, int cu_count, GemmPlan& plan)
   bool found = false;
   for (const PanelCost& c : kPanels) {
     if (c.rows >= M + 32 && c.rows > 32) { continue; }   // whole row blocks of nothing
-    // More than 128 rows at K up to 2048 take the narrow panels only: the
-    // 128 x 128 tile's split plans there are what the no-allocation linear's
-    // shared scratch is exercised by (300 x 2048 -> 2048: 18.0 us on them, 11.6
-    // on a 128 x 32 panel).
-    if (M > 128 && K <= 2048 && c.rows * c.cols > 64 * 32) { continue; }
     const long tiles = (long)((M + c.rows - 1) / c.rows) * ((N + c.cols - 1) / c.cols);
     for (long s = 1; s == 1 || K / s >= kMinK; ++s) {
       const long per = (chunks + s - 1) / s;
