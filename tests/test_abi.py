@@ -293,8 +293,8 @@ def test_noalloc_refuses_the_int8_tier_before_device_use(pkg, lib):
 def test_every_planned_split_fits_the_noalloc_scratch(pkg):
     """Split-K partials of every plan the planner makes for a 256-CU device
     fit the no-allocation linear's 32 MiB: the M <= 128 kernel keeps
-    (N / 32) x splits within 3 workgroups per CU, and the 128 x 128 tile
-    splits only until its workgroups cover the CUs once."""
+    (N / 32) x splits within 3 workgroups per CU, the panels within one, and
+    the 128 x 128 tile splits only until its workgroups cover the CUs once."""
     cap = pkg.noalloc_scratch_bytes()
     worst = 0
     for M in [1, 16, 64, 126, 128, 129, 192, 255, 256, 300, 384, 512, 640, 1000, 1024, 2040,

@@ -16,11 +16,13 @@ from gpu_util import make_qweight, rng_normal, say
 
 pytestmark = pytest.mark.gpu
 
-# (name, M, K, N, bits, group, bias dtype, epilogue)
+# (name, M, K, N, bits, group, bias dtype, epilogue, tile, K splits)
 CASES = [
-    ("mid split-K (128x128 tile)", 256, 2048, 2048, 8, 64, "f32", 1),
-    ("M <= 128 kernel, split-K", 126, 8192, 2048, 8, 64, "bf16", 0),
-    ("256x256 fused w8 tile", 4096, 2048, 4096, 8, 64, None, 1),
+    ("mid split-K (128x128 tile)", 640, 2048, 6144, 8, 64, "f32", 1, 2, 2),
+    ("mid split-K (panels)", 150, 16384, 700, 8, 64, "bf16", 0, 2, 7),
+    ("mid, one K split (panels)", 256, 2048, 2048, 8, 64, "f32", 1, 2, 1),
+    ("M <= 128 kernel, split-K", 126, 8192, 2048, 8, 64, "bf16", 0, 3, 4),
+    ("256x256 fused w8 tile", 4096, 2048, 4096, 8, 64, None, 1, 1, 1),
 ]
 
 
@@ -37,10 +39,14 @@ def _operands(pkg, M, K, N, bits, group, bias_dt, seed):
     return x, qw, bias
 
 
-@pytest.mark.parametrize("name,M,K,N,bits,group,bias_dt,epi", CASES, ids=[c[0] for c in CASES])
-def test_noalloc_linear_replays_in_a_graph(pkg, lib, name, M, K, N, bits, group, bias_dt, epi):
+@pytest.mark.parametrize("name,M,K,N,bits,group,bias_dt,epi,tile,splits", CASES,
+                         ids=[c[0] for c in CASES])
+def test_noalloc_linear_replays_in_a_graph(pkg, lib, name, M, K, N, bits, group, bias_dt, epi, tile,
+                                           splits):
     assert lib.ltx25_init() == 0, pkg.last_error()
     pkg.set_tile(pkg.TILE_AUTO)
+    route = pkg.linear_route(M, K, N, bits)
+    assert (route["tile"], route["splits"]) == (tile, splits), route
     x, qw, bias = _operands(pkg, M, K, N, bits, group, bias_dt, 11)
     # another call of the same plan family, run eagerly between replays: it
     # rewrites the scratch array the captured call uses

@@ -46,7 +46,7 @@ SHAPES = [  # name, M, K, N, rank, the route AUTO takes
     ("GEMM pair, rank 128, no padding", 300, 2048, 1024, 128, P),
     ("GEMM pair, rank 450 padded to 512", 512, 1024, 2048, 450, P),
     ("GEMM pair, ragged M and N", 777, 512, 1000, 200, P),
-    ("GEMM pair, rank 1000 (split-K second GEMM)", 256, 512, 640, 1000, P),
+    ("GEMM pair, rank 1000", 256, 512, 640, 1000, P),
     # r first (M >= 512, rank % 8 == 0, rank < 96): r = x . A^T by the dense GEMM, then the
     # fused kernel's second phase reads it
     ("r first: rank 32 at the FFN width", 1024, 4096, 16384, 32, RF),
@@ -56,8 +56,8 @@ SHAPES = [  # name, M, K, N, rank, the route AUTO takes
     # super blocks ahead (ranks up to 64) run past the column split's end
     ("r first: rank 16, ragged N", 640, 1024, 1000, 16, RF),
     ("r first: rank 64, N = 4104", 520, 256, 4104, 64, RF),
-    # more rows: r's GEMM covers the CUs with fewer K splits; ragged M, a rank that is not a
-    # multiple of 16, K that is not a multiple of 512
+    # more rows, so more of r's panels; ragged M, a rank that is not a multiple of 16, K that is
+    # not a multiple of 512
     ("r first, 2085 rows: rank 40, K = 2624", 2085, 2624, 1024, 40, RF),
     ("r first, 2112 rows: rank 8, K = 1088", 2112, 1088, 256, 8, RF),
     ("r first, 2048 rows: rank 64, K = 4096", 2048, 4096, 512, 64, RF),
@@ -102,6 +102,21 @@ def test_lora_add_against_oracle_and_f64(pkg, dev, what, M, K, N, rank, route):
     say(f"lora_add {what}: M={M} K={K} N={N} rank={rank}")
     assert pkg.lora_on_matrix_cores(M, K, N, rank) == (route == P)
     assert run_and_check(pkg, what, M, K, N, rank) == ROUTE[route]
+
+
+@pytest.mark.parametrize("M,N,rank,tile", [(256, 640, 1000, 2), (64, 264, 16384, 0)])
+def test_pair_with_a_split_k_second_gemm(pkg, dev, M, N, rank, tile):
+    """y = bf16(y + r . b^T) with r . b^T split over K (128 x 128 tiles; the M <= 128 kernel): y is
+    added once, by the launch that sums the partials."""
+    pkg.set_tile(tile)
+    pkg.set_lora_route(pkg.LORA_PAIR)
+    try:
+        assert pkg.linear_route(M, (rank + 63) & ~63, N, 16)["splits"] > 1
+        say(f"lora_add pair, split-K second GEMM M={M} N={N} rank={rank} tile={tile}")
+        assert run_and_check(pkg, f"split second {M}", M, 512, N, rank) == ROUTE[P]
+    finally:
+        pkg.set_tile(pkg.TILE_AUTO)
+        pkg.set_lora_route(pkg.LORA_AUTO)
 
 
 # the same shapes on every route that can take them (the A/B hook, ltx25_set_lora_route)
