@@ -286,10 +286,11 @@ int ltx25_linear_route(int M, int K, int N, int bits, ltx25_route* out);
  * - otherwise the fused kernel, one launch per 512 adapter columns (16-byte
  *   aligned x, a and y with K % 8 == 0 and N % 8 == 0 take its vector path;
  *   when the rank is not a multiple of 8, b is first copied with its rows
- *   zero-padded to one). On the vector path with K % 64 == 0 it leaves x . a^T
- *   to a dense GEMM ahead of it where K >= 1536 or M >= 512, rank <= 512; and
- *   from rank 96 and K = 512 (N % 8 == 0) both products run on the dense GEMM,
- *   in the pair's manner, below the pair's 256 tokens too. These two keep r and a
+ *   zero-padded to one). On the vector path with K % 64 == 0 and rank < 96 it
+ *   leaves x . a^T to a dense GEMM ahead of it where K times the rows of x and a
+ *   makes up for the launch; and from rank 96 and K = 512 (N % 8 == 0) both
+ *   products run on the dense GEMM by the same measure, in the pair's manner,
+ *   below the pair's 256 tokens too. These two keep r and a
  *   padded b in scratch of the call's own stream, so such calls may overlap on
  *   several streams. Up to 8 streams of a device hold scratch at a time, and a
  *   stream whose work has ended gives it up to one that asks. Further streams, the

@@ -157,16 +157,16 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan, float* ws, hipSt
   EXPECT(g_error == hipSuccess, "an error is left for the launch's check");
   note("gemm", st, {{ws, plan.workspace_bytes}, {d.x, (size_t)d.M * d.K * 2},
                     {d.w, (size_t)(d.wn > 0 ? d.wn : d.N) * d.K * 2}, {d.y, (size_t)d.M * d.N * 2}});
-  return hipSuccess;
+  return d.done != nullptr ? hipEventRecord(d.done, st) : hipSuccess;
 }
 
 hipError_t launch_lora(const uint16_t*, const uint16_t*, const uint16_t* b, uint16_t*, int M, int,
                        int N, int rank, int ldb, bool, int, hipStream_t st, const uint16_t* r_in,
-                       bool)
+                       bool, hipEvent_t done)
 {
   note(r_in != nullptr ? "lora y" : "lora", st,
        {{b, ((size_t)(N - 1) * ldb + rank) * 2}, {r_in, (size_t)M * rank * 2}});
-  return hipSuccess;
+  return done != nullptr ? hipEventRecord(done, st) : hipSuccess;
 }
 
 hipError_t launch_lora_pad(const uint16_t*, int rows, int, int, uint16_t* dst, int ld_dst,

@@ -184,14 +184,23 @@ def test_lora_is_deterministic(pkg, dev):
     assert np.array_equal(outs[0], outs[1])
 
 
-# the plans under the FUSED answer: r by the dense GEMM ahead of the y phase (from K = 1536),
-# both products on the dense GEMM (from rank 96 and K = 512), one pass below; at each line's
-# sides, ranks that are not multiples of 8 or 64, one token, ragged N
+# the plans under the FUSED answer: r by the dense GEMM ahead of the y phase, both products on the
+# dense GEMM (from rank 96 and K = 512), one pass below; at each line's sides, ranks that are not
+# multiples of 8 or 64, one token, ragged N
 PLANS = [  # M, K, N, rank
-    (128, 1536, 1032, 32), (128, 1472, 1032, 32), (1, 4096, 520, 5), (33, 2048, 8, 90),
-    (255, 2048, 4104, 17), (700, 512, 264, 6), (20, 1600, 512, 95), (255, 512, 264, 96),
-    (3, 512, 1000, 450), (255, 448, 264, 96), (70, 1600, 200, 512), (64, 1600, 200, 520),
-    (40, 1536, 1000, 1), (300, 1536, 96, 12),
+    (128, 1344, 1032, 32), (128, 1280, 1032, 32), (23, 2112, 1032, 32), (23, 2048, 1032, 32),
+    (255, 1024, 1032, 32), (255, 960, 1032, 32), (70, 1088, 264, 40), (70, 1024, 264, 40),
+    # b copied
+    (1, 11456, 520, 5), (1, 11392, 520, 5), (33, 1024, 8, 90), (20, 1088, 512, 95),
+    (20, 960, 512, 95), (255, 2304, 4104, 17), (255, 2240, 4104, 17), (300, 2560, 96, 12),
+    (40, 1536, 1000, 1), (700, 3904, 264, 6), (700, 3840, 264, 6), (600, 2688, 4104, 6),
+    (600, 2624, 4104, 6), (600, 1024, 264, 90),
+    # both on the dense GEMM
+    (255, 1024, 264, 96), (255, 512, 264, 96), (64, 512, 264, 128), (1, 512, 264, 128),
+    (3, 512, 1000, 450), (3, 448, 1000, 450), (255, 512, 264, 128), (255, 512, 2056, 128),
+    (200, 640, 264, 192), (200, 576, 264, 192), (200, 512, 264, 450), (200, 512, 264, 225),
+    (100, 512, 264, 100), (1, 512, 264, 100), (32, 768, 264, 104), (16, 768, 264, 104),
+    (70, 1600, 200, 512), (64, 1600, 200, 520),
 ]
 
 
@@ -289,7 +298,7 @@ def test_plans_under_capture_run_in_one_pass(pkg, dev, M, K, N, rank):
 
 
 # ranks whose b is copied with its rows padded: r ahead, and both products on the dense GEMM
-COPIED = [(128, 2048, 1032, 12), (33, 2048, 4104, 17), (64, 1024, 1024, 450)]
+COPIED = [(128, 4352, 1032, 12), (33, 4096, 4104, 17), (64, 1024, 1024, 450)]
 
 
 @pytest.mark.parametrize("M,K,N,rank", COPIED)

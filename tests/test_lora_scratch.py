@@ -42,8 +42,8 @@ def test_the_tile_switch_may_change_during_a_call(exe, rank, before, after):
 # the plans under the fused route: r ahead of the y phase, both products on the dense GEMM; ranks
 # and addresses of b that the kernels read as they are, and that need a copy
 PLANS = [  # M, K, N, rank, bytes of b off 16-byte alignment
-    (128, 4096, 1032, 32, 0), (128, 4096, 1032, 32, 2), (128, 2048, 1032, 12, 0),
-    (33, 2048, 4104, 17, 0), (64, 1024, 1024, 450, 0), (100, 2048, 1000, 192, 6),
+    (128, 4096, 1032, 32, 0), (128, 4096, 1032, 32, 2), (128, 4352, 1032, 12, 0),
+    (33, 4096, 4104, 17, 0), (64, 1024, 1024, 450, 0), (100, 2048, 1000, 192, 6),
 ]
 
 

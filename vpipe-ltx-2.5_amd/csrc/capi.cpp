@@ -552,10 +552,10 @@ LoraPairPlan plan_lora_pair(const DeviceState* ds, const void* a, const void* b,
 }
 
 // `own`: p.operand_bytes() + p.ws_bytes of the call's own, instead of the
-// library's scratch.
+// library's scratch; `done`: an event that the last launch records.
 int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void* x,
               const void* a, const void* b, void* y, void* r_caller, int M, int K, int N, int rank,
-              char* own = nullptr)
+              char* own = nullptr, hipEvent_t done = nullptr)
 {
   const int rk = p.rk;
   const bool pad_a = p.pad_a, pad_b = p.pad_b;
@@ -600,6 +600,7 @@ int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void
       d.w = pb;
       d.y = (uint16_t*)y;
       d.y_in = (const uint16_t*)y;
+      d.done = done;
       d.N = N;
       d.K = rk;
     }
@@ -621,22 +622,67 @@ int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void
 
 // FUSED's two other plans under AUTO (a forced FUSED is always the one-pass
 // kernel). That kernel computes r = x . A^T once per row block and column split,
-// from 16-byte loads of 32 rows each, so its time grows with K and, past rank 32
-// or so, with the rank. From kLoraAheadMinK of K r comes from the dense GEMM, as
-// on the r-first route, and the kernel runs its y phase: rank 32, 128 x 4096 ->
-// 16384 22.8 us in one pass, 15.6 so; rank 40, 24 x 15360 -> 13264 79.5 and
-// 16.1; 246 x 2816 -> 208, rank 24 14.0 and 9.6 (at K = 1024, 9 tokens, 8.9 and
-// 10.7). From rank kLoraPairMinRank and kLoraWideMinK both products run on the
-// dense GEMM, as in the pair: rank 448, 64 x 1024 -> 1024 67.5 us in one pass,
-// 10.4 so; rank 128, 128 x 4096 -> 4096 66.5 and 14.5; rank 200, 126 x 8192 ->
-// 2048 189 and 22.5.
+// from 16-byte loads of 32 rows each, so its time grows with K and with the rows
+// of x and A that it reads: 0.6 us and 0.045 us a row per 1024 of K up to rank 32,
+// more above. Either r comes from the dense GEMM, as on the r-first route, and
+// the kernel runs its y phase (`ahead`), or both products run on the dense GEMM, as
+// in the pair (`wide`). Rank 32, 128 x 4096 -> 16384 21.2 us in one pass, 14.7
+// ahead; rank 40, 24 x 15360 -> 13264 66 and 14.6; rank 448, 64 x 1024 -> 1024 62 in
+// one pass, 10.5 on the GEMMs; rank 128, 128 x 4096 -> 4096 66 and 15.0; rank 200,
+// 126 x 8192 -> 2048 188 and 18.9 (lora_add in a loop, its host work included).
 // The one-pass kernel needs no scratch where it reads b as it is (rank % 8 == 0, b
 // 16-byte aligned): such calls may overlap on several streams, be captured
 // unprepared, and never fail for memory. The other plans keep all of that: their
 // scratch, a padded copy of b included, belongs to the call's stream (lora_slot),
 // and where there is none the one-pass kernel runs.
-constexpr int kLoraAheadMinK = 1536;
-constexpr int kLoraWideMinK = 512;
+
+// K times the rows of x and A that phase 1 reads for a row block: what the one-pass
+// kernel spends on r, where the plans spend launches, an event and a wider copy of b.
+// The lines below lie where both sides took the same time in a sweep of 5300 shapes (M 1
+// to 8160, K 512 to 8192, N 64 to 8192); the figures are one pass and the plan, us.
+long lora_phase1(int M, int K, int rank) { return (long)K * (rank + std::min(M + 8, 32)); }
+
+// Rank 8, 64 x 1536 -> 512 8.9 and 9.2, x 3072 12.5 and 11.4; rank 17 (b copied), 64 x 3072 ->
+// 512 16.6 and 16.7, x 4096 18.9 and 17.3; rank 50, 64 x 1024 -> 512 13.8 and 15.0, x 2048
+// 18.0 and 16.6; rank 4, 600 x 1024 -> 512 11.6 and 13.4, x 4096 16.9 and 15.2. From 512 tokens
+// only a b that is copied gets here; with many columns the one-pass kernel then
+// repeats phase 1 for each of its column splits.
+bool lora_ahead_pays(int M, int K, int N, int rank, bool copies_b)
+{
+  long line = copies_b ? 120000 : 75000;   // two or three rank blocks
+  if (rank <= 32 && copies_b) {
+    line = M <= 128 ? 160000 : M < kLoraRFirstMinM ? 110000 : N >= 4096 ? 100000 : 146000;
+  } else if (rank <= 32) {
+    line = M < 24 ? 130000 : M <= 128 ? 82000 : 62000;
+  }
+  return lora_phase1(M, K, rank) >= line;
+}
+
+// From rank 96; phase 1 then has an instance's 128, 256 or 512 rows of A. Without a copy of b, or
+// with one on both sides, the pair is ahead from 512 of K nearly everywhere (below that it has
+// not been tried here): rank 128, 1 x 512 -> 64 9.5 and 8.2; rank 100, 1 x 512 -> 24 11.4 and
+// 12.1, x 768 -> 512 14.1 and 13.2. Where only the pair copies b (to 64 columns): rank 96, 1 x 1024
+// -> 24 12.2 and 12.8, 128 x 512 -> 1024 14.4 and 13.1; rank 104, 16 x 768 -> 256 12.7 and 13.3, 64 x
+// 1024 -> 256 18.1 and 14.1. Above 128 rows r's GEMM takes slower tiles below 1024 of K: rank 128,
+// 200 x 512 -> 24 12.0 and 15.6, -> 1024 17.7 and 16.7; rank 240, 200 x 512 -> 1024 22.8 and 21.9;
+// rank 450 -> 24 30.3 and 23.5.
+bool lora_wide_pays(int M, int K, int N, int rank, bool copies_b, bool pair_copies_b)
+{
+  const bool many = N >= 1024;
+  const bool slow_r = M > 128 && K < 1024;
+  long line = 0;
+  if (!pair_copies_b) {
+    line = slow_r && !many ? 184000 : 0;
+  } else if (copies_b) {
+    line = slow_r ? (many ? 147000 : 258000) : many ? 0 : 74000;
+  } else {
+    line = slow_r ? (many ? 221000 : 278000)
+           : many ? (M < 16 ? 92000 : 77000)
+                  : (M < 16 ? 145000 : 117000);
+  }
+  const int rows = rank <= 128 ? 128 : rank <= 256 ? 256 : (rank + 511) / 512 * 512;
+  return K >= 512 && lora_phase1(M, K, rows) >= line;
+}
 
 // While it lives, this thread's allocations do not end another thread's capture
 struct RelaxedCapture {
@@ -683,8 +729,9 @@ LoraSlot* lora_slot(DeviceState* ds, hipStream_t st, size_t need)
     }
     bool ok = slot != nullptr;
     if (ok && slot->done == nullptr) {
-      // orders streams of this device only: with the system-scope fence of a plain event
-      // 128 x 4096 -> 16384 at rank 32 takes 46.0 us, without it 44.2 (no event: 43.5)
+      // orders streams of this device only. 128 x 4096 -> 16384 at rank 32: 46.0 us with a plain
+      // event, which fences the system, recorded behind the call; 44.2 without the fence;
+      // 43.5 as the last kernel's own completion (launch_done), as with no event
       ok = hipEventCreateWithFlags(&slot->done, hipEventDisableTiming |
                                                     hipEventDisableSystemFence) == hipSuccess;
     }
@@ -723,9 +770,14 @@ LoraSlot* lora_slot(DeviceState* ds, hipStream_t st, size_t need)
 struct LoraSlotUse {
   LoraSlot* slot = nullptr;
   hipStream_t st = nullptr;
+  bool marked = false;   // the last launch has recorded the event itself
   ~LoraSlotUse()
   {
     if (slot == nullptr) { return; }
+    if (marked) {
+      slot->recorded = true;
+      return;
+    }
     slot->recorded = hipEventRecord(slot->done, st) == hipSuccess;
     if (!slot->recorded) {
       (void)hipGetLastError();
@@ -759,14 +811,14 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
   const bool planned =
       route == LTX25_LORA_FUSED &&
       g_lora_force.load(std::memory_order_relaxed) == LTX25_LORA_AUTO && vec && K % 64 == 0;
-  bool wide = planned && rank >= kLoraPairMinRank && K >= kLoraWideMinK &&
+  const bool pad_b = vec && (rank != rank8 || !aligned16(b));
+  bool wide = planned && rank >= kLoraPairMinRank &&
+              lora_wide_pays(M, K, N, rank, pad_b, rank % 64 != 0 || !aligned16(b)) &&
               lora_pair_ok(M, K, N, rank, x, y);
   bool ahead = route == LTX25_LORA_RFIRST ||
-               (planned && !wide && rank <= ltx25::kLoraMaxRank &&
-                below_limit((size_t)M * rank8 * 2) &&
-                (K >= kLoraAheadMinK || M >= kLoraRFirstMinM));
+               (planned && rank < kLoraPairMinRank && below_limit((size_t)M * rank8 * 2) &&
+                lora_ahead_pays(M, K, N, rank, pad_b));
   const bool few = route == LTX25_LORA_FUSED && (wide || ahead);
-  const bool pad_b = vec && (rank != rank8 || !aligned16(b));
   const ltx25::GemmPlan r_plan = ltx25::plan_gemm(M, rank8, K, 16, ds->cu_count);
   const size_t r_bytes = align256((size_t)M * rank8 * 2);
   const size_t b_bytes = pad_b ? align256((size_t)N * rank8 * 2) : 0;
@@ -791,16 +843,21 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     if (own != nullptr && pad_b) {
       // A capture of this shape later runs the one-pass kernel and cannot
       // allocate its copy of b: this call does, and goes on if there is no room.
-      RelaxedCapture relaxed;
+      const size_t need = (size_t)N * rank8 * 2;
       std::lock_guard<std::mutex> lk(g_mu);
-      if (grow(&ds->lora_b, &ds->lora_b_bytes, (size_t)N * rank8 * 2) != LTX25_OK) {
-        (void)hipGetLastError();
-        g_err.clear();
+      if (ds->lora_b_bytes < need) {
+        RelaxedCapture relaxed;
+        if (grow(&ds->lora_b, &ds->lora_b_bytes, need) != LTX25_OK) {
+          (void)hipGetLastError();
+          g_err.clear();
+        }
       }
     }
   }
   if (route == LTX25_LORA_PAIR || wide) {
-    const int rc2 = lora_pair(ds, st, pair, x, a, b, y, wide ? nullptr : r, M, K, N, rank, own);
+    const int rc2 = lora_pair(ds, st, pair, x, a, b, y, wide ? nullptr : r, M, K, N, rank, own,
+                              wide ? use.slot->done : nullptr);
+    use.marked = wide && rc2 == LTX25_OK;
     return rc2 != LTX25_OK ? rc2 : gelu_pass();
   }
   const uint16_t* pa = (const uint16_t*)a;
@@ -855,8 +912,9 @@ int run_lora(hipStream_t st, const void* x, const void* a, const void* b, void* 
     hipError_t e = ltx25::launch_gemm(gd, r_plan, ws, st);
     if (e != hipSuccess) { return hip_fail(e, "lora r gemm launch"); }
     e = ltx25::launch_lora((const uint16_t*)x, pa, pb, (uint16_t*)y, M, K, N, rank8, ldb, vec,
-                           ds->cu_count, st, rb, gelu);
+                           ds->cu_count, st, rb, gelu, own != nullptr ? use.slot->done : nullptr);
     if (e != hipSuccess) { return hip_fail(e, "lora launch"); }
+    use.marked = own != nullptr;
     return LTX25_OK;
   }
   for (int c = 0; c < rank; c += ltx25::kLoraMaxRank) {

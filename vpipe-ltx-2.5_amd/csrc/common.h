@@ -2,6 +2,7 @@
 // launcher interface between the kernels and the C ABI layer (capi.cpp).
 #pragma once
 
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -53,6 +54,26 @@ __device__ __forceinline__ float gelu_tanh(float x)
 }
 
 // ---- internal launcher interface ------------------------------------------
+
+// kernel<<<grid, block, 0, stream>>>(args...); with `done`, an event that becomes the
+// kernel's own completion: the host time of a call grows by 2 us, with an event
+// recorded behind the kernel by 4 (torch's HIP 7.0 runtime).
+template <typename T>
+struct Param {
+  using type = T;
+};
+template <typename... P>
+inline hipError_t launch_done(void (*kernel)(P...), dim3 grid, int block, hipStream_t stream,
+                              hipEvent_t done, typename Param<P>::type... args)
+{
+  if (done == nullptr) {
+    hipLaunchKernelGGL(kernel, grid, dim3((unsigned)block), 0, stream, args...);
+    return hipGetLastError();
+  }
+  void* list[] = {&args...};
+  return hipExtLaunchKernel((const void*)kernel, grid, dim3((unsigned)block), list, 0, stream,
+                            nullptr, done, 0);
+}
 
 // Record `code` and a printf-style message as this thread's last error
 // (what ltx25_last_error returns); returns `code`.
@@ -114,6 +135,7 @@ struct GemmDesc {
   int epilogue = kEpiNone;
   uint16_t* y = nullptr;
   const uint16_t* y_in = nullptr;   // when set: y = bf16(acc + bias + y_in), y_in may be y
+  hipEvent_t done = nullptr;        // when set: an event that the last launch records
   int M = 0, N = 0, K = 0;
 };
 
@@ -195,9 +217,10 @@ constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
 hipError_t noalloc_scratch(void** out);
 // Sums `splits` f32 partial planes [M][N] in split order, adds bias and
 // y_in, applies the epilogue and rounds to bf16 once.
+// `done`: an event recorded as the launch's completion, or null.
 hipError_t launch_splitk_reduce(const float* partial, int splits, const void* bias, int bias_type,
                                 int epilogue, const uint16_t* y_in, uint16_t* y, int M, int N,
-                                hipStream_t stream);
+                                hipStream_t stream, hipEvent_t done = nullptr);
 
 // The low-rank adapter delta y += (x . A^T) . B^T (lora.hip). One launch
 // covers at most kLoraMaxRank adapter columns: `a` points at the pass's
@@ -207,13 +230,15 @@ hipError_t launch_splitk_reduce(const float* partial, int splits, const void* bi
 // `rank` up to the next multiple of 8).
 // With `r_in` set ([M][rank] bf16, rank % 8 == 0, vector path only) the
 // launch skips the x . A^T phase and reads r from it. `gelu` (vector path):
-// y = bf16(gelu(bf16(y + delta))), the bits of a GELU pass after the launch.
+// y = bf16(gelu(bf16(y + delta))), the bits of a GELU pass after the launch. `done`
+// (with `r_in`): an event that the launch records as its own completion.
 constexpr int kLoraMaxRank = 512;
 int lora_splits(int M, int N, int rank, int cu_count, bool pre_r);
 hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
                        uint16_t* y, int M, int K, int N, int rank, int ldb,
                        bool vec, int cu_count, hipStream_t stream,
-                       const uint16_t* r_in = nullptr, bool gelu = false);
+                       const uint16_t* r_in = nullptr, bool gelu = false,
+                       hipEvent_t done = nullptr);
 // B [rows][cols] (row stride ld_src) -> `width` columns of each dst row
 // (row stride ld_dst; width 0 = ld_dst) with zeros past `cols`: the vector
 // path's copy of an adapter whose rank is not a multiple of 8, and the

@@ -382,12 +382,14 @@ __global__ __launch_bounds__(kLoraThreads) void lora_kernel(LoraParams p)
 }
 
 template <int RB>
-hipError_t launch_rb(const LoraParams& p, bool vec, bool gelu, dim3 grid, hipStream_t stream)
+hipError_t launch_rb(const LoraParams& p, bool vec, bool gelu, dim3 grid, hipStream_t stream,
+                     hipEvent_t done)
 {
   if (p.r_in != nullptr) {
-    gelu ? lora_kernel<RB, true, true, true><<<grid, kLoraThreads, 0, stream>>>(p)
-         : lora_kernel<RB, true, true, false><<<grid, kLoraThreads, 0, stream>>>(p);
-  } else if (vec) {
+    const auto kernel = gelu ? lora_kernel<RB, true, true, true> : lora_kernel<RB, true, true, false>;
+    return launch_done(kernel, grid, kLoraThreads, stream, done, p);
+  }
+  if (vec) {
     gelu ? lora_kernel<RB, true, false, true><<<grid, kLoraThreads, 0, stream>>>(p)
          : lora_kernel<RB, true, false, false><<<grid, kLoraThreads, 0, stream>>>(p);
   } else {
@@ -679,8 +681,9 @@ int lora_splits(int M, int N, int rank, int cu_count, bool pre_r)
 hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
                        uint16_t* y, int M, int K, int N, int rank, int ldb,
                        bool vec, int cu_count, hipStream_t stream, const uint16_t* r_in,
-                       bool gelu)
+                       bool gelu, hipEvent_t done)
 {
+  if (done != nullptr && r_in == nullptr) { return hipErrorInvalidValue; }
   if (rank <= 0 || rank > kLoraMaxRank) { return hipErrorInvalidValue; }
   if (r_in != nullptr && (!vec || rank % 8 != 0)) { return hipErrorInvalidValue; }
   if (gelu && !vec) { return hipErrorInvalidValue; }
@@ -693,11 +696,11 @@ hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
   LoraParams p{r_in, x, a, b, y, M, K, N, rank, ldb, n_split};
   const dim3 grid((unsigned)((M + kLoraRows - 1) / kLoraRows), (unsigned)gy);
   const int rb = (rank + 31) / 32;
-  if (rb <= 1) { return launch_rb<1>(p, vec, gelu, grid, stream); }
-  if (rb <= 2) { return launch_rb<2>(p, vec, gelu, grid, stream); }
-  if (rb <= 4) { return launch_rb<4>(p, vec, gelu, grid, stream); }
-  if (rb <= 8) { return launch_rb<8>(p, vec, gelu, grid, stream); }
-  return launch_rb<16>(p, vec, gelu, grid, stream);
+  if (rb <= 1) { return launch_rb<1>(p, vec, gelu, grid, stream, done); }
+  if (rb <= 2) { return launch_rb<2>(p, vec, gelu, grid, stream, done); }
+  if (rb <= 4) { return launch_rb<4>(p, vec, gelu, grid, stream, done); }
+  if (rb <= 8) { return launch_rb<8>(p, vec, gelu, grid, stream, done); }
+  return launch_rb<16>(p, vec, gelu, grid, stream, done);
 }
 
 }  // namespace ltx25

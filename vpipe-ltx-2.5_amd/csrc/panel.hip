@@ -589,27 +589,25 @@ panel_kernel(PanelParams p)
 }
 
 template <int BITS, int RB, int CB>
-hipError_t launch_cfg(const PanelParams& p, dim3 grid, hipStream_t stream)
+hipError_t launch_cfg(const PanelParams& p, dim3 grid, hipStream_t stream, hipEvent_t done)
 {
-  if (p.splits > 1) {
-    hipLaunchKernelGGL((panel_kernel<BITS, RB, CB, true>), grid, dim3(kThreads), 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((panel_kernel<BITS, RB, CB, false>), grid, dim3(kThreads), 0, stream, p);
-  }
-  return hipGetLastError();
+  return p.splits > 1
+             ? launch_done(panel_kernel<BITS, RB, CB, true>, grid, kThreads, stream, nullptr, p)
+             : launch_done(panel_kernel<BITS, RB, CB, false>, grid, kThreads, stream, done, p);
 }
 
 template <int BITS>
-hipError_t launch_bits(const PanelParams& p, int rb, int cb, dim3 grid, hipStream_t stream)
+hipError_t launch_bits(const PanelParams& p, int rb, int cb, dim3 grid, hipStream_t stream,
+                       hipEvent_t done)
 {
   if (cb == 2) {
-    return rb == 4   ? launch_cfg<BITS, 4, 2>(p, grid, stream)
-           : rb == 2 ? launch_cfg<BITS, 2, 2>(p, grid, stream)
-                     : launch_cfg<BITS, 1, 2>(p, grid, stream);
+    return rb == 4   ? launch_cfg<BITS, 4, 2>(p, grid, stream, done)
+           : rb == 2 ? launch_cfg<BITS, 2, 2>(p, grid, stream, done)
+                     : launch_cfg<BITS, 1, 2>(p, grid, stream, done);
   }
-  return rb == 4   ? launch_cfg<BITS, 4, 1>(p, grid, stream)
-         : rb == 2 ? launch_cfg<BITS, 2, 1>(p, grid, stream)
-                   : launch_cfg<BITS, 1, 1>(p, grid, stream);
+  return rb == 4   ? launch_cfg<BITS, 4, 1>(p, grid, stream, done)
+         : rb == 2 ? launch_cfg<BITS, 2, 1>(p, grid, stream, done)
+                   : launch_cfg<BITS, 1, 1>(p, grid, stream, done);
 }
 
 // The panels, with the time of one workgroup as measured on w8g64 calls whose
@@ -716,12 +714,12 @@ hipError_t launch_panel(const GemmDesc& d, const GemmPlan& plan, float* workspac
   p.by_m = (size_t)d.M * 16 > (size_t)d.N * d.bits;
   p.splits = plan.splits;
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * plan.splits));
-  const hipError_t e = d.bits == 8    ? launch_bits<8>(p, rb, cb, grid, stream)
-                       : d.bits == 16 ? launch_bits<16>(p, rb, cb, grid, stream)
-                                      : launch_bits<4>(p, rb, cb, grid, stream);
+  const hipError_t e = d.bits == 8    ? launch_bits<8>(p, rb, cb, grid, stream, d.done)
+                       : d.bits == 16 ? launch_bits<16>(p, rb, cb, grid, stream, d.done)
+                                      : launch_bits<4>(p, rb, cb, grid, stream, d.done);
   if (e != hipSuccess || plan.splits <= 1) { return e; }
   return launch_splitk_reduce(workspace, plan.splits, d.bias, p.bias_type, d.epilogue, d.y_in,
-                              d.y, d.M, d.N, stream);
+                              d.y, d.M, d.N, stream, d.done);
 }
 
 }  // namespace ltx25

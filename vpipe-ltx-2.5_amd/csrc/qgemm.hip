@@ -923,13 +923,12 @@ hipError_t launch_i8_gemm(const int8_t* xq, const float* sx, const int8_t* wq, c
 
 hipError_t launch_splitk_reduce(const float* partial, int splits, const void* bias, int bias_type,
                                 int epilogue, const uint16_t* y_in, uint16_t* y, int M, int N,
-                                hipStream_t stream)
+                                hipStream_t stream, hipEvent_t done)
 {
   const size_t total = (size_t)M * N;
   const unsigned blocks = (unsigned)((total + 1023) / 1024);
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, stream, partial, splits,
-                     bias, bias != nullptr ? bias_type : kBiasNone, epilogue, y_in, y, M, N);
-  return hipGetLastError();
+  return launch_done(splitk_reduce_kernel, dim3(blocks), 256, stream, done, partial, splits, bias,
+                     bias != nullptr ? bias_type : (int)kBiasNone, epilogue, y_in, y, M, N);
 }
 
 hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
@@ -944,8 +943,11 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
   }
   if (plan.tile == 2) { return launch_skinny(d, plan, workspace, stream); }
   if (plan.panel_rows > 0 && d.x2 == nullptr) { return launch_panel(d, plan, workspace, stream); }
+  auto record = [&](hipError_t e) {
+    return e == hipSuccess && d.done != nullptr ? hipEventRecord(d.done, stream) : e;
+  };
   if (tall_dense_takes(d, plan) || tall_w8_takes(d, plan)) {
-    return launch_tall_dense(d, stream, plan.half_tall ? 128 : 256, plan.cu_count);
+    return record(launch_tall_dense(d, stream, plan.half_tall ? 128 : 256, plan.cu_count));
   }
   KParams kp = {};
   kp.x = d.x;
@@ -977,9 +979,9 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
                      ? launch_tile<256, 256, kTallWM, kTallWN>(kp, d.bits, plan.splits, stream)
                      : launch_tile<128, kMidBN, 2 * 128 / kMidBN, kMidBN / 64>(
                            kp, d.bits, plan.splits, stream);
-  if (e != hipSuccess || plan.splits <= 1) { return e; }
+  if (e != hipSuccess || plan.splits <= 1) { return record(e); }
   return launch_splitk_reduce(workspace, plan.splits, kp.bias, kp.bias_type, d.epilogue, d.y_in,
-                              d.y, d.M, d.N, stream);
+                              d.y, d.M, d.N, stream, d.done);
 }
 
 }  // namespace ltx25

@@ -538,24 +538,22 @@ skinny_kernel(SParams p)
 }
 
 template <int BITS, int ROWS>
-hipError_t launch_rows(const SParams& p, const GemmPlan& plan, hipStream_t stream)
+hipError_t launch_rows(const SParams& p, const GemmPlan& plan, hipStream_t stream, hipEvent_t done)
 {
   const dim3 grid((unsigned)((p.N + kCols - 1) / kCols), (unsigned)plan.splits,
                   (unsigned)((p.M + ROWS - 1) / ROWS));
-  if (plan.splits > 1) {
-    hipLaunchKernelGGL((skinny_kernel<BITS, true, ROWS>), grid, dim3(kThreads), 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((skinny_kernel<BITS, false, ROWS>), grid, dim3(kThreads), 0, stream, p);
-  }
-  return hipGetLastError();
+  return plan.splits > 1
+             ? launch_done(skinny_kernel<BITS, true, ROWS>, grid, kThreads, stream, nullptr, p)
+             : launch_done(skinny_kernel<BITS, false, ROWS>, grid, kThreads, stream, done, p);
 }
 
 template <int BITS>
-hipError_t launch_bits(const SParams& p, const GemmPlan& plan, int rows, hipStream_t stream)
+hipError_t launch_bits(const SParams& p, const GemmPlan& plan, int rows, hipStream_t stream,
+                       hipEvent_t done)
 {
-  return rows == 32   ? launch_rows<BITS, 32>(p, plan, stream)
-         : rows == 64 ? launch_rows<BITS, 64>(p, plan, stream)
-                      : launch_rows<BITS, 128>(p, plan, stream);
+  return rows == 32   ? launch_rows<BITS, 32>(p, plan, stream, done)
+         : rows == 64 ? launch_rows<BITS, 64>(p, plan, stream, done)
+                      : launch_rows<BITS, 128>(p, plan, stream, done);
 }
 
 // Token rows per workgroup. A workgroup's time is set by the X rows it pulls
@@ -651,13 +649,13 @@ hipError_t launch_skinny(const GemmDesc& d, const GemmPlan& plan, float* workspa
     e = hipGetLastError();
   } else {
     const int rows = rows_for(d.M, d.N, plan.splits, plan.cu_count);
-    e = d.bits == 8    ? launch_bits<8>(p, plan, rows, stream)
-        : d.bits == 16 ? launch_bits<16>(p, plan, rows, stream)
-                       : launch_bits<4>(p, plan, rows, stream);
+    e = d.bits == 8    ? launch_bits<8>(p, plan, rows, stream, d.done)
+        : d.bits == 16 ? launch_bits<16>(p, plan, rows, stream, d.done)
+                       : launch_bits<4>(p, plan, rows, stream, d.done);
   }
   if (e != hipSuccess || !split) { return e; }
   return launch_splitk_reduce(workspace, plan.splits, d.bias, p.bias_type, d.epilogue, d.y_in,
-                              d.y, d.M, d.N, stream);
+                              d.y, d.M, d.N, stream, d.done);
 }
 
 }  // namespace ltx25
