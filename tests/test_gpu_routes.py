@@ -102,11 +102,11 @@ def test_row_slabs_past_2gib(pkg, quantized):
 
 
 # where the planner leaves the 128 x 128 tile with one K split for larger ones: 128 x 256 tiles
-# (dense weights) and 256 x 256 tiles that do not fill the CUs; 1, 2, 3 and many K steps, ragged
-# M and N
+# (dense weights, from K = 1024) and 256 x 256 tiles that do not fill the CUs; 1, 2, 3 and many K
+# steps, ragged M and N
 LARGER = [  # M, K, N, tile
-    (1024, 64, 8192, 2), (300, 128, 16392, 2), (897, 192, 8008, 2), (1000, 1088, 8192, 2),
-    (257, 320, 16000, 2), (700, 64, 16384, 1), (900, 128, 12296, 1), (641, 960, 13000, 1),
+    (1024, 64, 8192, 2), (300, 960, 16392, 2), (300, 1024, 16392, 2), (897, 1152, 8008, 2),
+    (1000, 1088, 8192, 2), (257, 1024, 16000, 2), (700, 64, 16384, 1), (900, 128, 12296, 1), (641, 960, 13000, 1),
 ]
 
 
@@ -142,8 +142,8 @@ def test_larger_tiles_give_the_same_bits(pkg, M, K, N, tile, bias, epi):
         assert np.array_equal(outs[0], outs[2])
 
 
-@pytest.mark.parametrize("M,K,N", [(1024, 128, 8192), (300, 256, 16392), (1000, 1152, 8200),
-                                   (1500, 384, 9000)])
+@pytest.mark.parametrize("M,K,N", [(1024, 1408, 8192), (1024, 1536, 8192), (300, 1664, 16392),
+                                   (1000, 1792, 8200), (1500, 384, 9000)])
 def test_larger_int8_tiles_are_exact(pkg, M, K, N):
     """int8 on 128 x 256 tiles and on 256 x 256 tiles that do not fill the CUs: int32 accumulators
     and bf16 outputs exact."""
@@ -163,11 +163,11 @@ def test_larger_int8_tiles_are_exact(pkg, M, K, N):
     assert torch.equal(y, want.to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("rank", [100, 192])
-def test_larger_tiles_under_the_lora_pair(pkg, rank):
-    """The pair's second GEMM, accumulators seeded from y, and the fold's two-part activation on
-    128 x 256 tiles: the bits of the forced 256 x 256 tile."""
-    M, K, N = 1024, 256, 8192
+@pytest.mark.parametrize("rank,K", [(100, 256), (1000, 192), (1088, 1024)])
+def test_larger_tiles_under_the_lora_pair(pkg, rank, K):
+    """The pair's second GEMM, accumulators seeded from y (from 1024 columns of rank), and the
+    fold's two-part activation on 128 x 256 tiles: the bits of the forced 256 x 256 tile."""
+    M, N = 1024, 8192
     rng = np.random.default_rng(rank)
     x, a, b = (dev_bf16(orc.bf16_rne(rng_normal(rng, s, 0.1))) for s in ((M, K), (rank, K), (N, rank)))
     y0 = dev_bf16(orc.bf16_rne(rng_normal(rng, (M, N))))

@@ -165,8 +165,9 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmPlan& plan,
                        float* workspace, hipStream_t stream);
 // Rows of the ping-pong kernel's tile that an unsplit GEMM is best served by:
 // 256, 128, or 0 where the 128 x 128 tile is (dense weights and int8 operands;
-// codes, dequantized in registers, have no 128-row one).
-int tall_rows(int M, int N, int cu_count);
+// codes, dequantized in registers, have no 128-row one). `steps`: K steps of 128
+// bytes of an operand's row.
+int tall_rows(int M, int N, int steps, bool i8, int cu_count);
 // The M <= 128 route (skinny.hip): 32 output columns per workgroup, K split
 // between its 8 waves, and across workgroups above 2048. Fills `plan` and
 // returns true when it takes the shape (up to 3 workgroups per CU);

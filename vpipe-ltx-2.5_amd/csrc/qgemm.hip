@@ -833,7 +833,7 @@ GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force, bool 
   // a forced M <= 128 kernel that cannot take the shape leaves the choice
   // to the planner
   const bool plans = force == 0 || force == 3;
-  const int rows = plans && M > 128 && N % 8 == 0 ? tall_rows(M, N, cu_count) : 0;
+  const int rows = plans && M > 128 && N % 8 == 0 ? tall_rows(M, N, K / 64, false, cu_count) : 0;
   if (force == 1 || rows == 256 || (plans && M > 128 && tall_tiles >= cu_count)) {
     plan.tile = 0;
     plan.splits = 1;
@@ -869,14 +869,17 @@ GemmPlan plan_gemm(int M, int N, int K, int bits, int cu_count, int force, bool 
 // dense 63 against 75 us (256 x 256: 77), 300 x 4096 -> 16384 60 and 69, int8 1024 x
 // 4096 -> 8192 35 and 41. With one workgroup per CU the 128 x 128 tile is ahead:
 // 8160 x 4096 -> 512 41 against 51, as are 256 x 256 tiles past one round of 128 x
-// 256 ones: 2040 x 4096 -> 8192 100 against 123.
-int tall_rows(int M, int N, int cu_count)
+// 256 ones: 2040 x 4096 -> 8192 100 against 123. Few K steps don't pay for the 128 x 256
+// tile's fixed part either: over 40 such shapes w8 takes 0.97 to 1.06 of the 128 x 128
+// tile's time at K = 512, 0.95 to 1.02 at 1024, 0.92 to 1.00 at 1280; int8 0.93 to 1.03 at
+// 1024, 0.92 to 0.99 at 1536.
+int tall_rows(int M, int N, int steps, bool i8, int cu_count)
 {
   const long mid = (long)((M + 127) / 128) * ((N + 127) / 128);
   const long half = (long)((M + 127) / 128) * ((N + 255) / 256);
   const long tall = (long)((M + 255) / 256) * ((N + 255) / 256);
   if (tall >= cu_count || mid > 2L * cu_count) { return 256; }
-  return mid > cu_count && half <= cu_count ? 128 : 0;
+  return mid > cu_count && half <= cu_count && steps >= (i8 ? 12 : 16) ? 128 : 0;
 }
 
 hipError_t launch_i8_gemm(const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
@@ -906,7 +909,7 @@ hipError_t launch_i8_gemm(const int8_t* xq, const float* sx, const int8_t* wq, c
   }
   // the tall tile when it fills the GPU or serves it better, else 128 x 128
   const bool fills = (long)((M + 255) / 256) * ((N + 255) / 256) >= cus;
-  const int rows = tall_rows(M, N, cus);
+  const int rows = tall_rows(M, N, K / 128, true, cus);
   if (rows > 0 && tall_i8_takes(M, N, K)) {
     return launch_tall_i8(xq, sx, wq, sw, bias, kp.bias_type, epilogue, y, acc, M, K, N, stream,
                           rows, cus);
