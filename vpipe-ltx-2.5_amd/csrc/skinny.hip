@@ -244,14 +244,16 @@ skinny_kernel(SParams p)
     const int hf = u % kUpc;
     lds_u32* dst = (lds_u32*)(slot + (u % kRing) * kUnitBytes);
     const uint32_t soff = (uint32_t)(kw0 + t * kChunk) * 2;
+    // 8 rows a step by addition: with a product per load the kernel is 92 instructions
+    // longer, and 126 x 2048 -> 6144 takes 11.10 us where it takes 10.96
+    uint32_t row = (uint32_t)(m0 + kURows * hf + (lane >> 3)) * ((uint32_t)p.K * 2u);
 #pragma unroll
     for (int i = 0; i < kULoads; ++i) {
-      const int r0 = m0 + kURows * hf + 8 * i;     // first row of this load
-      // row r0 + l/8: swizzle (r/2) % 8 = (4 i + l/16) % 8 (r0 is a multiple of 8)
+      // row 8 i + l/8 of the unit: swizzle (r/2) % 8 = (4 i + l/16) % 8
       const int sw = ((4 * i) + (lane >> 4)) & 7;
-      const uint32_t vo = (uint32_t)((size_t)(r0 + (lane >> 3)) * p.K * 2 +
-                                     (((lane & 7) ^ sw) * 16));
+      const uint32_t vo = row + (((lane & 7) ^ sw) * 16);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, dst + i * 256, 16, (int)vo, (int)soff, 0, 0);
+      row += (uint32_t)p.K * 16u;
     }
   };
   // the units of the slot's first half go ahead of the weight, those of its
