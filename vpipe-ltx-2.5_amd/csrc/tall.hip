@@ -910,8 +910,8 @@ hipError_t launch_tall(const TallParams& p, int mode, int bm, hipStream_t stream
 // rest goes out as 128 x 256 tiles, which fit one round. At K = 4096 a last round of
 // r tiles takes about 58 + 0.16 r us, 2 r half tiles 40 + 0.18 r and the second
 // launch 3 us, so from 2048 of K (4096 int8). Dense 2040 x 4096 -> 12288 (384 tiles)
-// 174 -> 165 us, 5000 x 8192 -> 4096 (320) 316 -> 284; int8 8160 x 8192 -> 4352 (544)
-// 260 -> 244. The same bits.
+// 177 -> 160 us, 5000 x 8192 -> 4096 (320) 306 -> 281; int8 8160 x 8192 -> 4352 (544)
+// 256 -> 240; 60 such shapes, dense and int8, 0.89 to 0.99 of one launch. The same bits.
 hipError_t launch_rounds(const TallParams& p, int mode, int cu_count, hipStream_t stream)
 {
   const size_t eb = mode == kModeI8 ? 1 : 2;
