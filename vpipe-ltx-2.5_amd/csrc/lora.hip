@@ -32,6 +32,7 @@
 // where phase 1 is the larger part (K from 1536; from 512 for wide ranks). A linear's
 // GELU can follow the sum in the y phase, instead of a pass of its own.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -668,14 +669,19 @@ hipError_t launch_lora_pad(const uint16_t* src, int rows, int cols, int ld_src, 
 // workgroups to cover the CUs once; a narrow one, whose phase 2 is bound by
 // y traffic and wants waves in flight, gets two per CU. Never fewer than
 // 1024 columns per workgroup, or the 512 of one super-block stride where r is
-// given and nothing is recomputed.
+// given, nothing is recomputed and one workgroup per CU holds them all: 128 x
+// 4096 -> 16384 at rank 32 is faster so, while 6024 x 960 -> 656 at rank 88 takes 20.5
+// us on 189 workgroups and 23.0 on 378, 1012 x 960 -> 7576 at rank 48 20.2 on 256 and
+// 22.1 on 480.
 int lora_splits(int M, int N, int rank, int cu_count, bool pre_r)
 {
   const int mtiles = (M + kLoraRows - 1) / kLoraRows;
   const int per_cu = rank > 128 && !pre_r ? 1 : 2;
   const int want = per_cu * cu_count / mtiles;
-  const int cap = pre_r ? (N + 511) / 512 : (N + 1023) / 1024;
-  return want < 1 ? 1 : (want < cap ? want : cap);
+  const int cap = (N + 1023) / 1024;
+  const int splits = want < 1 ? 1 : (want < cap ? want : cap);
+  const int fine = pre_r ? std::min((N + 511) / 512, cu_count / mtiles) : 0;
+  return std::max(splits, fine);
 }
 
 hipError_t launch_lora(const uint16_t* x, const uint16_t* a, const uint16_t* b,
