@@ -192,9 +192,12 @@ PLANS = [  # M, K, N, rank
     (255, 1024, 1032, 32), (255, 960, 1032, 32), (70, 1088, 264, 40), (70, 1024, 264, 40),
     # b copied
     (1, 11456, 520, 5), (1, 11392, 520, 5), (33, 1024, 8, 90), (20, 1088, 512, 95),
-    (20, 960, 512, 95), (255, 2304, 4104, 17), (255, 2240, 4104, 17), (300, 2560, 96, 12),
-    (40, 1536, 1000, 1), (700, 3904, 264, 6), (700, 3840, 264, 6), (600, 2688, 4104, 6),
-    (600, 2624, 4104, 6), (600, 1024, 264, 90),
+    (20, 960, 512, 95), (255, 1472, 4104, 17), (255, 1408, 4104, 17), (300, 2560, 96, 12),
+    (40, 1536, 1000, 1), (700, 3008, 264, 6), (700, 2944, 264, 6), (600, 1984, 4104, 6),
+    (600, 1920, 4104, 6), (600, 1024, 264, 90), (3000, 3904, 40, 6), (64, 512, 2056, 90),
+    # many columns
+    (1, 10944, 2056, 8), (1, 4096, 2056, 8), (64, 1152, 2056, 8), (64, 1088, 2056, 8),
+    (64, 384, 2056, 64), (64, 320, 2056, 64),
     # both on the dense GEMM
     (255, 1024, 264, 96), (255, 512, 264, 96), (64, 512, 264, 128), (1, 512, 264, 128),
     (3, 512, 1000, 450), (3, 448, 1000, 450), (255, 512, 264, 128), (255, 512, 2056, 128),

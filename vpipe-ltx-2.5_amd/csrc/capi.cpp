@@ -643,17 +643,29 @@ int lora_pair(DeviceState* ds, hipStream_t st, const LoraPairPlan& p, const void
 long lora_phase1(int M, int K, int rank) { return (long)K * (rank + std::min(M + 8, 32)); }
 
 // Rank 8, 64 x 1536 -> 512 8.9 and 9.2, x 3072 12.5 and 11.4; rank 17 (b copied), 64 x 3072 ->
-// 512 16.6 and 16.7, x 4096 18.9 and 17.3; rank 50, 64 x 1024 -> 512 13.8 and 15.0, x 2048
-// 18.0 and 16.6; rank 4, 600 x 1024 -> 512 11.6 and 13.4, x 4096 16.9 and 15.2. From 512 tokens
-// only a b that is copied gets here; with many columns the one-pass kernel then
-// repeats phase 1 for each of its column splits.
+// 512 16.6 and 16.7, -> 2048 17.8 and 16.8; rank 50, 64 x 1024 -> 512 13.8 and 15.0, x 2048 18.0
+// and 16.6; rank 4, 600 x 1024 -> 512 11.6 and 13.4, x 4096 16.9 and 15.2. With many columns the
+// y phase's finer split counts too; from 512 tokens, where only a b that is copied gets
+// here, the one-pass kernel also repeats phase 1 for each of its own: rank 4, 1500 x 2048 ->
+// 512 12.8 and 14.0, -> 8192 27.2 and 22.7. Above 128 rows r's GEMM takes slower tiles
+// below 1024 of K.
 bool lora_ahead_pays(int M, int K, int N, int rank, bool copies_b)
 {
-  long line = copies_b ? 120000 : 75000;   // two or three rank blocks
-  if (rank <= 32 && copies_b) {
-    line = M <= 128 ? 160000 : M < kLoraRFirstMinM ? 110000 : N >= 4096 ? 100000 : 146000;
-  } else if (rank <= 32) {
-    line = M < 24 ? 130000 : M <= 128 ? 82000 : 62000;
+  const bool many = N >= 2048;
+  long line = 0;
+  if (rank > 32) {   // two or three rank blocks
+    if (M > 128) {
+      line = copies_b ? (many && K >= 1024 ? 84000 : 124000) : (K >= 1024 ? 73000 : 98000);
+    } else {
+      line = copies_b ? (many ? 60000 : 120000) : (many ? 36000 : 78000);
+    }
+  } else if (copies_b) {
+    line = M <= 128              ? (many ? 114000 : 160000)
+           : M < kLoraRFirstMinM ? (many ? 70000 : 111000)
+           : many                ? 74000
+                                 : (M < 3000 ? 113000 : 147000);
+  } else {
+    line = M < 24 ? (many ? 98000 : 133000) : M <= 128 ? (many ? 45000 : 82000) : 62000;
   }
   return lora_phase1(M, K, rank) >= line;
 }
